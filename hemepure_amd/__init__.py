@@ -200,6 +200,7 @@ _SIGS = {
     "hlb_xtr_write_fields": (C.c_int, [C.c_void_p, C.c_int64, C.c_void_p, C.c_void_p, C.c_void_p,
                                        C.c_void_p, C.c_void_p]),
     "hlb_get_stress": (C.c_int, [C.c_void_p] + [C.c_void_p] * 6),
+    "hlb_get_stress_rows": (C.c_int, [C.c_void_p, C.c_void_p]),
     "hlb_xtr_site_count": (C.c_int64, [C.c_void_p]),
     "hlb_xtr_close": (None, [C.c_void_p]),
     "hlb_checkpoint_read": (C.c_int, [C.c_void_p, C.c_char_p, C.c_int64, C.POINTER(C.c_int64),
@@ -539,11 +540,9 @@ class Lattice:
         """Stress caches from the state entering the next step, n x 17: stress
         tensor (xx, xy, xz, yy, yz, zz), von Mises, shear rate, traction,
         tangential and normal projections of the traction."""
-        n = self.n
-        ten, vm, rate = np.empty((n, 6)), np.empty(n), np.empty(n)
-        tr, tt, tn = np.empty((n, 3)), np.empty((n, 3)), np.empty((n, 3))
-        _check(lib().hlb_get_stress(self._h, _ptr(ten), _ptr(vm), _ptr(rate), _ptr(tr), _ptr(tt), _ptr(tn)))
-        return np.concatenate([ten, vm[:, None], rate[:, None], tr, tt, tn], axis=1)
+        rows = np.empty((self.n, 17))
+        _check(lib().hlb_get_stress_rows(self._h, _ptr(rows)))
+        return rows
 
     def timestep(self) -> int:
         return int(lib().hlb_timestep(self._h))

@@ -19,7 +19,7 @@ CSRC = PKG / "csrc"
 BUILD = PKG / "_build"
 LIB = PKG / "libhemepure_amd.so"
 
-SOURCES = ["capi.hip", "batch.hip", "server.hip", "lbm_fp64.hip", "lbm_fp32.hip", "lattice.cpp", "geometry_gen.cpp", "gmy_reader.cpp",
+SOURCES = ["capi.hip", "batch.hip", "server.hip", "lbm_fp64.hip", "lbm_fp32.hip", "transfer.hip", "lattice.cpp", "geometry_gen.cpp", "gmy_reader.cpp",
            "extraction.cpp"]
 # Host-only sources built with the system C++ compiler: their complex
 # arithmetic and transcendental calls must round as the reference's build of

@@ -28,6 +28,7 @@
 #include "iolet_math.h"
 #include "lattice.h"
 #include "lbm_kernels.h"
+#include "transfer.h"
 
 namespace hlb {
 
@@ -698,7 +699,8 @@ int ensure_device(hlb_lattice* h) {
   HLB_CHECK(hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking));
   HLB_CHECK(hipEventCreate(&h->ev0));
   HLB_CHECK(hipEventCreate(&h->ev1));
-  const int rc = upload_lattice(h);
+  int rc = upload_lattice(h);
+  if (rc == HLB_OK) rc = transfer_open(h);
   if (rc != HLB_OK) return rc;
   h->device_ready = true;
   return HLB_OK;
@@ -1306,35 +1308,20 @@ extern "C" int hlb_upload_f(hlb_handle h, const double* f, int64_t t0) {
     const int rc = ensure_device(h);
     if (rc != HLB_OK) return rc;
   }
-  const int64_t N = h->L.N, S = h->S;
   // The copy below replaces F: queued steps that still read it (hlb_step is
   // asynchronous, on the handle's or its batch's stream) finish first.
   if (h->batch) HLB_CHECK(hipStreamSynchronize(batch_stream(h->batch)));
   HLB_CHECK(hipStreamSynchronize(h->stream));
+  const size_t count = (size_t)Q * h->S;
   if (h->fp32()) {
-    std::vector<float> soa((size_t)Q * S, 0.0f);
-    for (int64_t k = 0; k < N; ++k) {
-      const double* src = f + (size_t)k * Q;
-      const int64_t d = h->inv[k];
-      for (int j = 0; j < Q; ++j) soa[(size_t)j * S + d] = (float)(src[j] - Wt(j));
-    }
-    if (!h->F32.p) HLB_CHECK(h->F32.alloc((size_t)Q * S));
-    HLB_CHECK(hipMemcpyAsync(h->F32.p, soa.data(), sizeof(float) * soa.size(), hipMemcpyHostToDevice, h->stream));
-    HLB_CHECK(hipStreamSynchronize(h->stream));
-    h->have_post = false;
-    h->f_valid = true;
-    h->t = t0;
-    return HLB_OK;
+    if (!h->F32.p) HLB_CHECK(h->F32.alloc(count));
+  } else if (!h->F.p) {
+    HLB_CHECK(h->F.alloc(count));
   }
-  std::vector<double> soa((size_t)Q * S, 0.0);
-  for (int64_t k = 0; k < N; ++k) {
-    const double* src = f + (size_t)k * Q;
-    const int64_t d = h->inv[k];
-    for (int j = 0; j < Q; ++j) soa[(size_t)j * S + d] = src[j];
+  {
+    const int rc = import_sites(h, f, h->fp32() ? (void*)h->F32.p : (void*)h->F.p, h->fp32());
+    if (rc != HLB_OK) return rc;
   }
-  if (!h->F.p) HLB_CHECK(h->F.alloc((size_t)Q * S));
-  HLB_CHECK(hipMemcpyAsync(h->F.p, soa.data(), sizeof(double) * soa.size(), hipMemcpyHostToDevice, h->stream));
-  HLB_CHECK(hipStreamSynchronize(h->stream));
   h->have_post = false;
   h->f_valid = true;
   h->t = t0;
@@ -1422,61 +1409,29 @@ extern "C" int hlb_synchronize(hlb_handle h) {
 extern "C" int hlb_download_f(hlb_handle h, double* f) {
   if (!h || (!f && h->L.N > 0)) return fail(HLB_EINVAL, "hlb_download_f: null argument");
   if (!h->f_valid) return fail(HLB_EINVAL, "hlb_download_f: no state");
-  int rc = materialise_f(h);
+  const int rc = materialise_f(h);
   if (rc != HLB_OK) return rc;
-  const int64_t N = h->L.N, S = h->S;
-  if (h->fp32()) {
-    std::vector<float> soa((size_t)Q * S);
-    HLB_CHECK(hipMemcpyAsync(soa.data(), h->F32.p, sizeof(float) * soa.size(), hipMemcpyDeviceToHost, h->stream));
-    HLB_CHECK(hipStreamSynchronize(h->stream));
-    for (int64_t k = 0; k < N; ++k) {
-      double* dst = f + (size_t)k * Q;
-      const int64_t d = h->inv[k];
-      for (int j = 0; j < Q; ++j) dst[j] = (double)soa[(size_t)j * S + d] + Wt(j);
-    }
-    return HLB_OK;
-  }
-  std::vector<double> soa((size_t)Q * S);
-  HLB_CHECK(hipMemcpyAsync(soa.data(), h->F.p, sizeof(double) * soa.size(), hipMemcpyDeviceToHost, h->stream));
-  HLB_CHECK(hipStreamSynchronize(h->stream));
-  for (int64_t k = 0; k < N; ++k) {
-    double* dst = f + (size_t)k * Q;
-    const int64_t d = h->inv[k];
-    for (int j = 0; j < Q; ++j) dst[j] = soa[(size_t)j * S + d];
-  }
-  return HLB_OK;
+  const TransferPart part{h->fp32() ? (const void*)h->F32.p : (const void*)h->F.p, Q, f};
+  return export_sites(h, &part, 1, h->fp32());
 }
 
 extern "C" int hlb_get_fields(hlb_handle h, double* rho, double* u, double* wss) {
   if (!h) return fail(HLB_EINVAL, "hlb_get_fields: null handle");
   if (!h->device_ready) return fail(HLB_EINVAL, "hlb_get_fields: no state");
-  const int64_t N = h->L.N, S = h->S;
-  HLB_CHECK(hipStreamSynchronize(h->stream));
-  std::vector<double> tmp((size_t)3 * S);
-  if (rho) {
-    HLB_CHECK(hipMemcpy(tmp.data(), h->rho.p, sizeof(double) * S, hipMemcpyDeviceToHost));
-    for (int64_t k = 0; k < N; ++k) rho[k] = tmp[h->inv[k]];
-  }
-  if (wss) {
-    HLB_CHECK(hipMemcpy(tmp.data(), h->wss.p, sizeof(double) * S, hipMemcpyDeviceToHost));
-    for (int64_t k = 0; k < N; ++k) wss[k] = tmp[h->inv[k]];
-  }
-  if (u) {
-    HLB_CHECK(hipMemcpy(tmp.data(), h->u.p, sizeof(double) * tmp.size(), hipMemcpyDeviceToHost));
-    for (int64_t k = 0; k < N; ++k)
-      for (int a = 0; a < 3; ++a) u[3 * (size_t)k + a] = tmp[(size_t)a * S + h->inv[k]];
-  }
-  return HLB_OK;
+  const TransferPart parts[] = {{h->rho.p, 1, rho}, {h->u.p, 3, u}, {h->wss.p, 1, wss}};
+  return export_sites(h, parts, 3, false);
 }
 
-extern "C" int hlb_get_stress(hlb_handle h, double* tensor, double* von_mises, double* shear_rate,
-                              double* traction, double* tangential, double* normal) {
-  if (!h) return fail(HLB_EINVAL, "hlb_get_stress: null handle");
-  if (!h->f_valid) return fail(HLB_EINVAL, "hlb_get_stress: no state");
+namespace hlb {
+namespace {
+
+// The 17 stress planes of the state entering the next step, queued on the
+// handle's stream.
+int compute_stress(hlb_lattice* h, const char* who) {
+  if (!h->f_valid) return fail(HLB_EINVAL, std::string(who) + ": no state");
   int rc = materialise_f(h);
   if (rc != HLB_OK) return rc;
-  const int64_t N = h->L.N, S = h->S;
-  if (!h->stress.p) HLB_CHECK(h->stress.alloc((size_t)17 * S));
+  if (!h->stress.p) HLB_CHECK(h->stress.alloc((size_t)17 * h->S));
   const StepArgs a = make_args(h, nullptr, nullptr);
   if (h->sponge_life > 0) {
     // the relaxation time of the step the materialised state enters
@@ -1486,23 +1441,31 @@ extern "C" int hlb_get_stress(hlb_handle h, double* tensor, double* von_mises, d
   }
   if (h->fp32()) HLB_CHECK(launch_stress_fp64(a, h->params.kernel, h->F32.p, true, h->stress.p, h->stream));
   else HLB_CHECK(launch_stress_fp64(a, h->params.kernel, h->F.p, false, h->stress.p, h->stream));
-  HLB_CHECK(hipStreamSynchronize(h->stream));
-  std::vector<double> tmp((size_t)S);
-  // (destination, first plane, planes)
-  const struct {
-    double* dst;
-    int first, n;
-  } parts[] = {{tensor, 0, 6}, {von_mises, 6, 1}, {shear_rate, 7, 1}, {traction, 8, 3}, {tangential, 11, 3},
-               {normal, 14, 3}};
-  for (const auto& p : parts) {
-    if (!p.dst) continue;
-    for (int c = 0; c < p.n; ++c) {
-      HLB_CHECK(hipMemcpy(tmp.data(), h->stress.p + (size_t)(p.first + c) * S, sizeof(double) * S,
-                          hipMemcpyDeviceToHost));
-      for (int64_t k = 0; k < N; ++k) p.dst[(size_t)k * p.n + c] = tmp[h->inv[k]];
-    }
-  }
   return HLB_OK;
+}
+
+}  // namespace
+}  // namespace hlb
+
+extern "C" int hlb_get_stress(hlb_handle h, double* tensor, double* von_mises, double* shear_rate,
+                              double* traction, double* tangential, double* normal) {
+  if (!h) return fail(HLB_EINVAL, "hlb_get_stress: null handle");
+  const int rc = compute_stress(h, "hlb_get_stress");
+  if (rc != HLB_OK) return rc;
+  const int64_t S = h->S;
+  // planes: tensor 0-5, von Mises 6, shear rate 7, traction 8-10, its tangential 11-13 and normal 14-16 projections
+  const double* p = h->stress.p;
+  const TransferPart parts[] = {{p, 6, tensor},         {p + 6 * S, 1, von_mises},   {p + 7 * S, 1, shear_rate},
+                                {p + 8 * S, 3, traction}, {p + 11 * S, 3, tangential}, {p + 14 * S, 3, normal}};
+  return export_sites(h, parts, 6, false);
+}
+
+extern "C" int hlb_get_stress_rows(hlb_handle h, double* rows) {
+  if (!h || (!rows && h->L.N > 0)) return fail(HLB_EINVAL, "hlb_get_stress_rows: null argument");
+  const int rc = compute_stress(h, "hlb_get_stress_rows");
+  if (rc != HLB_OK) return rc;
+  const TransferPart part{h->stress.p, 17, rows};
+  return export_sites(h, &part, 1, false);
 }
 
 extern "C" int64_t hlb_timestep(hlb_handle h) { return h ? h->t : -1; }

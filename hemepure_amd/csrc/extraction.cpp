@@ -206,7 +206,7 @@ struct hlb_xtr {
   bool wantFields = false, wantF = false, wantStress = false;
   int64_t captured = -1;   // step whose entering state f and stress hold
   std::vector<double> f;       // n*19
-  std::vector<double> stress;  // n*17, the hlb_get_stress layout
+  std::vector<double> stress;  // n*17, the hlb_get_stress_rows layout
   std::vector<double> normal;  // n*3, GetWallNormal (inf where none)
 };
 
@@ -450,21 +450,9 @@ extern "C" int hlb_xtr_capture(hlb_xtr_handle x) {
       if (rc != HLB_OK) return rc;
     }
     if (x->wantStress) {
-      std::vector<double> ten(N * 6), vm(N), rate(N), tr(N * 3), tt(N * 3), tn(N * 3);
-      const int rc = hlb_get_stress(x->lattice, ten.data(), vm.data(), rate.data(), tr.data(), tt.data(), tn.data());
-      if (rc != HLB_OK) return rc;
       x->stress.resize(N * 17);
-      for (size_t k = 0; k < N; ++k) {
-        double* o = &x->stress[17 * k];
-        for (int c = 0; c < 6; ++c) o[c] = ten[6 * k + c];
-        o[6] = vm[k];
-        o[7] = rate[k];
-        for (int a = 0; a < 3; ++a) {
-          o[8 + a] = tr[3 * k + a];
-          o[11 + a] = tt[3 * k + a];
-          o[14 + a] = tn[3 * k + a];
-        }
-      }
+      const int rc = hlb_get_stress_rows(x->lattice, x->stress.data());
+      if (rc != HLB_OK) return rc;
     }
   } catch (const std::bad_alloc&) {
     return fail(HLB_EINVAL, "hlb_xtr_capture: out of host memory");

@@ -12,6 +12,7 @@
 #include "errors.h"
 #include "lattice.h"
 #include "lbm_kernels.h"
+#include "transfer.h"
 
 namespace hlb {
 
@@ -117,6 +118,7 @@ struct hlb_lattice {
   hlb::DevBuf<int32_t> bgi, bii;
   hlb::DevBuf<hlb::SlabRec> rec;  // slab records
   hlb::DevBuf<float> bq, bnrm, io_nf;
+  hlb::DevBuf<int32_t> dinv;      // inv on the device (transfer.hip)
   hlb::DevBuf<int> flag;
   // Guo-Zheng-Shi walls (params.wall_bc == HLB_WALL_GZS).
   std::vector<hlb::GzsLink> gz_links_host;
@@ -194,6 +196,7 @@ struct hlb_lattice {
     if (ev1) (void)hipEventDestroy(ev1);
     if (h_stage) (void)hipHostFree(h_stage);
     if (h_mem) (void)hipHostFree(h_mem);
+    if (device_ready) hlb::transfer_close();
   }
   bool fp32() const { return params.precision == HLB_FP32_SHIFTED; }
   hlb::GzsTables gz_tables() const {

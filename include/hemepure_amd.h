@@ -256,6 +256,9 @@ int hlb_get_fields(hlb_handle h, double* rho, double* u, double* wss);
  * NULL. */
 int hlb_get_stress(hlb_handle h, double* tensor, double* von_mises, double* shear_rate, double* traction,
                    double* tangential, double* normal);
+/* The same as one n*17 record array: per site the tensor's 6, von Mises, shear
+ * rate, traction 3, tangential 3, normal 3. */
+int hlb_get_stress_rows(hlb_handle h, double* rows);
 /* SimulationState::GetTimeStep (src/lb/SimulationState.cc:50): the 1-indexed
  * step that runs next. */
 int64_t hlb_timestep(hlb_handle h);
@@ -329,7 +332,7 @@ int hlb_xtr_write(hlb_xtr_handle x, int64_t* timestep);
 /* Writes one record from caller arrays in the lattice's site order, lattice
  * units: rho n, u n*3, wss n, f n*19, stress n*17 (per site the stress
  * tensor's 6, von Mises, shear rate, traction 3, tangential 3, normal 3, as
- * hlb_get_stress returns them); arrays no field uses may be NULL. */
+ * hlb_get_stress_rows returns them); arrays no field uses may be NULL. */
 int hlb_xtr_write_fields(hlb_xtr_handle x, int64_t timestep, const double* rho, const double* u,
                          const double* wss, const double* f, const double* stress);
 int64_t hlb_xtr_site_count(hlb_xtr_handle x);
