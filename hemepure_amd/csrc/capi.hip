@@ -84,10 +84,7 @@ StepArgs make_args(hlb_lattice* h, const double* ain, double* aout) {
   a.gz = h->gz_tables();
   a.P = h->P64.p;
   a.GW = h->GW64.p;
-  a.bwall = h->bwall.p;
-  a.biolet = h->biolet.p;
-  a.bgi = h->bgi.p;
-  a.bii = h->bii.p;
+  a.bnd = h->bnd.p;
   a.bq = h->bq.p;
   a.bnrm = h->bnrm.p;
   a.G = h->G.p;
@@ -96,7 +93,6 @@ StepArgs make_args(hlb_lattice* h, const double* ain, double* aout) {
   a.rho = h->rho.p;
   a.u = h->u.p;
   a.wss = h->wss.p;
-  a.io_nf = h->io_nf.p;
   a.io_n = h->io_n.p;
   a.io_dens = h->io_dens.p;
   a.io_vmax = h->io_vmax.p;
@@ -109,7 +105,6 @@ StepArgs make_args(hlb_lattice* h, const double* ain, double* aout) {
   a.SB = h->SB;
   a.SI = h->SI;
   a.n_in = h->n_in;
-  a.wall_bc = h->params.wall_bc;
   a.inlet_bc = h->params.inlet_bc;
   a.outlet_bc = h->params.outlet_bc;
   a.tau = h->params.tau;
@@ -551,10 +546,7 @@ int upload_lattice(hlb_lattice* h) {
     HLB_CHECK(hipMemsetAsync(h->A[1].p, 0, sizeof(double) * Q * S, h->stream));
     HLB_CHECK(hipMemsetAsync(h->G.p, 0, sizeof(double) * Q * SI, h->stream));
   }
-  HLB_CHECK(h->bwall.alloc((size_t)SB));
-  HLB_CHECK(h->biolet.alloc((size_t)SB));
-  HLB_CHECK(h->bgi.alloc((size_t)SB));
-  HLB_CHECK(h->bii.alloc((size_t)SB));
+  HLB_CHECK(h->bnd.alloc((size_t)SB));
   HLB_CHECK(h->bq.alloc((size_t)18 * SB));
   HLB_CHECK(h->bnrm.alloc((size_t)3 * SB));
   HLB_CHECK(h->ladd_s.alloc((size_t)36 * SI));
@@ -600,24 +592,29 @@ int upload_lattice(hlb_lattice* h) {
   {
     std::vector<int32_t> iolIndex(N, -1);
     for (int64_t i = 0; i < h->NI; ++i) iolIndex[h->isite[i]] = (int32_t)i;
-    std::vector<uint32_t> w(SB, 0), io(SB, 0);
-    std::vector<int32_t> gi(SB, -1), ii(SB, -1);
+    std::vector<BndRec> rec(SB, BndRec{0, 0, 0, 0});
     std::vector<float> q((size_t)18 * SB, 0.0f), nr((size_t)3 * SB, 0.0f);
     for (int64_t b = 0; b < NB; ++b) {
       const int64_t k = h->bsite[b];
-      w[b] = L.wall[k];
-      io[b] = L.iolet[k];
+      BndRec& R = rec[b];
+      const uint32_t wm = L.wall[k];
+      R.iolet = L.iolet[k];
+      if (wm != 0) R.far |= 1u << 31;
+      // BouzidiFirdaousLallemandDelegate.h:44-93: a wall link whose opposite is
+      // no wall interpolates, with the site's own opposite value from q = 1/2 on
+      for (int j = 1; j < Q && h->params.wall_bc == HLB_WALL_BFL; ++j) {
+        const int ib = INV[j];
+        if (!((wm >> (ib - 1)) & 1u) || ((wm >> (j - 1)) & 1u)) continue;
+        (L.q[k * 18 + ib - 1] < 0.5f ? R.near : R.far) |= 1u << (j - 1);
+      }
       if (k >= L.off[2]) {
-        gi[b] = side_iolet(h, k);
-        ii[b] = iolIndex[k];
+        R.near |= (uint32_t)side_iolet(h, k) << 18;
+        R.ii = (uint32_t)iolIndex[k];
       }
       for (int d = 0; d < 18; ++d) q[(size_t)d * SB + b] = L.q[k * 18 + d];
       for (int a = 0; a < 3; ++a) nr[(size_t)a * SB + b] = L.nrm[k * 3 + a];
     }
-    HLB_CHECK(hipMemcpy(h->bwall.p, w.data(), sizeof(uint32_t) * SB, hipMemcpyHostToDevice));
-    HLB_CHECK(hipMemcpy(h->biolet.p, io.data(), sizeof(uint32_t) * SB, hipMemcpyHostToDevice));
-    HLB_CHECK(hipMemcpy(h->bgi.p, gi.data(), sizeof(int32_t) * SB, hipMemcpyHostToDevice));
-    HLB_CHECK(hipMemcpy(h->bii.p, ii.data(), sizeof(int32_t) * SB, hipMemcpyHostToDevice));
+    HLB_CHECK(hipMemcpy(h->bnd.p, rec.data(), sizeof(BndRec) * SB, hipMemcpyHostToDevice));
     HLB_CHECK(hipMemcpy(h->bq.p, q.data(), sizeof(float) * q.size(), hipMemcpyHostToDevice));
     HLB_CHECK(hipMemcpy(h->bnrm.p, nr.data(), sizeof(float) * nr.size(), hipMemcpyHostToDevice));
   }
@@ -876,10 +873,7 @@ Member32 member_record(const hlb_lattice* h, int props_at) {
   m.gz = h->gz_tables();
   m.P = h->P32.p;
   m.GW = h->GW32.p;
-  m.bwall = h->bwall.p;
-  m.biolet = h->biolet.p;
-  m.bgi = h->bgi.p;
-  m.bii = h->bii.p;
+  m.bnd = h->bnd.p;
   m.bq = h->bq.p;
   m.bnrm = h->bnrm.p;
   m.G = h->G32.p;
@@ -903,7 +897,6 @@ Member32 member_record(const hlb_lattice* h, int props_at) {
   m.nio = std::max<int>(1, (int)h->iolets.size());
   m.n_in = h->n_in;
   m.kernel = h->params.kernel;
-  m.wall_bc = h->params.wall_bc;
   m.inlet_bc = h->params.inlet_bc;
   m.outlet_bc = h->params.outlet_bc;
   m.cur0 = h->cur;

@@ -139,9 +139,9 @@ __device__ __forceinline__ uint32_t lanes_below(uint64_t mask) {
 // of fluid positions below DELTA are scalar work and the per-lane count is
 // one mbcnt pair.
 template <int DELTA>
-__device__ __forceinline__ uint32_t shifted_slot(uint64_t m, int32_t base, uint64_t& fluid) {
+__device__ __forceinline__ uint32_t shifted_slot(uint64_t m, uint32_t base, uint64_t& fluid) {
   uint64_t ms = m;
-  uint32_t add = (uint32_t)base;
+  uint32_t add = base;
   if constexpr (DELTA > 0) {
     ms = m >> DELTA;
     add += (uint32_t)__builtin_popcountll(m & ((1ull << DELTA) - 1ull));
@@ -164,9 +164,10 @@ constexpr uint64_t kLanesZ0 = 0x0101010101010101ull, kLanesZ7 = 0x80808080808080
 // lanes whose y / z step leaves the brick -- 64 or 8 positions back in the
 // neighbouring brick's slab: at most four candidates, each one mbcnt pair,
 // picked with constant lane masks; the fluid test combines the candidates'
-// shifted masks with scalar logic into one lane mask.
+// shifted masks with scalar logic into one lane mask.  plus (wave-uniform) is
+// added to every candidate's base, scalar work as well.
 template <int J>
-__device__ __forceinline__ uint32_t upstream_pos(const Lane& L, uint64_t& fluid_lanes) {
+__device__ __forceinline__ uint32_t upstream_pos(const Lane& L, uint64_t& fluid_lanes, uint32_t plus = 0) {
   constexpr int ox = -CX[J], oy = -CY[J], oz = -CZ[J];
   constexpr int d00 = 8 * oy + oz;
   // lanes whose step leaves the brick in y / in z
@@ -177,32 +178,65 @@ __device__ __forceinline__ uint32_t upstream_pos(const Lane& L, uint64_t& fluid_
   // constant entry indices only, so the masks and bases stay in scalar registers
   constexpr int e00 = reach_entry(ox, 0, 0);
   uint64_t m00 = 0;
-  uint32_t slot = shifted_slot<d00>(L.fm[e00], L.base[e00], m00);
+  uint32_t slot = shifted_slot<d00>(L.fm[e00], (uint32_t)L.base[e00] + plus, m00);
   uint64_t fluid = m00 & ~(Y | Z);
   if constexpr (oy != 0 && oz != 0) {
     static_assert(ox == 0, "D3Q19 links have at most two nonzero components");
     constexpr int e10 = reach_entry(0, oy, 0), e01 = reach_entry(0, 0, oz), e11 = reach_entry(0, oy, oz);
     uint64_t m10 = 0, m01 = 0, m11 = 0;
-    const uint32_t s10 = shifted_slot<d00 - 64 * oy>(L.fm[e10], L.base[e10], m10);
-    const uint32_t s01 = shifted_slot<d00 - 8 * oz>(L.fm[e01], L.base[e01], m01);
-    const uint32_t s11 = shifted_slot<d00 - 64 * oy - 8 * oz>(L.fm[e11], L.base[e11], m11);
+    const uint32_t s10 = shifted_slot<d00 - 64 * oy>(L.fm[e10], (uint32_t)L.base[e10] + plus, m10);
+    const uint32_t s01 = shifted_slot<d00 - 8 * oz>(L.fm[e01], (uint32_t)L.base[e01] + plus, m01);
+    const uint32_t s11 = shifted_slot<d00 - 64 * oy - 8 * oz>(L.fm[e11], (uint32_t)L.base[e11] + plus, m11);
     slot = yo ? (zo ? s11 : s10) : (zo ? s01 : slot);
     fluid |= (m10 & (Y & ~Z)) | (m01 & (Z & ~Y)) | (m11 & (Y & Z));
   } else if constexpr (oy != 0) {
     constexpr int e10 = reach_entry(ox, oy, 0);
     uint64_t m10 = 0;
-    const uint32_t s10 = shifted_slot<d00 - 64 * oy>(L.fm[e10], L.base[e10], m10);
+    const uint32_t s10 = shifted_slot<d00 - 64 * oy>(L.fm[e10], (uint32_t)L.base[e10] + plus, m10);
     slot = yo ? s10 : slot;
     fluid |= m10 & Y;
   } else if constexpr (oz != 0) {
     constexpr int e01 = reach_entry(ox, 0, oz);
     uint64_t m01 = 0;
-    const uint32_t s01 = shifted_slot<d00 - 8 * oz>(L.fm[e01], L.base[e01], m01);
+    const uint32_t s01 = shifted_slot<d00 - 8 * oz>(L.fm[e01], (uint32_t)L.base[e01] + plus, m01);
     slot = zo ? s01 : slot;
     fluid |= m01 & Z;
   }
   fluid_lanes = fluid;
   return slot;
+}
+
+// The steady step's gather of pull direction J.  The planes of an opposite
+// pair (J, INV[J]) are adjacent, so both are reached from the lower one with a
+// 32-bit element offset (2 S elements; see launch_step_fp64 for FP64's limit):
+// where the upstream position is not fluid (a wall or iolet link ib = INV[J])
+// the lane reads its own value in plane ib -- the bounce-back value, which SBB
+// keeps, BFL keeps or interpolates from and iolet and GZS links replace -- so
+// no boundary delegate loads it.  The pair's plane offset is folded into the
+// scalar bases, and own[k] (the own slot in the k-th plane of a pair) into two
+// values a lane forms once, so the choice costs one select.
+template <int J, typename T>
+__device__ __forceinline__ T gather_bb(const T* lower, uint32_t S, const Lane& L, const uint32_t (&own)[2]) {
+  constexpr bool upper = J > INV[J];
+  uint64_t fluid = 0;
+  const uint32_t up = upstream_pos<J>(L, fluid, upper ? S : 0u);
+  return ldp(lower, __builtin_amdgcn_inverse_ballot_w64(fluid) ? up : own[upper ? 0 : 1]);
+}
+
+// Velocity iolet links whose profile factors are loaded together: in groups of
+// three the delegate needs no more registers than the collision.
+constexpr int kLaddGroup = 3;
+
+// A boundary site's record (BndRec), read with one 16-byte load.
+struct Bnd {
+  uint32_t far, near, iolet, gi, ii;
+  bool wall;
+};
+__device__ __forceinline__ Bnd no_bnd() { return Bnd{0, 0, 0, 0, 0, false}; }
+__device__ __forceinline__ Bnd load_bnd(const BndRec* rec, uint32_t b) {
+  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+  const u32x4 v = *(const HLB_GLOBAL u32x4*)(rec + b);
+  return Bnd{v.x & kLinkBits, v.y & kLinkBits, v.z, v.y >> 18, v.w, (v.x >> 31) != 0};
 }
 
 template <int J>

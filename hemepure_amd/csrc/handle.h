@@ -114,8 +114,7 @@ struct hlb_lattice {
   std::vector<int32_t> isite;  // reference index of iolet slot i
   int64_t S = 0, NB = 0, SB = 0, NI = 0, SI = 0;
   hlb::DevBuf<double> A[2], F, G, ladd_s, rho, u, wss, io_n, io_dens, io_vmax, io_vmax2, feq_vals;
-  hlb::DevBuf<uint32_t> bwall, biolet;
-  hlb::DevBuf<int32_t> bgi, bii;
+  hlb::DevBuf<hlb::BndRec> bnd;  // boundary records
   hlb::DevBuf<hlb::SlabRec> rec;  // slab records
   hlb::DevBuf<float> bq, bnrm, io_nf;
   hlb::DevBuf<int32_t> dinv;      // inv on the device (transfer.hip)

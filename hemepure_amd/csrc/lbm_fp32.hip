@@ -143,100 +143,143 @@ __device__ __forceinline__ Planes member_planes(const Member32& m, int step) {
   return p;
 }
 
-// The upstream gather, as gather_up in the FP64 pass: wall and iolet links
-// read the lane's own slot and the boundary delegates replace the value.
+// The upstream gather (gather_bb): bounce-back values in the place of wall
+// and iolet links.
 template <int J = 1>
-__device__ __forceinline__ void gather_up32(const float* in, int64_t S, const Lane& L, float* g) {
+__device__ __forceinline__ void gather_up32(const float* in, int64_t S, const Lane& L, const uint32_t (&own)[2],
+                                            float* g) {
   if constexpr (J < Q) {
-    g[J] = ldp(uplane(in, S, J), upstream_slot<J>(L));
-    gather_up32<J + 1>(in, S, L, g);
+    g[J] = gather_bb<J>(uplane(in, S, J < INV[J] ? J : INV[J]), (uint32_t)S, L, own);
+    gather_up32<J + 1>(in, S, L, own, g);
   }
 }
 
-// The boundary delegates of one flagged site, as boundary_fixup in the FP64
+__device__ __forceinline__ void gather_site32(const float* in, int64_t S, const Lane& L, float* g) {
+  const uint32_t own[2] = {L.slot, L.slot + (uint32_t)S};
+  g[0] = ldp(in, L.slot);
+  gather_up32(in, S, L, own, g);
+}
+
+// The boundary delegates of one gathered site, as boundary_fixup in the FP64
 // pass (SimpleBounceBackDelegate.h:36-44, BouzidiFirdaousLallemandDelegate.h:
 // 44-93, iolet values from G).
 __device__ __forceinline__ void boundary_fixup32(const Member32& m, const float* in, uint32_t d, uint32_t b,
-                                                 uint32_t wm, uint32_t im, float* g) {
-  float own[Q];
-#pragma unroll
-  for (int j = 1; j < Q; ++j) own[j] = ldp(uplane(in, m.S, j), d);
-  const bool bfl = m.wall_bc == HLB_WALL_BFL;
-  float q[Q];
-  if (bfl && wm != 0) {
+                                                 const Bnd& r, float* g) {
+  float q[Q], own[Q];
+  if ((r.far | r.near) != 0) {
 #pragma unroll
     for (int k = 1; k < Q; ++k) q[k] = ldp(m.bq + (int64_t)(k - 1) * m.SB, b);
+    if (r.far != 0) {
+#pragma unroll
+      for (int j = 1; j < Q; ++j) own[j] = ldp(uplane(in, m.S, j), d);
+    }
   }
-  if (im != 0) {
-    const uint32_t i = (uint32_t)ldp(m.bii, b);
+  if (r.iolet != 0) {
 #pragma unroll
     for (int j = 1; j < Q; ++j)
-      if (im & (1u << (INV[j] - 1))) g[j] = ldp(plane(m.G, m.SI, j), i);
+      if (r.iolet & (1u << (INV[j] - 1))) g[j] = ldp(plane(m.G, m.SI, j), r.ii);
   }
-  uint32_t gzm = 0;
-  int32_t gzb = 0;
-  if (m.gz.bgz != nullptr && wm != 0) {
-    gzm = ldp(m.gz.bgz, b);
-    gzb = ldp(m.gz.bgzbase, b);
+  if (m.gz.bgz != nullptr && r.wall) {
+    const uint32_t gzm = ldp(m.gz.bgz, b);
+    const int32_t gzb = ldp(m.gz.bgzbase, b);
+#pragma unroll
+    for (int j = 1; j < Q; ++j) {
+      const uint32_t bit = 1u << (INV[j] - 1);
+      if (gzm & bit) g[j] = ldp(m.GW, (uint32_t)(gzb + __builtin_popcount(gzm & (bit - 1u))));
+    }
   }
-  if (wm != 0) {
+  if ((r.far | r.near) != 0) {
 #pragma unroll
     for (int j = 1; j < Q; ++j) {
       const int ib = INV[j];
-      const uint32_t bit = 1u << (ib - 1), bitJ = 1u << (j - 1);
-      if ((wm & bit) && !(im & bit)) {
-        if (gzm & bit) {
-          g[j] = ldp(m.GW, (uint32_t)(gzb + __builtin_popcount(gzm & (bit - 1u))));
-          continue;
-        }
-        const float qd = bfl ? q[ib] : 0.0f;
-        if (!bfl || (wm & bitJ) || qd < 0.5f) g[j] = own[ib];
-        else g[j] = (own[ib] + (2.0f * qd - 1.0f) * own[j]) / (2.0f * qd);
-      }
-    }
-    if (bfl) {
-#pragma unroll
-      for (int k = 1; k < Q; ++k) {
-        const int j = INV[k];
-        const float qk = q[k];
-        if ((wm & (1u << (k - 1))) && !(wm & (1u << (j - 1))) && qk < 0.5f)
-          g[j] = 2.0f * qk * g[j] + (1.0f - 2.0f * qk) * g[k];
-      }
+      const float q2 = 2.0f * q[ib];
+      if (r.near & (1u << (j - 1))) g[j] = q2 * g[j] + (1.0f - q2) * g[ib];
+      if (r.far & (1u << (j - 1))) g[j] = (g[j] + (q2 - 1.0f) * own[j]) / q2;
     }
   }
 }
 
-// Nash ghost equilibrium / Ladd moving-wall bounce-back for each iolet link
-// (NashZerothOrderPressureDelegate.h:36-76, LaddIoletDelegate.h:37-86), in
-// shifted form.
+// What the Nash delegates of a site read per iolet, loaded ahead of the
+// collision: ghost density, its deviation, the normal, the Windkessel link.
+struct IoletIn32 {
+  float rho, drho, n[3];
+  uint32_t wk;
+};
+__device__ __forceinline__ IoletIn32 load_iolet32(const Member32& m, int step, uint32_t gi) {
+  const double dens = ldp(m.io_dens + (int64_t)step * m.nio, gi);
+  return IoletIn32{(float)dens,
+                   (float)(dens - 1.0),
+                   {ldp(m.io_nf, 3u * gi), ldp(m.io_nf, 3u * gi + 1), ldp(m.io_nf, 3u * gi + 2)},
+                   ldp(m.wk_bit, gi)};
+}
+
 template <int D = 1>
-__device__ __forceinline__ void iolet_links32(const Member32& m, const double* dens, const double* vmax,
-                                              const double* vmax2, uint32_t i, uint32_t im, int gi, int bc, float rho, float vx,
-                                              float vy, float vz, const float* gpost) {
+__device__ __forceinline__ void nash_links32(const Member32& m, const Bnd& r, float drg, float inv, float usq15,
+                                             float gx, float gy, float gz) {
   if constexpr (D < Q) {
-    constexpr int U = INV[D];
-    if (im & (1u << (D - 1))) {
-      float val;
-      if (bc == HLB_IOLET_NASH) {
-        const double rgd = ldp(dens, (uint32_t)gi);
-        const float rg = (float)rgd, drg = (float)(rgd - 1.0);
-        const float nx = ldp(m.io_nf, 3u * gi), ny = ldp(m.io_nf, 3u * gi + 1), nz = ldp(m.io_nf, 3u * gi + 2);
-        const float component = vx * nx + vy * ny + vz * nz;
-        const float gx = nx * component * rg, gy = ny * component * rg, gz = nz * component * rg;
-        const float inv = 1.0f / rg;
-        const float usq15 = 1.5f * (gx * gx + gy * gy + gz * gz) * inv;
-        val = geq_dir<U>(drg, inv, usq15, gx, gy, gz);
-      } else {
-        const float s = (float)(ldp(vmax, (uint32_t)gi) * ldp(m.ladd_s + (int64_t)(D - 1) * m.SI, i) +
-                                ldp(vmax2, (uint32_t)gi) * ldp(m.ladd_s2 + (int64_t)(D - 1) * m.SI, i));
-        const float wx = (float)ldp(m.io_n, 3u * gi) * s * rho, wy = (float)ldp(m.io_n, 3u * gi + 1) * s * rho,
-                    wz = (float)ldp(m.io_n, 3u * gi + 2) * s * rho;
-        const float correction = 2.0f * wf(D) * cdotf<D>(wx, wy, wz) * 3.0f;
-        val = gpost[D] - correction;
-      }
-      stp(plane(m.G, m.SI, U), i, val);
+    if (r.iolet & (1u << (D - 1)))
+      stp(plane(m.G, m.SI, INV[D]), r.ii, geq_dir<INV[D]>(drg, inv, usq15, gx, gy, gz));
+    nash_links32<D + 1>(m, r, drg, inv, usq15, gx, gy, gz);
+  }
+}
+
+struct LaddIn32 {
+  double vmax, vmax2;  // the step's speed factors
+  float n[3];
+};
+
+template <int D0, int D = D0>
+__device__ __forceinline__ void ladd_links32(const Member32& m, const Bnd& r, const LaddIn32& io, const double* s,
+                                             const double* s2, float rho, const float* gpost) {
+  if constexpr (D < Q && D < D0 + kLaddGroup) {
+    if (r.iolet & (1u << (D - 1))) {
+      const float v = (float)(io.vmax * s[D - D0] + io.vmax2 * s2[D - D0]);
+      const float wx = io.n[0] * v * rho, wy = io.n[1] * v * rho, wz = io.n[2] * v * rho;
+      const float correction = 2.0f * wf(D) * cdotf<D>(wx, wy, wz) * 3.0f;
+      stp(plane(m.G, m.SI, INV[D]), r.ii, gpost[D] - correction);
     }
-    iolet_links32<D + 1>(m, dens, vmax, vmax2, i, im, gi, bc, rho, vx, vy, vz, gpost);
+    ladd_links32<D0, D + 1>(m, r, io, s, s2, rho, gpost);
+  }
+}
+
+// The profile factors of kLaddGroup links at a time, then their values.
+template <int D0 = 1>
+__device__ __forceinline__ void ladd_groups32(const Member32& m, const Bnd& r, const LaddIn32& io, float rho,
+                                              const float* gpost) {
+  if constexpr (D0 < Q) {
+    double s[kLaddGroup], s2[kLaddGroup];
+#pragma unroll
+    for (int e = 0; e < kLaddGroup; ++e) {
+      if (!(r.iolet & (1u << (D0 + e - 1)))) continue;
+      s[e] = ldp(m.ladd_s + (int64_t)(D0 + e - 1) * m.SI, r.ii);
+      s2[e] = ldp(m.ladd_s2 + (int64_t)(D0 + e - 1) * m.SI, r.ii);
+    }
+    ladd_links32<D0>(m, r, io, s, s2, rho, gpost);
+    ladd_groups32<D0 + kLaddGroup>(m, r, io, rho, gpost);
+  }
+}
+
+// Nash ghost equilibrium (one per site) / Ladd moving-wall bounce-back for
+// each iolet link (NashZerothOrderPressureDelegate.h:36-76,
+// LaddIoletDelegate.h:37-86), in shifted form, and the Windkessel coupling
+// site's flux term.
+__device__ __forceinline__ void iolet_links32(const Member32& m, int step, const Bnd& r, const IoletIn32& io, float rho,
+                                              float vx, float vy, float vz, const float* gpost) {
+  if (((int)r.gi < m.n_in ? m.inlet_bc : m.outlet_bc) == HLB_IOLET_NASH) {
+    const float component = vx * io.n[0] + vy * io.n[1] + vz * io.n[2];
+    const float gx = io.n[0] * component * io.rho, gy = io.n[1] * component * io.rho, gz = io.n[2] * component * io.rho;
+    const float inv = 1.0f / io.rho;
+    const float usq15 = 1.5f * (gx * gx + gy * gy + gz * gz) * inv;
+    nash_links32(m, r, io.drho, inv, usq15, gx, gy, gz);
+  } else {
+    const int64_t row = (int64_t)step * m.nio;
+    ladd_groups32(m, r, LaddIn32{ldp(m.io_vmax + row, r.gi), ldp(m.io_vmax2 + row, r.gi), {io.n[0], io.n[1], io.n[2]}},
+                  rho, gpost);
+  }
+  if (r.iolet & io.wk) {
+    const double c = (double)vx * -ldp(m.io_n, 3u * r.gi) + (double)vy * -ldp(m.io_n, 3u * r.gi + 1) +
+                     (double)vz * -ldp(m.io_n, 3u * r.gi + 2);
+    stp(m.wk_contrib, (uint32_t)ldp(m.wk_pos, r.ii), c);
   }
 }
 
@@ -349,50 +392,42 @@ __device__ __forceinline__ int member_of_tile(const int32_t* wg_member, uint32_t
   return wg_member ? __builtin_amdgcn_readfirstlane(ldp(wg_member, tile)) : 0;
 }
 
-// One site of a slab in flight: its lane, boundary masks and the
+// One site of a slab in flight: its lane, boundary record and the
 // pre-collision g being assembled.
 struct Site32 {
   Lane L;
   bool ok;
-  uint32_t wm, im;
+  Bnd bnd;
   float g[Q];
 };
 
 // Decodes slab record r for this lane and issues the site's gathers (the
 // loads are not waited for here).
 __device__ __forceinline__ void site_gather32(const Member32& m, const Planes& P, uint32_t r, Site32& s) {
-  s.wm = 0;
-  s.im = 0;
+  s.bnd = no_bnd();
   s.ok = slab_lane(m.bt, r, s.L);
   if (!s.ok) return;
-  const uint32_t d = s.L.slot;
-  if (s.L.boundary) {
-    s.wm = ldp(m.bwall, s.L.b);
-    s.im = ldp(m.biolet, s.L.b);
-  }
+  if (s.L.boundary) s.bnd = load_bnd(m.bnd, s.L.b);
   if (P.first) {
 #pragma unroll
-    for (int j = 0; j < Q; ++j) s.g[j] = ldp(uplane(P.in, m.S, j), d);
+    for (int j = 0; j < Q; ++j) s.g[j] = ldp(uplane(P.in, m.S, j), s.L.slot);
   } else {
-    s.g[0] = ldp(P.in, d);
-    gather_up32(P.in, m.S, s.L, s.g);
+    gather_site32(P.in, m.S, s.L, s.g);
   }
 }
 
 // The boundary delegates, the GZS staging, collision, stores, iolet values
 // and property fields of one gathered site.
 template <bool NT>
-__device__ __forceinline__ void site_finish32(const Member32& m, const Planes& P, int step, Site32& s) {
-  if (!s.ok) return;
-  const uint32_t d = s.L.slot;
-  const bool isB = s.L.boundary;
-  const uint32_t wm = s.wm, im = s.im;
-  float* g = s.g;
-  if (!P.first && isB) boundary_fixup32(m, P.in, d, s.L.b, wm, im, g);
+__device__ __forceinline__ void site_finish32(const Member32& m, const Planes& P, int step, const Lane& L, const Bnd& bnd,
+                                              const float* g) {
+  const uint32_t d = L.slot;
+  IoletIn32 io{};
+  if (bnd.iolet != 0) io = load_iolet32(m, step, bnd.gi);
   if (m.gz.pmask != nullptr) {
-    const uint64_t pm = uniform64(ldp(m.gz.pmask, s.L.r));
+    const uint64_t pm = uniform64(ldp(m.gz.pmask, L.r));
     if ((pm >> (threadIdx.x & 63u)) & 1u) {
-      const uint32_t pi = (uint32_t)__builtin_amdgcn_readfirstlane(ldp(m.gz.pbase, s.L.r)) + lanes_below(pm);
+      const uint32_t pi = (uint32_t)__builtin_amdgcn_readfirstlane(ldp(m.gz.pbase, L.r)) + lanes_below(pm);
 #pragma unroll
       for (int j = 0; j < Q; ++j) stp(plane(m.P, m.gz.SP, j), pi, g[j]);
     }
@@ -402,31 +437,13 @@ __device__ __forceinline__ void site_finish32(const Member32& m, const Planes& P
   const Collision32 cs = collide32(m, step, d, g, gpost);
   store_row32<NT>(m, P.out, d, gpost);
 
-  const bool props = step == m.props_at;
-  float w = FLT_MAX;
-  if (isB) {
-    const uint32_t b = s.L.b;
-    const int32_t ii = ldp(m.bii, b);
-    if (ii >= 0) {
-      const int gi = ldp(m.bgi, b);
-      const int bc = gi < m.n_in ? m.inlet_bc : m.outlet_bc;
-      const double* dens = m.io_dens + (int64_t)step * m.nio;
-      const double* vmax = m.io_vmax + (int64_t)step * m.nio;
-      const double* vmax2 = m.io_vmax2 + (int64_t)step * m.nio;
-      iolet_links32(m, dens, vmax, vmax2, (uint32_t)ii, im, gi, bc, cs.rho, cs.ux, cs.uy, cs.uz, gpost);
-      if (im & ldp(m.wk_bit, (uint32_t)gi)) {
-        const double c = (double)cs.ux * -ldp(m.io_n, 3u * gi) + (double)cs.uy * -ldp(m.io_n, 3u * gi + 1) +
-                         (double)cs.uz * -ldp(m.io_n, 3u * gi + 2);
-        stp(m.wk_contrib, (uint32_t)ldp(m.wk_pos, (uint32_t)ii), c);
-      }
-    }
-    if (props && wm != 0) w = wall_shear_stress32(m, b, cs.tau, g, gpost);
-  }
-  if (props) {
+  if (bnd.iolet != 0) iolet_links32(m, step, bnd, io, cs.rho, cs.ux, cs.uy, cs.uz, gpost);
+  if (step == m.props_at) {
     stp(m.rho, d, 1.0 + (double)cs.drho);
     stp(m.u, d, (double)cs.ux);
     stp(plane(m.u, m.S, 1), d, (double)cs.uy);
     stp(plane(m.u, m.S, 2), d, (double)cs.uz);
+    const float w = bnd.wall ? wall_shear_stress32(m, L.b, cs.tau, g, gpost) : FLT_MAX;
     stp(m.wss, d, w == FLT_MAX ? DBL_MAX : (double)w);
   }
 }
@@ -437,84 +454,37 @@ __device__ __forceinline__ void site_finish32(const Member32& m, const Planes& P
 template <int B, int ORDER, int W = 0, int SPT = 1, bool NT = false>
 __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(W > 0 ? W : 1))) void step_fp32(
     const Member32* __restrict__ members, const int32_t* __restrict__ wg_member, int step) {
+  const uint32_t tile = tile_index<ORDER>();
+  const int mi = member_of_tile(wg_member, tile);
+  if (mi < 0) return;  // padding tile
+  const Member32& m = members[mi];
+  const uint32_t r0 =
+      ((tile - m.wg_begin) * (B / kSlab) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * (uint32_t)SPT;
+  const Planes P = member_planes(m, step);
   if constexpr (SPT == 1) {
-    const uint32_t tile = tile_index<ORDER>();
-    const int mi = member_of_tile(wg_member, tile);
-    if (mi < 0) return;  // padding tile
-    const Member32& m = members[mi];
-    const uint32_t r = (tile - m.wg_begin) * (B / kSlab) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     Lane L;
-    if (!slab_lane(m.bt, r, L)) return;
-    const uint32_t d = L.slot;
-    const bool isB = L.boundary;
-    uint32_t wm = 0, im = 0;
-    if (isB) {
-      wm = ldp(m.bwall, L.b);
-      im = ldp(m.biolet, L.b);
-    }
-    const Planes P = member_planes(m, step);
+    if (!slab_lane(m.bt, r0, L)) return;
+    Bnd bnd = no_bnd();
+    if (L.boundary) bnd = load_bnd(m.bnd, L.b);
     float g[Q];
     if (P.first) {
 #pragma unroll
-      for (int j = 0; j < Q; ++j) g[j] = ldp(uplane(P.in, m.S, j), d);
+      for (int j = 0; j < Q; ++j) g[j] = ldp(uplane(P.in, m.S, j), L.slot);
     } else {
-      g[0] = ldp(P.in, d);
-      gather_up32(P.in, m.S, L, g);
-      if (isB) boundary_fixup32(m, P.in, d, L.b, wm, im, g);
+      gather_site32(P.in, m.S, L, g);
+      if (L.boundary) boundary_fixup32(m, P.in, L.slot, L.b, bnd, g);
     }
-    if (m.gz.pmask != nullptr) {
-      const uint64_t pm = uniform64(ldp(m.gz.pmask, L.r));
-      if ((pm >> (threadIdx.x & 63u)) & 1u) {
-        const uint32_t pi = (uint32_t)__builtin_amdgcn_readfirstlane(ldp(m.gz.pbase, L.r)) + lanes_below(pm);
-#pragma unroll
-        for (int j = 0; j < Q; ++j) stp(plane(m.P, m.gz.SP, j), pi, g[j]);
-      }
-    }
-
-    float gpost[Q];
-    const Collision32 cs = collide32(m, step, d, g, gpost);
-    store_row32<NT>(m, P.out, d, gpost);
-
-    const bool props = step == m.props_at;
-    float w = FLT_MAX;
-    if (isB) {
-      const uint32_t b = L.b;
-      const int32_t ii = ldp(m.bii, b);
-      if (ii >= 0) {
-        const int gi = ldp(m.bgi, b);
-        const int bc = gi < m.n_in ? m.inlet_bc : m.outlet_bc;
-        const double* dens = m.io_dens + (int64_t)step * m.nio;
-        const double* vmax = m.io_vmax + (int64_t)step * m.nio;
-        const double* vmax2 = m.io_vmax2 + (int64_t)step * m.nio;
-        iolet_links32(m, dens, vmax, vmax2, (uint32_t)ii, im, gi, bc, cs.rho, cs.ux, cs.uy, cs.uz, gpost);
-        if (im & ldp(m.wk_bit, (uint32_t)gi)) {
-          const double c = (double)cs.ux * -ldp(m.io_n, 3u * gi) + (double)cs.uy * -ldp(m.io_n, 3u * gi + 1) +
-                           (double)cs.uz * -ldp(m.io_n, 3u * gi + 2);
-          stp(m.wk_contrib, (uint32_t)ldp(m.wk_pos, (uint32_t)ii), c);
-        }
-      }
-      if (props && wm != 0) w = wall_shear_stress32(m, b, cs.tau, g, gpost);
-    }
-    if (props) {
-      stp(m.rho, d, 1.0 + (double)cs.drho);
-      stp(m.u, d, (double)cs.ux);
-      stp(plane(m.u, m.S, 1), d, (double)cs.uy);
-      stp(plane(m.u, m.S, 2), d, (double)cs.uz);
-      stp(m.wss, d, w == FLT_MAX ? DBL_MAX : (double)w);
-    }
+    site_finish32<NT>(m, P, step, L, bnd, g);
   } else {
-    const uint32_t tile = tile_index<ORDER>();
-    const int mi = member_of_tile(wg_member, tile);
-    if (mi < 0) return;  // padding tile
-    const Member32& m = members[mi];
-    const uint32_t r0 =
-        ((tile - m.wg_begin) * (B / kSlab) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * (uint32_t)SPT;
-    const Planes P = member_planes(m, step);
     Site32 s[SPT];
 #pragma unroll
     for (int k = 0; k < SPT; ++k) site_gather32(m, P, r0 + (uint32_t)k, s[k]);
 #pragma unroll
-    for (int k = 0; k < SPT; ++k) site_finish32<NT>(m, P, step, s[k]);
+    for (int k = 0; k < SPT; ++k) {
+      if (!s[k].ok) continue;
+      if (!P.first && s[k].L.boundary) boundary_fixup32(m, P.in, s[k].L.slot, s[k].L.b, s[k].bnd, s[k].g);
+      site_finish32<NT>(m, P, step, s[k].L, s[k].bnd, s[k].g);
+    }
   }
 }
 
@@ -590,15 +560,11 @@ __global__ __launch_bounds__(kBlock) void gather_fp32(const Member32* __restrict
   Lane L;
   if (!slab_lane(m.bt, slab_record4(), L)) return;
   const float* in = m.A[m.cur0];
-  uint32_t wm = 0, im = 0;
-  if (L.boundary) {
-    wm = ldp(m.bwall, L.b);
-    im = ldp(m.biolet, L.b);
-  }
+  Bnd bnd = no_bnd();
+  if (L.boundary) bnd = load_bnd(m.bnd, L.b);
   float g[Q];
-  g[0] = ldp(in, L.slot);
-  gather_up32(in, m.S, L, g);
-  if (L.boundary) boundary_fixup32(m, in, L.slot, L.b, wm, im, g);
+  gather_site32(in, m.S, L, g);
+  if (L.boundary) boundary_fixup32(m, in, L.slot, L.b, bnd, g);
 #pragma unroll
   for (int j = 0; j < Q; ++j) stp(plane(F, m.S, j), L.slot, g[j]);
 }

@@ -36,189 +36,139 @@ namespace hlb {
 
 namespace {
 
-// Gathers the upstream post-collision values.  A direction whose upstream
-// position is not fluid (a wall or iolet link) reads the lane's own slot, a
-// line the wave fetches anyway, and the boundary delegates replace the value;
-// the choice needs only the slab record, so the gathers do not wait on the
-// boundary masks.
-template <int J = 1>
-__device__ __forceinline__ void gather_up(const double* const* ain, const Lane& L, double* f) {
+// Gathers the pre-collision values, bounce-back ones in the place of wall and
+// iolet links.  NARROW: each pair of opposite planes fits 32-bit offsets from
+// its lower plane; otherwise the plane is picked with the 64-bit address.
+template <bool NARROW, int J = 1>
+__device__ __forceinline__ void gather_up(const StepArgs& a, const Lane& L, const uint32_t (&own)[2], double* f) {
   if constexpr (J < Q) {
-    f[J] = ldp(ain[J], upstream_slot<J>(L));
-    gather_up<J + 1>(ain, L, f);
+    if constexpr (NARROW) {
+      f[J] = gather_bb<J>(a.ain[J < INV[J] ? J : INV[J]], (uint32_t)a.S, L, own);
+    } else {
+      uint64_t fluid = 0;
+      const uint32_t up = upstream_pos<J>(L, fluid);
+      const bool plain = __builtin_amdgcn_inverse_ballot_w64(fluid);
+      f[J] = *(const HLB_GLOBAL double*)((plain ? a.ain[J] : a.ain[INV[J]]) + (plain ? up : L.slot));
+    }
+    gather_up<NARROW, J + 1>(a, L, own, f);
   }
 }
 
+template <bool NARROW>
 __device__ __forceinline__ void gather_site(const StepArgs& a, const Lane& L, double* f) {
+  const uint32_t own[2] = {L.slot, L.slot + (uint32_t)a.S};
   f[0] = ldp(a.ain[0], L.slot);
-  gather_up(a.ain, L, f);
+  gather_up<NARROW>(a, L, own, f);
 }
 
-// Boundary sites: per direction j the writer of the value is the site's link
-// INV[j] -- an iolet delegate (value kept in G), a wall delegate (the site's
-// own post-collision values) or the neighbour (already gathered).  The own
-// row and the link distances are loaded before any selection so a wave waits
-// on one round of loads.
-__device__ __forceinline__ void boundary_fixup(const StepArgs& a, uint32_t d, uint32_t b, uint32_t wm,
-                                               uint32_t im, double* f) {
-  double own[Q];
-#pragma unroll
-  for (int j = 1; j < Q; ++j) own[j] = ldp(a.ain[j], d);
-  const bool bfl = a.wall_bc == HLB_WALL_BFL;
+// The boundary delegates of one gathered site: f[j] already holds the site's
+// own post-collision value for every wall or iolet link INV[j], which is all
+// SimpleBounceBackDelegate.h:36-44 does.
+//
+// A wave with boundary lanes is bound by instructions and by the chain of
+// loads it waits for, not by bytes.  So what each direction does is worked out
+// on the host (BndRec: one bit test and, where no lane of the wave has it, one
+// skipped branch) and all loads are issued before any value is used.  With the
+// masks formed from the link masks per direction and the own values loaded
+// where they were needed, a wave spent ~800 more vector instructions and up to
+// a round of loads per link: the Y-bifurcation (0.70M sites) 46.2 -> 41.7 us a
+// step, the 30k-site cylinder, where the iolet layers' waves decide, 9.0 ->
+// 6.4 us, FP32: 29.1 -> 27.3 us, the 20-pipe ensemble 78.8 -> 72.9 us.
+__device__ __forceinline__ void boundary_fixup(const StepArgs& a, uint32_t d, uint32_t b, const Bnd& r, double* f) {
   float q[Q];
-  if (bfl && wm != 0) {
+  double own[Q];
+  if ((r.far | r.near) != 0) {
 #pragma unroll
     for (int k = 1; k < Q; ++k) q[k] = ldp(a.bq + (int64_t)(k - 1) * a.SB, b);
+    if (r.far != 0) {
+#pragma unroll
+      for (int j = 1; j < Q; ++j) own[j] = ldp(a.ain[j], d);
+    }
   }
-  if (im != 0) {
-    const uint32_t i = (uint32_t)ldp(a.bii, b);
+  if (r.iolet != 0) {
 #pragma unroll
     for (int j = 1; j < Q; ++j)
-      if (im & (1u << (INV[j] - 1))) f[j] = ldp(plane(a.G, a.SI, j), i);
+      if (r.iolet & (1u << (INV[j] - 1))) f[j] = ldp(plane(a.G, a.SI, j), r.ii);
   }
-  uint32_t gzm = 0;
-  int32_t gzb = 0;
-  if (a.gz.bgz != nullptr && wm != 0) {
-    gzm = ldp(a.gz.bgz, b);
-    gzb = ldp(a.gz.bgzbase, b);
+  if (a.gz.bgz != nullptr && r.wall) {
+    // GuoZhengShiDelegate: the link kernel's values.
+    const uint32_t gzm = ldp(a.gz.bgz, b);
+    const int32_t gzb = ldp(a.gz.bgzbase, b);
+#pragma unroll
+    for (int j = 1; j < Q; ++j) {
+      const uint32_t bit = 1u << (INV[j] - 1);
+      if (gzm & bit) f[j] = ldp(a.GW, (uint32_t)(gzb + __builtin_popcount(gzm & (bit - 1u))));
+    }
   }
-  if (wm != 0) {
+  if ((r.far | r.near) != 0) {
+    // BouzidiFirdaousLallemandDelegate.h: the stream of a wall link ib =
+    // INV[j] with q >= 1/2 (:44-70) and the post-step of one with q < 1/2
+    // (:72-93).  The post-step reads the streamed f[ib], which no other
+    // interpolation of the site writes.
 #pragma unroll
     for (int j = 1; j < Q; ++j) {
       const int ib = INV[j];
-      const uint32_t bit = 1u << (ib - 1), bitJ = 1u << (j - 1);
-      if ((wm & bit) && !(im & bit)) {
-        if (gzm & bit) {
-          // GuoZhengShiDelegate: the link kernel's value.
-          f[j] = ldp(a.GW, (uint32_t)(gzb + __builtin_popcount(gzm & (bit - 1u))));
-          continue;
-        }
-        // SimpleBounceBackDelegate.h:36-44; BFL StreamLink, :44-70.
-        const double qd = bfl ? (double)q[ib] : 0.0;
-        if (!bfl || (wm & bitJ) || qd < 0.5) f[j] = own[ib];
-        else f[j] = (own[ib] + (2.0 * qd - 1) * own[j]) / (2.0 * qd);
-      }
-    }
-    if (bfl) {
-      // BFL post-step for wall links k with q < 1/2 whose opposite link is
-      // not a wall (BouzidiFirdaousLallemandDelegate.h:72-93), in order.
-#pragma unroll
-      for (int k = 1; k < Q; ++k) {
-        const int j = INV[k];
-        const double qk = (double)q[k];
-        if ((wm & (1u << (k - 1))) && !(wm & (1u << (j - 1))) && qk < 0.5)
-          f[j] = 2.0 * qk * f[j] + (1.0 - 2.0 * qk) * f[k];
-      }
+      const double q2 = 2.0 * (double)q[ib];
+      if (r.near & (1u << (j - 1))) f[j] = q2 * f[j] + (1.0 - q2) * f[ib];
+      if (r.far & (1u << (j - 1))) f[j] = (f[j] + (q2 - 1) * own[j]) / q2;
     }
   }
 }
 
-// The steady gather when each pair of opposite planes (J, INV[J]) -- the
-// D3Q19 numbering pairs 2i-1 with 2i, adjacent in the allocation -- fits
-// 32-bit element offsets from its lower plane (2 S <= 2^29): a direction
-// whose upstream position is not fluid (a wall or iolet link ib = INV[J])
-// reads the lane's own value in plane ib -- the bounce-back value SBB keeps,
-// BFL keeps or interpolates from, an iolet or GZS link replaces -- so the
-// boundary delegates load no own row.  One load per direction either way:
-// the plane of the pair is picked per lane through the offset.
-template <int J = 1>
-__device__ __forceinline__ void gather_up_bb(const StepArgs& a, const Lane& L, double* f) {
-  if constexpr (J < Q) {
-    constexpr int lo = J < INV[J] ? J : INV[J];
-    uint64_t fluid = 0;
-    const uint32_t up = upstream_pos<J>(L, fluid);
-    const uint32_t pj = (uint32_t)((J - lo) * a.S), pi = (uint32_t)((INV[J] - lo) * a.S);
-    f[J] = ldp(a.ain[lo], __builtin_amdgcn_inverse_ballot_w64(fluid) ? pj + up : pi + L.slot);
-    gather_up_bb<J + 1>(a, L, f);
-  }
+// What the iolet delegates of a site read per iolet, loaded ahead of the
+// row's stores: ghost density, normal, the Windkessel link.
+struct IoletIn {
+  double dens, n[3];
+  uint32_t wk;
+};
+__device__ __forceinline__ IoletIn load_iolet(const StepArgs& a, uint32_t gi) {
+  return IoletIn{a.io_dens[gi], {a.io_n[3 * gi], a.io_n[3 * gi + 1], a.io_n[3 * gi + 2]}, a.wk_bit[gi]};
 }
 
-// boundary_fixup for gather_up_bb: f[j] already holds own[ib] for every wall
-// or iolet link ib; own[j] is read only where BFL interpolates.  Same
-// operations, in the same order, as boundary_fixup.
-__device__ __forceinline__ void boundary_fixup_bb(const StepArgs& a, uint32_t d, uint32_t b, uint32_t wm,
-                                                  uint32_t im, double* f) {
-  const bool bfl = a.wall_bc == HLB_WALL_BFL;
-  float q[Q];
-#pragma unroll
-  for (int k = 1; k < Q; ++k) q[k] = 0.0f;
-  if (bfl) {
-    // distances of the lane's wall links only (all loads first, then their uses)
-#pragma unroll
-    for (int k = 1; k < Q; ++k)
-      if (wm & (1u << (k - 1))) q[k] = ldp(a.bq + (int64_t)(k - 1) * a.SB, b);
-  }
-  if (im != 0) {
-    const uint32_t i = (uint32_t)ldp(a.bii, b);
-#pragma unroll
-    for (int j = 1; j < Q; ++j)
-      if (im & (1u << (INV[j] - 1))) f[j] = ldp(plane(a.G, a.SI, j), i);
-  }
-  uint32_t gzm = 0;
-  int32_t gzb = 0;
-  if (a.gz.bgz != nullptr && wm != 0) {
-    gzm = ldp(a.gz.bgz, b);
-    gzb = ldp(a.gz.bgzbase, b);
-  }
-  if (wm != 0) {
-#pragma unroll
-    for (int j = 1; j < Q; ++j) {
-      const int ib = INV[j];
-      const uint32_t bit = 1u << (ib - 1), bitJ = 1u << (j - 1);
-      if ((wm & bit) && !(im & bit)) {
-        if (gzm & bit) {
-          f[j] = ldp(a.GW, (uint32_t)(gzb + __builtin_popcount(gzm & (bit - 1u))));
-          continue;
-        }
-        const double qd = bfl ? (double)q[ib] : 0.0;
-        if (bfl && !(wm & bitJ) && !(qd < 0.5)) f[j] = (f[j] + (2.0 * qd - 1) * ldp(a.ain[j], d)) / (2.0 * qd);
-      }
-    }
-    if (bfl) {
-#pragma unroll
-      for (int k = 1; k < Q; ++k) {
-        const int j = INV[k];
-        const double qk = (double)q[k];
-        if ((wm & (1u << (k - 1))) && !(wm & (1u << (j - 1))) && qk < 0.5)
-          f[j] = 2.0 * qk * f[j] + (1.0 - 2.0 * qk) * f[k];
-      }
-    }
+template <int D = 1>
+__device__ __forceinline__ void nash_links(const StepArgs& a, const Bnd& r, const FeqPre& p, double gx, double gy,
+                                           double gz) {
+  if constexpr (D < Q) {
+    if (r.iolet & (1u << (D - 1))) stp(plane(a.G, a.SI, INV[D]), r.ii, feq_dir<INV[D]>(p, gx, gy, gz));
+    nash_links<D + 1>(a, r, p, gx, gy, gz);
   }
 }
 
 // Iolet delegates of one site: the value each iolet link k hands to the next
-// step in direction INV[k].  Nash: f_eq of the ghost state
-// (NashZerothOrderPressureDelegate.h:36-76).  Ladd: bounce-back minus the
-// moving-wall correction (LaddIoletDelegate.h:37-86).
-template <int D = 1>
-__device__ __forceinline__ void iolet_links(const StepArgs& a, uint32_t i, uint32_t im, int gi, int bc,
-                                            double rho, double vx, double vy, double vz,
-                                            const double* fpost) {
-  if constexpr (D < Q) {
-    constexpr int U = INV[D];
-    if (im & (1u << (D - 1))) {
-      double val;
-      if (bc == HLB_IOLET_NASH) {
-        const double rg = a.io_dens[gi];
-        const double nx = (double)a.io_nf[3 * gi], ny = (double)a.io_nf[3 * gi + 1],
-                     nz = (double)a.io_nf[3 * gi + 2];
-        const double component = vx * nx + vy * ny + vz * nz;
-        const double gx = nx * component * rg, gy = ny * component * rg, gz = nz * component * rg;
-        const FeqPre p = feq_pre(rg, gx, gy, gz);
-        val = feq_dir<U>(p, gx, gy, gz);
-      } else {
-        // speed along the normal: vmax s (parabolic, file) or -Re(K e^{iwt}) (Womersley)
-        const double m = a.io_vmax[gi] * ldp(a.ladd_s + (int64_t)(D - 1) * a.SI, i) +
-                         a.io_vmax2[gi] * ldp(a.ladd_s2 + (int64_t)(D - 1) * a.SI, i);
-        const double wx = a.io_n[3 * gi] * m * rho, wy = a.io_n[3 * gi + 1] * m * rho,
-                     wz = a.io_n[3 * gi + 2] * m * rho;
-        const double correction =
-            2. * Wt(D) * (wx * (double)CX[D] + wy * (double)CY[D] + wz * (double)CZ[D]) / CS2;
-        val = fpost[D] - correction;
+// step in direction INV[k].  Nash: f_eq of the ghost state, one per site
+// (NashZerothOrderPressureDelegate.h:36-76; the normal is its float copy).
+// Ladd: bounce-back minus the moving-wall correction (LaddIoletDelegate.h:37-86).
+__device__ __forceinline__ void iolet_links(const StepArgs& a, const Bnd& r, const IoletIn& io, int bc, double rho,
+                                            double vx, double vy, double vz, const double* fpost) {
+  if (bc == HLB_IOLET_NASH) {
+    const double rg = io.dens;
+    const double nx = (double)(float)io.n[0], ny = (double)(float)io.n[1], nz = (double)(float)io.n[2];
+    const double component = vx * nx + vy * ny + vz * nz;
+    const double gx = nx * component * rg, gy = ny * component * rg, gz = nz * component * rg;
+    nash_links(a, r, feq_pre(rg, gx, gy, gz), gx, gy, gz);
+  } else {
+    const double vmax = a.io_vmax[r.gi], vmax2 = a.io_vmax2[r.gi];
+#pragma unroll
+    for (int d0 = 1; d0 < Q; d0 += kLaddGroup) {
+      double s[kLaddGroup], s2[kLaddGroup];
+#pragma unroll
+      for (int e = 0; e < kLaddGroup; ++e) {
+        if (!(r.iolet & (1u << (d0 + e - 1)))) continue;
+        s[e] = ldp(a.ladd_s + (int64_t)(d0 + e - 1) * a.SI, r.ii);
+        s2[e] = ldp(a.ladd_s2 + (int64_t)(d0 + e - 1) * a.SI, r.ii);
       }
-      stp(plane(a.G, a.SI, U), i, val);
+#pragma unroll
+      for (int e = 0; e < kLaddGroup; ++e) {
+        const int d = d0 + e;
+        if (!(r.iolet & (1u << (d - 1)))) continue;
+        // speed along the normal: vmax s (parabolic, file) or -Re(K e^{iwt}) (Womersley)
+        const double m = vmax * s[e] + vmax2 * s2[e];
+        const double wx = io.n[0] * m * rho, wy = io.n[1] * m * rho, wz = io.n[2] * m * rho;
+        const double correction =
+            2. * Wt(d) * (wx * (double)CX[d] + wy * (double)CY[d] + wz * (double)CZ[d]) / CS2;
+        stp(plane(a.G, a.SI, INV[d]), r.ii, fpost[d] - correction);
+      }
     }
-    iolet_links<D + 1>(a, i, im, gi, bc, rho, vx, vy, vz, fpost);
   }
 }
 
@@ -315,8 +265,7 @@ __device__ __forceinline__ uint32_t slab_record() {
 
 // B threads (B / 64 slabs) per workgroup; ORDER: the tile order
 // (TileOrder).  NARROW: each pair of opposite planes fits 32-bit offsets from
-// its lower plane (2 S <= 2^29), so the steady step uses gather_up_bb /
-// boundary_fixup_bb.
+// its lower plane (narrow_planes).
 template <int KERNEL, bool FIRST, bool PROPS, int B = kBlock, int ORDER = kOrderXcd, int W = 0, bool NARROW = false,
           bool NT = false>
 __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(W > 0 ? W : 1))) void step_fp64(StepArgs a) {
@@ -324,24 +273,16 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(W > 0 ? W : 1
   const uint32_t tile = tile_index<ORDER>();
   if (!slab_lane(a.bt, tile * (B / kSlab) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), L)) return;
   const uint32_t d = L.slot;
-  const bool isB = L.boundary;
-  uint32_t wm = 0, im = 0;
-  if (isB) {
-    wm = ldp(a.bwall, L.b);
-    im = ldp(a.biolet, L.b);
-  }
+  Bnd bnd = no_bnd();
+  if (L.boundary) bnd = load_bnd(a.bnd, L.b);
   double f[Q];
   if constexpr (FIRST) {
     // Initial condition or checkpoint: f is the pre-collision state itself.
 #pragma unroll
     for (int j = 0; j < Q; ++j) f[j] = ldp(a.ain[j], d);
-  } else if constexpr (NARROW) {
-    f[0] = ldp(a.ain[0], L.slot);
-    gather_up_bb(a, L, f);
-    if (isB) boundary_fixup_bb(a, d, L.b, wm, im, f);
   } else {
-    gather_site(a, L, f);
-    if (isB) boundary_fixup(a, d, L.b, wm, im, f);
+    gather_site<NARROW>(a, L, f);
+    if (L.boundary) boundary_fixup(a, d, L.b, bnd, f);
   }
   if (a.gz.pmask != nullptr) {
     // Sites the Guo-Zheng-Shi link kernel reads keep their pre-collision f.
@@ -361,28 +302,21 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(W > 0 ? W : 1
   double fpost[Q];
   collide_site<KERNEL>(a, f, rho, mx, my, mz, d, tau, fpost);
 
+  IoletIn io{};
+  if (bnd.iolet != 0) io = load_iolet(a, bnd.gi);
 #pragma unroll
   for (int j = 0; j < Q; ++j) {
     if constexpr (NT) stp_nt(a.aout[j], d, fpost[j]);
     else stp(a.aout[j], d, fpost[j]);
   }
 
-  double w = DBL_MAX;
-  if (isB) {
-    const uint32_t b = L.b;
-    const int32_t ii = ldp(a.bii, b);
-    if (ii >= 0) {
-      const int gi = ldp(a.bgi, b);
-      const int bc = gi < a.n_in ? a.inlet_bc : a.outlet_bc;
-      iolet_links(a, (uint32_t)ii, im, gi, bc, rho, ux, uy, uz, fpost);
-      // InOutLetWK*::DoPreStreamCoupling: the coupling site's velocity.Dot(-normal).
-      if (im & a.wk_bit[gi]) {
-        const double c = ux * -a.io_n[3 * gi] + uy * -a.io_n[3 * gi + 1] + uz * -a.io_n[3 * gi + 2];
-        stp(a.wk_contrib, (uint32_t)ldp(a.wk_pos, (uint32_t)ii), c);
-      }
-    }
-    if constexpr (PROPS) {
-      if (wm != 0) w = wall_shear_stress(a, b, tau, f, fpost);
+  if (bnd.iolet != 0) {
+    const int bc = (int)bnd.gi < a.n_in ? a.inlet_bc : a.outlet_bc;
+    iolet_links(a, bnd, io, bc, rho, ux, uy, uz, fpost);
+    // InOutLetWK*::DoPreStreamCoupling: the coupling site's velocity.Dot(-normal).
+    if (bnd.iolet & io.wk) {
+      const double c = ux * -io.n[0] + uy * -io.n[1] + uz * -io.n[2];
+      stp(a.wk_contrib, (uint32_t)ldp(a.wk_pos, bnd.ii), c);
     }
   }
   if constexpr (PROPS) {
@@ -391,23 +325,21 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(W > 0 ? W : 1
     stp(a.u, d, ux);
     stp(plane(a.u, a.S, 1), d, uy);
     stp(plane(a.u, a.S, 2), d, uz);
-    stp(a.wss, d, w);
+    stp(a.wss, d, bnd.wall ? wall_shear_stress(a, L.b, tau, f, fpost) : DBL_MAX);
   }
 }
 
 // Materialises the pre-collision f (the reference's fOld entering the next
 // step) into F, device order.
+template <bool NARROW>
 __global__ __launch_bounds__(kBlock) void gather_fp64(StepArgs a, double* __restrict__ F, int64_t S) {
   Lane L;
   if (!slab_lane(a.bt, slab_record(), L)) return;
-  uint32_t wm = 0, im = 0;
-  if (L.boundary) {
-    wm = ldp(a.bwall, L.b);
-    im = ldp(a.biolet, L.b);
-  }
+  Bnd bnd = no_bnd();
+  if (L.boundary) bnd = load_bnd(a.bnd, L.b);
   double f[Q];
-  gather_site(a, L, f);
-  if (L.boundary) boundary_fixup(a, L.slot, L.b, wm, im, f);
+  gather_site<NARROW>(a, L, f);
+  if (L.boundary) boundary_fixup(a, L.slot, L.b, bnd, f);
 #pragma unroll
   for (int j = 0; j < Q; ++j) stp(plane(F, S, j), L.slot, f[j]);
 }
@@ -471,7 +403,7 @@ __global__ __launch_bounds__(kBlock) void stress_fp64(StepArgs a, const T* __res
   stp(plane(out, a.S, 7), d, sr);
   // traction and its projections at wall sites
   double tr[3] = {0.0, 0.0, 0.0}, tt[3] = {0.0, 0.0, 0.0}, tn[3] = {0.0, 0.0, 0.0};
-  if (L.boundary && ldp(a.bwall, L.b) != 0u) {
+  if (L.boundary && load_bnd(a.bnd, L.b).wall) {
     const double n[3] = {(double)ldp(a.bnrm, L.b), (double)ldp(a.bnrm + a.SB, L.b),
                          (double)ldp(a.bnrm + 2 * a.SB, L.b)};
 #pragma unroll
@@ -802,6 +734,14 @@ static unsigned slab_grid(int64_t nslab) {
   return (unsigned)((wg + kXcds - 1) / kXcds * kXcds);
 }
 
+// 32-bit element offsets from the lower plane of each opposite pair cover
+// both planes (the byte offset i * 8 stays below 2^32), and the planes are one
+// allocation.  Lattices above 2^28 slots, and every lattice when the handle
+// asks for it (a test switch), pick the plane with the 64-bit address.
+static bool narrow_planes(const StepArgs& a) {
+  return !a.general_gather && 2 * a.S <= (int64_t(1) << 29) && a.ain[18] == a.ain[0] + 18 * a.S;
+}
+
 // Steady-state steps in launch shape `variant` (as the FP32 kernel's); the
 // first step after an initial state and property steps use 256-thread tiles.
 template <int KN, bool NARROW>
@@ -840,12 +780,8 @@ void launch_variant_fp64(const StepArgs& a, int variant, hipStream_t s) {
 
 hipError_t launch_step_fp64(const StepArgs& a, int kernel, bool first, bool props, int variant, hipStream_t s) {
   if (a.bt.nslab <= 0) return hipSuccess;
+  const bool narrow = narrow_planes(a);
   if (!first && !props) {
-    // 32-bit element offsets from the lower plane of each opposite pair cover
-    // both planes (the byte offset i * 8 stays below 2^32), and the planes
-    // are one allocation.  Lattices above 2^28 slots, and every lattice when
-    // the handle asks for it (a test switch), take the general gather.
-    const bool narrow = !a.general_gather && 2 * a.S <= (int64_t(1) << 29) && a.ain[18] == a.ain[0] + 18 * a.S;
 #define HLB_K(KN)                                          \
   if (narrow) launch_variant_fp64<KN, true>(a, variant, s); \
   else launch_variant_fp64<KN, false>(a, variant, s);
@@ -858,14 +794,15 @@ hipError_t launch_step_fp64(const StepArgs& a, int kernel, bool first, bool prop
     return hipGetLastError();
   }
   const dim3 grid(slab_grid(a.bt.nslab)), block(kBlock);
-#define HLB_LAUNCH(KN, FI, PR) hipLaunchKernelGGL((step_fp64<KN, FI, PR>), grid, block, 0, s, a)
+#define HLB_LAUNCH(KN, FI, PR, NA) \
+  hipLaunchKernelGGL((step_fp64<KN, FI, PR, kBlock, kOrderXcd, 0, NA>), grid, block, 0, s, a)
 #define HLB_KSEL(KN)                                   \
   if (first) {                                         \
-    if (props) HLB_LAUNCH(KN, true, true);             \
-    else HLB_LAUNCH(KN, true, false);                  \
+    if (props) HLB_LAUNCH(KN, true, true, false);      \
+    else HLB_LAUNCH(KN, true, false, false);           \
   } else {                                             \
-    if (props) HLB_LAUNCH(KN, false, true);            \
-    else HLB_LAUNCH(KN, false, false);                 \
+    if (narrow) HLB_LAUNCH(KN, false, true, true);     \
+    else HLB_LAUNCH(KN, false, true, false);           \
   }
   switch (kernel) {
     case HLB_KERNEL_LBGK: HLB_KSEL(HLB_KERNEL_LBGK); break;
@@ -921,7 +858,9 @@ hipError_t launch_stress_fp64(const StepArgs& a, int kernel, const void* F, bool
 
 hipError_t launch_gather_fp64(const StepArgs& a, double* F, int64_t S, hipStream_t s) {
   if (a.bt.nslab <= 0) return hipSuccess;
-  hipLaunchKernelGGL(gather_fp64, dim3(slab_grid(a.bt.nslab)), dim3(kBlock), 0, s, a, F, S);
+  const dim3 grid(slab_grid(a.bt.nslab)), block(kBlock);
+  if (narrow_planes(a)) hipLaunchKernelGGL(gather_fp64<true>, grid, block, 0, s, a, F, S);
+  else hipLaunchKernelGGL(gather_fp64<false>, grid, block, 0, s, a, F, S);
   return hipGetLastError();
 }
 

@@ -26,9 +26,8 @@
 //          downloads).
 //   rec    one 256-byte record per active slab (SlabRec).  Boundary sites
 //          (collision classes 1-5) are numbered in slot order.
-//   boundary arrays (NB boundary sites, stride SB): wall and iolet link
-//          masks, global iolet index, compact iolet index, 18 planes of float
-//          link distances, 3 planes of float wall normals.
+//   boundary arrays (NB boundary sites, stride SB): one BndRec, 18 planes of
+//          float link distances, 3 planes of float wall normals.
 //   iolet arrays (NI sites with iolet links, slot order, stride SI): G, 19
 //          planes of the values the site's iolet delegates computed for the
 //          next step, and 18 planes of Ladd profile factors.
@@ -69,6 +68,18 @@ struct SlabRec {
   int32_t pad[3];
 };
 static_assert(sizeof(SlabRec) == 256, "slab record is four 64-byte scalar loads");
+
+// One boundary site, for one 16-byte load issued ahead of the site's gathers.
+// Bits are links (d - 1) or pull directions (j - 1); direction j's value is
+// written by link INV[j].
+struct BndRec {
+  uint32_t far;    // directions BFL interpolates with the site's own value (q >= 1/2); bit 31: a wall site
+  uint32_t near;   // directions BFL interpolates with the streamed value (q < 1/2); bits 18..: global iolet index
+  uint32_t iolet;  // iolet links
+  uint32_t ii;     // compact iolet index (sites with iolet links)
+};
+static_assert(sizeof(BndRec) == 16, "one 16-byte load");
+constexpr uint32_t kLinkBits = (1u << 18) - 1u;
 
 // The brick tables of one lattice.
 struct BrickTables {
@@ -171,10 +182,7 @@ struct StepArgs {
   const double* ain[19];
   double* aout[19];
   BrickTables bt;
-  const uint32_t* __restrict__ bwall;
-  const uint32_t* __restrict__ biolet;
-  const int32_t* __restrict__ bgi;  // global iolet index: inlets 0..n_in-1, outlets follow
-  const int32_t* __restrict__ bii;  // compact iolet index, -1 without iolet links
+  const BndRec* __restrict__ bnd;  // global iolet index: inlets 0..n_in-1, outlets follow
   const float* __restrict__ bq;
   const float* __restrict__ bnrm;
   double* __restrict__ G;
@@ -183,7 +191,6 @@ struct StepArgs {
   double* __restrict__ rho;
   double* __restrict__ u;
   double* __restrict__ wss;
-  const float* __restrict__ io_nf;    // 3 per iolet: the normal narrowed to float (Nash)
   const double* __restrict__ io_n;    // 3 per iolet: the normal in double (Ladd)
   const double* __restrict__ io_dens; // this step's ghost density per iolet
   const double* __restrict__ io_vmax; // this step's peak speed per iolet (Womersley: cos wt)
@@ -193,7 +200,6 @@ struct StepArgs {
   double* __restrict__ wk_contrib;     // u.(-n) of this step per coupling site, in the coupling order
   int64_t N, S, SB, SI;
   int32_t n_in;
-  int32_t wall_bc;
   int32_t inlet_bc;
   int32_t outlet_bc;
   double tau;         // LbmParameters tau
@@ -222,10 +228,7 @@ struct Member32 {
   float* A[2];            // post-collision g, 19 planes of S
   const float* F;         // pre-collision g (initial state / checkpoint)
   BrickTables bt;
-  const uint32_t* bwall;
-  const uint32_t* biolet;
-  const int32_t* bgi;
-  const int32_t* bii;
+  const BndRec* bnd;
   const float* bq;
   const float* bnrm;
   float* G;               // iolet values for the next step, 19 planes of SI
@@ -244,7 +247,7 @@ struct Member32 {
   double* wk_contrib;
   int64_t N, S, SB, SI;
   int32_t nio, n_in;
-  int32_t kernel, wall_bc, inlet_bc, outlet_bc;
+  int32_t kernel, inlet_bc, outlet_bc;
   int32_t cur0;           // A[cur0] holds the latest values when the sequence starts
   int32_t first0;         // 1: step 0 of the sequence reads F (pre-collision)
   int32_t props_at;       // step of the sequence that writes rho, u, WSS (-1: none)
