@@ -30,6 +30,7 @@ struct hlb_batch {
   int device = -1;
   int variant = hlb::kFp32DefaultVariant;
   bool variant_chosen = false;  // set by hlb_batch_set_variant / autotune; else default_variant
+  int launch = hlb::kFp32DefaultVariant;  // the variant steps are launched in, as of the last rebuild
   bool use_graph = true;
   bool dirty = true;  // member set or variant changed: rebuild tables, drop graphs
   uint32_t grid = 0;
@@ -94,8 +95,11 @@ int rebuild(hlb_batch* b) {
     int64_t bytes = 0;
     for (const hlb_lattice* m : b->members) bytes += distribution_bytes(m->S, true);
     b->variant = default_variant(bytes, true);
+    b->launch = default_launch(bytes, true, true);
+  } else {
+    b->launch = b->variant;
   }
-  const LaunchShape shape = launch_shape(b->variant, true);
+  const LaunchShape shape = launch_shape(b->launch, true);
   const int64_t per = shape_slabs(shape);
   std::vector<int32_t> map;
   std::vector<WkRef> refs;
@@ -128,7 +132,7 @@ int rebuild(hlb_batch* b) {
 int enqueue_sequence(hlb_batch* b, int64_t n) {
   for (int64_t s = 0; s < n; ++s) {
     HLB_CHECK(launch_wk_begin(b->refs.p, b->nwk, (int)s, b->stream));
-    HLB_CHECK(launch_step_fp32(b->mem.p, b->wg_member.p, b->grid, (int)s, b->variant, b->stream));
+    HLB_CHECK(launch_step_fp32(b->mem.p, b->wg_member.p, b->grid, (int)s, b->launch, b->stream));
     for (size_t i = 0; i < b->members.size(); ++i) {  // GZS walls, per member
       const hlb_lattice* m = b->members[i];
       if (!m->gz_links_host.empty())
@@ -179,7 +183,7 @@ int check_members(hlb_batch* b, const char* who) {
 // Stages a chunk (<= kChunk steps): every member's iolet values and record.
 int stage_chunk(hlb_batch* b, int64_t n, int props_at) {
   HLB_CHECK(hipStreamSynchronize(b->stream));  // staging buffers are free again
-  const int64_t per = shape_slabs(launch_shape(b->variant, true));
+  const int64_t per = shape_slabs(launch_shape(b->launch, true));
   uint32_t wg = 0;
   for (size_t i = 0; i < b->members.size(); ++i) {
     hlb_lattice* m = b->members[i];

@@ -964,11 +964,12 @@ namespace {
 int enqueue_steps(hlb_lattice* h, int64_t n, bool props_last) {
   const int nio = std::max<int>(1, (int)h->iolets.size());
   const int nwk = (int)h->wk_refs_host.size();
+  const int variant = h->launch_variant();
   if (h->fp32()) {
-    const uint32_t grid = member_grid(h->nslab, h->variant);
+    const uint32_t grid = member_grid(h->nslab, variant);
     for (int64_t s = 0; s < n; ++s) {
       HLB_CHECK(launch_wk_begin(h->wk_refs.p, nwk, (int)s, h->stream));
-      HLB_CHECK(launch_step_fp32(h->mem.p, nullptr, grid, (int)s, h->variant, h->stream));
+      HLB_CHECK(launch_step_fp32(h->mem.p, nullptr, grid, (int)s, variant, h->stream));
       HLB_CHECK(launch_gzs_fp32(h->mem.p, h->gz_links.p, (int)h->gz_links_host.size(), (int)s, h->stream));
       HLB_CHECK(launch_wk_end(h->wk_refs.p, nwk, h->stream));
     }
@@ -986,7 +987,7 @@ int enqueue_steps(hlb_lattice* h, int64_t n, bool props_last) {
     a.io_vmax2 = h->io_vmax2.p + s * nio;
     a.sp_t = h->io_sp.p + s;
     HLB_CHECK(launch_wk_begin(h->wk_refs.p, nwk, (int)s, h->stream));
-    HLB_CHECK(launch_step_fp64(a, h->params.kernel, first, props, h->variant, h->stream));
+    HLB_CHECK(launch_step_fp64(a, h->params.kernel, first, props, variant, h->stream));
     HLB_CHECK(launch_gzs_fp64(a, h->params.kernel, h->gz_links.p, (int)h->gz_links_host.size(), a.io_vmax,
                               h->GW64.p, h->stream));
     HLB_CHECK(launch_wk_end(h->wk_refs.p, nwk, h->stream));
@@ -1006,7 +1007,7 @@ const hlb_lattice::StepGraph* find_graph(const hlb_lattice* h, int64_t n, bool p
   const int cur = h->fp32() ? 0 : h->cur;
   const int props = props_last ? 1 : 0;
   for (const auto& g : h->graphs)
-    if (g.n == n && g.props == props && g.first == first && g.cur == cur && g.variant == h->variant) return &g;
+    if (g.n == n && g.props == props && g.first == first && g.cur == cur && g.variant == h->launch_variant()) return &g;
   return nullptr;
 }
 
@@ -1042,7 +1043,7 @@ int prepare_graph(hlb_lattice* h, int64_t n, bool props_last) {
     (void)hipGraphExecDestroy(h->graphs.front().exec);
     h->graphs.erase(h->graphs.begin());
   }
-  h->graphs.push_back({n, props_last ? 1 : 0, first, cur, h->variant, exec});
+  h->graphs.push_back({n, props_last ? 1 : 0, first, cur, h->launch_variant(), exec});
   return HLB_OK;
 }
 
@@ -1372,6 +1373,7 @@ extern "C" int hlb_autotune(hlb_handle h, int64_t trial_steps, int* variant, dou
   if (!h) return fail(HLB_EINVAL, "hlb_autotune: null handle");
   if (trial_steps < 1 || trial_steps > kChunk) return fail(HLB_EINVAL, "hlb_autotune: 1 to 1024 trial steps");
   int best = h->variant;
+  h->variant_chosen = true;
   double best_ms = 1e300;
   const int nvar = h->fp32() ? kFp32Variants : kFp64Variants;
   for (int v = 0; v < nvar; ++v) {
@@ -1386,7 +1388,6 @@ extern "C" int hlb_autotune(hlb_handle h, int64_t trial_steps, int* variant, dou
     }
   }
   h->variant = best;
-  h->variant_chosen = true;
   if (variant) *variant = best;
   if (ms_per_step) *ms_per_step = best_ms / (double)trial_steps;
   return HLB_OK;

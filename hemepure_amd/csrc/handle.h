@@ -167,8 +167,12 @@ struct hlb_lattice {
   std::vector<double> h_ladd_s;  // Ladd profile factors, 2 x 18 planes of SI, device iolet order
   bool device_ready = false;
   bool iolets_set = false;   // hlb_create with params, or hlb_set_iolets
-  int variant = hlb::kFp32DefaultVariant;  // launch shape of the steady-state step
+  int variant = hlb::kFp32DefaultVariant;  // launch shape of the steady-state step, as reported
   bool variant_chosen = false;              // set by hlb_set_variant / hlb_autotune; else default_variant
+  // The variant steps are launched in.
+  int launch_variant() const {
+    return variant_chosen ? variant : hlb::default_launch(hlb::distribution_bytes(S, fp32()), fp32());
+  }
   bool general_gather = false;  // HLB_FP64_GENERAL_GATHER=1 when the device state was made
   // Step sequences captured into HIP graphs and replayed: one per (length,
   // property flag, first-step flag, buffer parity, launch shape); the FP32

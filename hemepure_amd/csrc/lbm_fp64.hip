@@ -742,8 +742,7 @@ static bool narrow_planes(const StepArgs& a) {
   return !a.general_gather && 2 * a.S <= (int64_t(1) << 29) && a.ain[18] == a.ain[0] + 18 * a.S;
 }
 
-// Steady-state steps in launch shape `variant` (as the FP32 kernel's); the
-// first step after an initial state and property steps use 256-thread tiles.
+// Steady-state steps in launch shape `variant` (as the FP32 kernel's).
 template <int KN, bool NARROW>
 void launch_variant_fp64(const StepArgs& a, int variant, hipStream_t s) {
   const LaunchShape l = launch_shape(variant, false);
@@ -793,9 +792,14 @@ hipError_t launch_step_fp64(const StepArgs& a, int kernel, bool first, bool prop
 #undef HLB_K
     return hipGetLastError();
   }
-  const dim3 grid(slab_grid(a.bt.nslab)), block(kBlock);
-#define HLB_LAUNCH(KN, FI, PR, NA) \
-  hipLaunchKernelGGL((step_fp64<KN, FI, PR, kBlock, kOrderXcd, 0, NA>), grid, block, 0, s, a)
+  // one-slab tiles in XCD order, the store policy of the variant
+  const LaunchShape l{kSlab, kOrderXcd, 0, 1, launch_shape(variant, false).nt};
+  const dim3 grid(shape_grid(l, a.bt.nslab)), block(kSlab);
+#define HLB_LAUNCH(KN, FI, PR, NA)                                                                       \
+  do {                                                                                                   \
+    if (l.nt) hipLaunchKernelGGL((step_fp64<KN, FI, PR, kSlab, kOrderXcd, 0, NA, true>), grid, block, 0, s, a); \
+    else hipLaunchKernelGGL((step_fp64<KN, FI, PR, kSlab, kOrderXcd, 0, NA, false>), grid, block, 0, s, a);     \
+  } while (0)
 #define HLB_KSEL(KN)                                   \
   if (first) {                                         \
     if (props) HLB_LAUNCH(KN, true, true, false);      \

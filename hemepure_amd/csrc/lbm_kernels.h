@@ -142,16 +142,37 @@ inline uint32_t shape_grid(const LaunchShape& l, int64_t tiles) {
 }
 unsigned shape_lds(const LaunchShape& l);  // dynamic LDS bytes per workgroup
 
-// The variant a lattice or batch steps with until one is set or autotuned:
-// the default shape, with non-temporal row stores once its distributions
-// (two sets of 19 planes) exceed the 256 MB Infinity Cache -- the store
-// policy the autotuner picks for HBM-resident lattices and batches -- else
-// with cached ones.
+// The variant a lattice or batch reports until one is set or autotuned: the
+// default, or its non-temporal twin once its distributions (two sets of 19
+// planes) exceed the 256 MB Infinity Cache.
 constexpr int64_t kInfinityCacheBytes = int64_t(256) << 20;
 inline int64_t distribution_bytes(int64_t S, bool fp32) { return 2 * 19 * (fp32 ? 4 : 8) * S; }
 inline int default_variant(int64_t dist_bytes, bool fp32) {
   const bool nt = dist_bytes > kInfinityCacheBytes;
   return kFp32DefaultVariant + (nt ? (fp32 ? kFp32Shapes : kFp64Shapes) : 0);
+}
+
+// The shape it is launched in meanwhile, by where its distributions live.
+//   In the Infinity Cache: one-slab tiles in XCD order, cached stores (variant
+//   5).  Against the two-slab tiles of variant 1 a step of the 30k-site
+//   cylinder takes 5.75 instead of 6.4 us (its 480 waves reach more CUs), of a
+//   6k-site pipe 6.6 / 7.0, of the 0.70M-site Y-bifurcation the same (FP64
+//   45.3 / 45.6, FP32 27.1 / 27.3).
+//   Beyond it: non-temporal row stores; up to 2.5 caches the two-slab tiles in
+//   XCD order (0.58 GB FP64 pipe 110.9 us against 116.6 in chunks, 289 MB FP32
+//   pipe 58.6 / 61.1; 0.50 GB bifurcation the other way, 112.7 / 105.9), above
+//   that one-slab tiles in XCD chunks, which keep all XCDs within a few chunks
+//   of one another, so that lines shared across a chunk's edge are still in
+//   the Infinity Cache (XCD order / chunks: 0.70 GB FP32 tree 174 / 159 us, 1.5
+//   GB FP64 pipe 307 / 293, 1.0 GB FP32 pipe 290 / 233, 2.7 GB FP64 tree 604 /
+//   563, 2.5 GB FP64 bifurcation 522 / 508).  A batch takes the chunks from the
+//   cache's size on: a chunk's edge cuts few of its small members (20 pipes,
+//   0.29 GB: 73.1 / 67.8 us).
+inline int default_launch(int64_t dist_bytes, bool fp32, bool batch = false) {
+  const int chunk64 = (fp32 ? 2 * kShapeVariants : kShapeVariants) + 2;
+  if (dist_bytes <= kInfinityCacheBytes) return 5;
+  const bool chunks = batch || dist_bytes > kInfinityCacheBytes * 5 / 2;
+  return (fp32 ? kFp32Shapes : kFp64Shapes) + (chunks ? chunk64 : 1);
 }
 
 // Guo-Zheng-Shi wall links (GuoZhengShiDelegate.h:123-294).  Sites whose

@@ -109,12 +109,6 @@ void release_device(hlb_server* s, Request* r) {
   s->in_use -= r->bytes;
 }
 
-// The launch variant for what is running (default_variant: the default
-// shape, with non-temporal row stores once the running distributions exceed
-// the Infinity Cache).  Requests come and go too often to autotune each
-// running set.
-int64_t running_bytes(const hlb_lattice* h) { return distribution_bytes(h->S, h->fp32()); }
-
 // Starts request r (removed from the queue by the caller).
 void start(hlb_server* s, Request* r) {
   int rc = hlb_init_equilibrium(r->lat, r->rho0, 1);
@@ -252,6 +246,8 @@ extern "C" int hlb_server_advance(hlb_server_handle s, int* running, int* queued
     admit(s);
   }
   if (!s->running.empty()) {
+    // The launch shape follows the running set (default_launch): requests come
+    // and go too often to autotune each one.
     // Every running request advances by the quantum, capped per request by
     // retiring it as soon as it reaches its cap (caps are rounded up to the
     // quantum).  Only this thread changes the running set.
@@ -259,16 +255,10 @@ extern "C" int hlb_server_advance(hlb_server_handle s, int* running, int* queued
     hipStream_t st;
     if (s->mode == HLB_SERVE_PLAIN) {
       hlb_lattice* lat = s->running.front()->lat;
-      const int v = default_variant(running_bytes(lat), lat->fp32());
-      rc = hlb_variant(lat) == v ? HLB_OK : hlb_set_variant(lat, v);
-      if (rc == HLB_OK) rc = hlb_step(lat, s->quantum, HLB_STEP_PROPERTIES);
+      rc = hlb_step(lat, s->quantum, HLB_STEP_PROPERTIES);
       st = lat->stream;
     } else {
-      int64_t bytes = 0;
-      for (const Request* r : s->running) bytes += running_bytes(r->lat);
-      const int v = default_variant(bytes, true);
-      rc = hlb_batch_variant(s->batch) == v ? HLB_OK : hlb_batch_set_variant(s->batch, v);
-      if (rc == HLB_OK) rc = hlb_batch_step(s->batch, s->quantum, HLB_STEP_PROPERTIES);
+      rc = hlb_batch_step(s->batch, s->quantum, HLB_STEP_PROPERTIES);
       st = batch_stream(s->batch);
     }
     if (rc != HLB_OK) return rc;

@@ -205,8 +205,10 @@ int hlb_step(hlb_handle h, int64_t nsteps, uint32_t flags);
  * order, level 0..3 = at most (unlimited, 4, 3, 2) waves per SIMD, level
  * 4..5 = compiled for at least (5, 6) waves per SIMD in FP64 and (6, 7) in
  * the FP32-shifted form.  Until a variant is set or autotuned a lattice (and
- * a batch) steps with variant 1, or with its non-temporal-store twin (FP64
- * 55, FP32 109) while its distributions exceed the 256 MB Infinity Cache.  FP64 36..53 = block + 3 * level with
+ * a batch) reports variant 1, or its non-temporal-store twin (FP64 55, FP32
+ * 109) while its distributions exceed the 256 MB Infinity Cache, and is
+ * launched in the shape that fits their size: variant 5 while they fit the
+ * cache, 55 / 109 up to 2.5 times its size (a batch 182), 92 / 182 beyond.  FP64 36..53 = block + 3 * level with
  * block 0..2 = 128/256/64 slots in the XCD-chunk order (chunks of 32
  * workgroup tiles dealt to the XCDs in turn).  The FP32-shifted form takes
  * 0..35, 36..71 = 0..35 with two consecutive slabs per wavefront (both
@@ -388,9 +390,8 @@ int hlb_batch_autotune(hlb_batch_handle b, int64_t trial_steps, int* variant, do
  * a cycle end, and retires requests that converged (max |du| < tolerance) or
  * reached max_steps, keeping their rho, u and WSS on the host.  Times are
  * seconds since hlb_server_create.  hlb_server_advance is called from one
- * thread at a time.  Both modes step with the default launch shape, with
- * non-temporal row stores while the running distributions exceed the
- * 256 MB Infinity Cache (see hlb_set_variant).
+ * thread at a time.  Both modes step in the default launch shape for the size of
+ * the running distributions (see hlb_set_variant).
  * HLB_SERVE_PLAIN (hlb_server_set_mode, before the first submission) serves
  * the way the reference runs many cases: one request at a time in arrival
  * order, each stepped alone with hlb_step, in either storage form -- the
