@@ -130,22 +130,25 @@ int rebuild(hlb_batch* b) {
 }
 
 int enqueue_sequence(hlb_batch* b, int64_t n) {
+  if (n <= 0) return HLB_OK;
+  const WkLaunch wk = wk_launch(b->refs.p, b->nwk, n);
+  HLB_CHECK(launch_wk_start(b->refs.p, b->nwk, b->stream));
   for (int64_t s = 0; s < n; ++s) {
-    HLB_CHECK(launch_wk_begin(b->refs.p, b->nwk, (int)s, b->stream));
-    HLB_CHECK(launch_step_fp32(b->mem.p, b->wg_member.p, b->grid, (int)s, b->launch, b->stream));
+    HLB_CHECK(launch_step_fp32(b->mem.p, b->wg_member.p, b->grid, (int)s, wk, b->launch, b->stream));
     for (size_t i = 0; i < b->members.size(); ++i) {  // GZS walls, per member
       const hlb_lattice* m = b->members[i];
       if (!m->gz_links_host.empty())
         HLB_CHECK(launch_gzs_fp32(b->mem.p + i, m->gz_links.p, (int)m->gz_links_host.size(), (int)s, b->stream));
     }
-    HLB_CHECK(launch_wk_end(b->refs.p, b->nwk, b->stream));
   }
+  HLB_CHECK(launch_wk_flush(b->refs.p, b->nwk, (int)(n - 1), b->stream));
   return HLB_OK;
 }
 
 // Launches n steps whose iolet values and member records are staged, from
 // a captured graph when enabled.
 int launch_sequence(hlb_batch* b, int64_t n, int props_at) {
+  if (n <= 0) return HLB_OK;
   if (!b->use_graph) return enqueue_sequence(b, n);
   for (const auto& g : b->graphs)
     if (g.n == n && g.props_at == props_at) {

@@ -647,7 +647,7 @@ int upload_lattice(hlb_lattice* h) {
     HLB_CHECK(h->wk.alloc(h->wk_host.size()));
     HLB_CHECK(hipMemcpy(h->wk.p, h->wk_host.data(), sizeof(WkIolet) * h->wk_host.size(), hipMemcpyHostToDevice));
     // the coupling terms, written by the step in the coupling order
-    const size_t ncoup = std::max<size_t>(1, h->wk_list.size());
+    const size_t ncoup = 2 * (size_t)h->wk_stride();
     HLB_CHECK(h->wk_contrib.alloc(ncoup));
     HLB_CHECK(hipMemsetAsync(h->wk_contrib.p, 0, sizeof(double) * ncoup, h->stream));
     std::vector<int32_t> pos((size_t)std::max<int64_t>(1, SI), -1);
@@ -657,7 +657,7 @@ int upload_lattice(hlb_lattice* h) {
     h->wk_refs_host.clear();
     for (size_t g = 0; g < h->iolets.size(); ++g)
       if (h->iolets[g].IsWK())
-        h->wk_refs_host.push_back(WkRef{h->wk.p + g, h->io_dens.p, h->wk_contrib.p, (int32_t)g, nio,
+        h->wk_refs_host.push_back(WkRef{h->wk.p + g, h->io_dens.p, h->wk_contrib.p, h->wk_stride(), (int32_t)g, nio,
                                         h->fp32() ? 0 : 1, 0});
     HLB_CHECK(h->wk_refs.alloc(std::max<size_t>(1, h->wk_refs_host.size())));
     if (!h->wk_refs_host.empty())
@@ -890,6 +890,7 @@ Member32 member_record(const hlb_lattice* h, int props_at) {
   m.wk_bit = h->wk_bit.p;
   m.wk_pos = h->wk_pos.p;
   m.wk_contrib = h->wk_contrib.p;
+  m.wk_stride = h->wk_stride();
   m.N = h->L.N;
   m.S = h->S;
   m.SB = h->SB;
@@ -962,17 +963,19 @@ namespace {
 // form, member record) are staged: kernel launches only, so the sequence can
 // be captured into a graph.
 int enqueue_steps(hlb_lattice* h, int64_t n, bool props_last) {
+  if (n <= 0) return HLB_OK;
   const int nio = std::max<int>(1, (int)h->iolets.size());
   const int nwk = (int)h->wk_refs_host.size();
   const int variant = h->launch_variant();
+  const WkLaunch wk = wk_launch(h->wk_refs.p, nwk, n);
+  HLB_CHECK(launch_wk_start(h->wk_refs.p, nwk, h->stream));
   if (h->fp32()) {
     const uint32_t grid = member_grid(h->nslab, variant);
     for (int64_t s = 0; s < n; ++s) {
-      HLB_CHECK(launch_wk_begin(h->wk_refs.p, nwk, (int)s, h->stream));
-      HLB_CHECK(launch_step_fp32(h->mem.p, nullptr, grid, (int)s, variant, h->stream));
+      HLB_CHECK(launch_step_fp32(h->mem.p, nullptr, grid, (int)s, wk, variant, h->stream));
       HLB_CHECK(launch_gzs_fp32(h->mem.p, h->gz_links.p, (int)h->gz_links_host.size(), (int)s, h->stream));
-      HLB_CHECK(launch_wk_end(h->wk_refs.p, nwk, h->stream));
     }
+    HLB_CHECK(launch_wk_flush(h->wk_refs.p, nwk, (int)(n - 1), h->stream));
     advance_state(h, n);
     return HLB_OK;
   }
@@ -986,14 +989,16 @@ int enqueue_steps(hlb_lattice* h, int64_t n, bool props_last) {
     a.io_vmax = h->io_vmax.p + s * nio;
     a.io_vmax2 = h->io_vmax2.p + s * nio;
     a.sp_t = h->io_sp.p + s;
-    HLB_CHECK(launch_wk_begin(h->wk_refs.p, nwk, (int)s, h->stream));
+    a.step = (int32_t)s;
+    a.wk = wk;
+    a.wk_contrib = h->wk_contrib.p + (s & 1) * h->wk_stride();
     HLB_CHECK(launch_step_fp64(a, h->params.kernel, first, props, variant, h->stream));
     HLB_CHECK(launch_gzs_fp64(a, h->params.kernel, h->gz_links.p, (int)h->gz_links_host.size(), a.io_vmax,
                               h->GW64.p, h->stream));
-    HLB_CHECK(launch_wk_end(h->wk_refs.p, nwk, h->stream));
     if (!first) h->cur ^= 1;
     h->have_post = true;
   }
+  HLB_CHECK(launch_wk_flush(h->wk_refs.p, nwk, (int)(n - 1), h->stream));
   h->t += n;
   return HLB_OK;
 }

@@ -45,31 +45,31 @@ __device__ __forceinline__ T* plane(T* p, int64_t S, int j) {
   return p + (int64_t)j * S;
 }
 
-// XCD-contiguous workgroup order: the hardware hands workgroup w to XCD
-// w mod 8, so logical tile (w mod 8) * (grid / 8) + w / 8 gives each XCD one
-// contiguous eighth of the tiles (grid is a multiple of 8).
-__device__ __forceinline__ uint32_t xcd_tile() {
-  const uint32_t per = gridDim.x / kXcds;
-  return (blockIdx.x % kXcds) * per + blockIdx.x / kXcds;
+// Tile orders over the workgroups behind the first `lead` ones (a multiple of
+// the XCD count, so a workgroup's XCD stays its index mod 8).
+// XCD-contiguous: the hardware hands workgroup w to XCD w mod 8, so logical
+// tile (w mod 8) * (grid / 8) + w / 8 gives each XCD one contiguous eighth of
+// the tiles (grid is a multiple of 8).
+__device__ __forceinline__ uint32_t xcd_tile(uint32_t lead = 0) {
+  const uint32_t w = blockIdx.x - lead, per = (gridDim.x - lead) / kXcds;
+  return (w % kXcds) * per + w / kXcds;
 }
 
-// XCD-chunk order: XCD x's k-th workgroup takes tile k mod C of chunk
-// x + 8 (k / C), C = kXcdChunk, so chunks of C consecutive tiles go to the
-// XCDs in turn (grid is a multiple of 8 C; a bijection on [0, grid)).
-__device__ __forceinline__ uint32_t xcd_chunk_tile() {
-  const uint32_t x = blockIdx.x % kXcds, k = blockIdx.x / kXcds;
+// XCD chunks: XCD x's k-th workgroup takes tile k mod C of chunk x + 8 (k / C),
+// C = kXcdChunk, so chunks of C consecutive tiles go to the XCDs in turn (grid
+// is a multiple of 8 C; a bijection on [0, grid)).
+__device__ __forceinline__ uint32_t xcd_chunk_tile(uint32_t lead = 0) {
+  const uint32_t w = blockIdx.x - lead, x = w % kXcds, k = w / kXcds;
   return (x + kXcds * (k / kXcdChunk)) * kXcdChunk + k % kXcdChunk;
 }
 
 // The logical tile of this workgroup in tile order ORDER (a TileOrder).
 template <int ORDER>
-__device__ __forceinline__ uint32_t tile_index() {
-  if constexpr (ORDER == kOrderXcd) return xcd_tile();
-  else if constexpr (ORDER == kOrderXcdChunks) return xcd_chunk_tile();
-  else return blockIdx.x;
+__device__ __forceinline__ uint32_t tile_index(uint32_t lead) {
+  if constexpr (ORDER == kOrderXcd) return xcd_tile(lead);
+  else if constexpr (ORDER == kOrderXcdChunks) return xcd_chunk_tile(lead);
+  else return blockIdx.x - lead;
 }
-
-__device__ __forceinline__ uint32_t site_index() { return xcd_tile() * kBlock + threadIdx.x; }
 
 __device__ __forceinline__ uint64_t uniform64(uint64_t v) {
   const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);

@@ -28,10 +28,10 @@ hipError_t launch_gather_fp64(const StepArgs& a, double* F, int64_t S, hipStream
 hipError_t launch_stress_fp64(const StepArgs& a, int kernel, const void* F, bool fp32, double* out, hipStream_t s);
 hipError_t launch_fill_fp64(double* F, int64_t N, int64_t S, const double* vals, hipStream_t s);
 hipError_t launch_unstable_fp64(const BrickTables& bt, const double* F, int64_t S, int* flag, hipStream_t s);
-hipError_t launch_wk_begin(const WkRef* refs, int n, int step, hipStream_t s);
-hipError_t launch_wk_end(const WkRef* refs, int n, hipStream_t s);
+hipError_t launch_wk_start(const WkRef* refs, int n, hipStream_t s);
+hipError_t launch_wk_flush(const WkRef* refs, int n, int last, hipStream_t s);
 hipError_t launch_step_fp32(const Member32* members, const int32_t* wg_member, uint32_t grid, int step,
-                            int variant, hipStream_t s);
+                            const WkLaunch& wk, int variant, hipStream_t s);
 hipError_t launch_gather_fp32(const Member32* members, int64_t nslab, float* F, hipStream_t s);
 hipError_t launch_fill_fp32(float* F, int64_t N, int64_t S, const float* vals, hipStream_t s);
 hipError_t launch_unstable_fp32(const BrickTables& bt, const float* F, int64_t S, int* flag, hipStream_t s);
@@ -145,7 +145,8 @@ struct hlb_lattice {
   std::vector<hlb::WkIolet> wk_host;
   hlb::DevBuf<hlb::WkIolet> wk;
   hlb::DevBuf<uint32_t> wk_bit;
-  hlb::DevBuf<double> wk_contrib;
+  hlb::DevBuf<double> wk_contrib;  // two buffers of wk_stride() terms, even and odd steps'
+  int64_t wk_stride() const { return (int64_t)(wk_list.empty() ? 1 : wk_list.size()); }
   hlb::DevBuf<int32_t> wk_pos;  // per iolet site: its place in wk_list (coupling sites), else -1
   std::vector<hlb::WkRef> wk_refs_host;  // one per Windkessel iolet
   hlb::DevBuf<hlb::WkRef> wk_refs;

@@ -24,6 +24,7 @@
 #include "d3q19.h"
 #include "device_util.h"
 #include "lbm_kernels.h"
+#include "windkessel.h"
 
 namespace hlb {
 
@@ -279,7 +280,7 @@ __device__ __forceinline__ void iolet_links32(const Member32& m, int step, const
   if (r.iolet & io.wk) {
     const double c = (double)vx * -ldp(m.io_n, 3u * r.gi) + (double)vy * -ldp(m.io_n, 3u * r.gi + 1) +
                      (double)vz * -ldp(m.io_n, 3u * r.gi + 2);
-    stp(m.wk_contrib, (uint32_t)ldp(m.wk_pos, r.ii), c);
+    stp(m.wk_contrib + (step & 1) * m.wk_stride, (uint32_t)ldp(m.wk_pos, r.ii), c);
   }
 }
 
@@ -453,8 +454,9 @@ __device__ __forceinline__ void site_finish32(const Member32& m, const Planes& P
 // order (TileOrder); NT: non-temporal stores of the post-collision rows.
 template <int B, int ORDER, int W = 0, int SPT = 1, bool NT = false>
 __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(W > 0 ? W : 1))) void step_fp32(
-    const Member32* __restrict__ members, const int32_t* __restrict__ wg_member, int step) {
-  const uint32_t tile = tile_index<ORDER>();
+    const Member32* __restrict__ members, const int32_t* __restrict__ wg_member, int step, WkLaunch wk) {
+  if (wk_workgroup(wk, step)) return;
+  const uint32_t tile = tile_index<ORDER>(wk.groups);
   const int mi = member_of_tile(wg_member, tile);
   if (mi < 0) return;  // padding tile
   const Member32& m = members[mi];
@@ -666,15 +668,16 @@ unsigned shape_lds(const LaunchShape& l) {
 // `grid` workgroup tiles of the variant's size, padded as shape_grid pads
 // them (padding tiles map to member -1).
 hipError_t launch_step_fp32(const Member32* members, const int32_t* wg_member, uint32_t grid, int step,
-                            int variant, hipStream_t s) {
+                            const WkLaunch& wk, int variant, hipStream_t s) {
   if (grid == 0) return hipSuccess;
+  grid += wk.groups;
   const LaunchShape l = launch_shape(variant, true);
   const unsigned lds = shape_lds(l);
 #define HLB_VN(B, O, W, NT)                                                                                  \
   if (l.spt == 2)                                                                                            \
-    hipLaunchKernelGGL((step_fp32<B, O, W, 2, NT>), dim3(grid), dim3(B), lds, s, members, wg_member, step);  \
+    hipLaunchKernelGGL((step_fp32<B, O, W, 2, NT>), dim3(grid), dim3(B), lds, s, members, wg_member, step, wk);  \
   else                                                                                                       \
-    hipLaunchKernelGGL((step_fp32<B, O, W, 1, NT>), dim3(grid), dim3(B), lds, s, members, wg_member, step)
+    hipLaunchKernelGGL((step_fp32<B, O, W, 1, NT>), dim3(grid), dim3(B), lds, s, members, wg_member, step, wk)
 #define HLB_V(B, O, W)     \
   if (l.nt) {              \
     HLB_VN(B, O, W, true); \

@@ -31,6 +31,7 @@
 #include "d3q19.h"
 #include "device_util.h"
 #include "lbm_kernels.h"
+#include "windkessel.h"
 
 namespace hlb {
 
@@ -269,8 +270,9 @@ __device__ __forceinline__ uint32_t slab_record() {
 template <int KERNEL, bool FIRST, bool PROPS, int B = kBlock, int ORDER = kOrderXcd, int W = 0, bool NARROW = false,
           bool NT = false>
 __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(W > 0 ? W : 1))) void step_fp64(StepArgs a) {
+  if (wk_workgroup(a.wk, a.step)) return;
   Lane L;
-  const uint32_t tile = tile_index<ORDER>();
+  const uint32_t tile = tile_index<ORDER>(a.wk.groups);
   if (!slab_lane(a.bt, tile * (B / kSlab) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), L)) return;
   const uint32_t d = L.slot;
   Bnd bnd = no_bnd();
@@ -594,134 +596,36 @@ __global__ __launch_bounds__(kBlock) void unstable_fp64(BrickTables bt, const do
   if (bad) *flag = 1;
 }
 
-// Start of a step for the Windkessel iolets: InOutLetWK*::DoComms
-// (InOutLetWK3.cc:33-52) -- density <- densityNew, flowRate <- the previous
-// step's sum scaled by area / siteCount -- and the ghost density the step's
-// Nash links read.  One thread per Windkessel iolet.
-__global__ __launch_bounds__(256) void wk_begin(const WkRef* __restrict__ refs, int n, int step) {
+// First row of a sequence: the ghost densities its first step reads
+// (InOutLetWK*::DoComms, density <- densityNew).  One thread per iolet.
+__global__ __launch_bounds__(256) void wk_start(const WkRef* __restrict__ refs, int n) {
   const int r = blockIdx.x * blockDim.x + threadIdx.x;
   if (r >= n) return;
   const WkRef ref = refs[r];
-  WkIolet& w = *ref.w;
-  w.density = w.densityNew;
-  w.flowRate = w.flowRateNew;
-  if (w.siteCount != 0) w.flowRate = w.flowRate * w.area / w.siteCount;
-  w.flowRateNew = 0.0;
-  w.siteCount = 0;
-  ref.io_dens[(int64_t)step * ref.nio + ref.g] = w.density;
+  ref.io_dens[ref.g] = ref.w->densityNew;
 }
 
-// End of a step: the coupling sites' terms summed, the centre site's
-// pressure update (InOutLetWK2.cc:82-95, InOutLetWK3.cc:70-95) and the
-// post-stream commit (:97-106).  One workgroup per iolet.  The step wrote the
-// terms contiguously in the reference's site order (InOutLetWK3.cc:33-52
-// accumulates flowRateNew += u.(-n) site by site), so the FP64 form runs that
-// same sequential chain -- its rounding is the reference's: the workgroup
-// stages the terms in LDS, then one wavefront adds them in order, its LDS
-// reads running a group ahead of the additions (the chain of dependent FP64
-// additions is then the whole cost, about 7.5 ns a term on MI355X).  The
-// FP32-shifted form needs no order: each thread sums a strided share into
-// four partial sums (four loads in flight), and the 256 partial sums are
-// combined across lanes and waves in a fixed order, all in FP64.
-constexpr int kWkThreads = 256;
-constexpr int kWkStage = 4096;  // terms staged per pass (32 KB of LDS)
-constexpr int kWkGroup = 32;    // LDS reads ahead of the additions
-
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
-}
-
-// sum + st[0] + st[1] + ... + st[n-1], in that order (st wave-uniform).
-__device__ __forceinline__ double chain_sum(double sum, const double* st, int n) {
-  constexpr int G = kWkGroup;
-  int i = 0;
-  if (n >= G) {
-    double cur[G], nxt[G];
-#pragma unroll
-    for (int k = 0; k < G; ++k) cur[k] = st[k];
-    for (; i + 2 * G <= n; i += G) {
-#pragma unroll
-      for (int k = 0; k < G; ++k) nxt[k] = st[i + G + k];
-#pragma unroll
-      for (int k = 0; k < G; ++k) sum += cur[k];
-#pragma unroll
-      for (int k = 0; k < G; ++k) cur[k] = nxt[k];
-    }
-#pragma unroll
-    for (int k = 0; k < G; ++k) sum += cur[k];
-    i += G;
-  }
-  for (; i < n; ++i) sum += st[i];
-  return sum;
-}
-
-__global__ __launch_bounds__(kWkThreads) void wk_end(const WkRef* __restrict__ refs) {
-  __shared__ double st[kWkStage];
+// End of a sequence: the sum of its last step's flux terms, which the next
+// step's DoComms scales.  One wavefront per iolet.
+__global__ __launch_bounds__(64) void wk_flush(const WkRef* __restrict__ refs, int last) {
   const WkRef ref = refs[blockIdx.x];
-  WkIolet& w = *ref.w;
-  const HLB_GLOBAL double* __restrict__ t = (const HLB_GLOBAL double*)ref.contrib;
-  const int32_t lb = __builtin_amdgcn_readfirstlane(w.list_begin);
-  const int32_t le = __builtin_amdgcn_readfirstlane(w.list_end);
-  double sum = w.flowRateNew;
-  if (ref.ordered) {
-    for (int32_t c0 = lb; c0 < le; c0 += kWkStage) {
-      const int32_t cn = min(kWkStage, le - c0);
-      for (int32_t i = (int32_t)threadIdx.x; i < cn; i += kWkThreads) st[i] = t[c0 + i];
-      __syncthreads();
-      if (threadIdx.x < 64) sum = chain_sum(sum, st, cn);
-      __syncthreads();
-    }
-  } else {
-    double p0 = 0.0, p1 = 0.0, p2 = 0.0, p3 = 0.0;
-    int32_t e = lb + (int32_t)threadIdx.x;
-    for (; e + 3 * kWkThreads < le; e += 4 * kWkThreads) {
-      p0 += t[e];
-      p1 += t[e + kWkThreads];
-      p2 += t[e + 2 * kWkThreads];
-      p3 += t[e + 3 * kWkThreads];
-    }
-    for (; e < le; e += kWkThreads) p0 += t[e];
-    const double part = wave_sum((p0 + p1) + (p2 + p3));
-    if ((threadIdx.x & 63) == 0) st[threadIdx.x >> 6] = part;
-    __syncthreads();
-    sum += (st[0] + st[1]) + (st[2] + st[3]);
-  }
+  const double sum = wk_flux_sum(ref, last);
   if (threadIdx.x != 0) return;
-  if (w.centre_coupled) {
-    const double pressure = w.density * CS2;
-    if (w.kind == HLB_IOLET_WK2) {
-      const double R0 = w.resistance, C0 = w.capacitance;
-      const double pressureNew = R0 / (1.0 + R0 * C0) * (w.flowRate + C0 * pressure);
-      w.densityNew = pressureNew / CS2;
-    } else {
-      const double Rc = w.r_c, Rp = w.r_p, Cp = w.capacitance;
-      const double pressureNew = (Rp * Cp * pressure + (Rc + Rp) * (2.0 * w.flowRate - w.flowRateOld) +
-                                  Rc * Rp * Cp * (w.flowRate - w.flowRateOld)) /
-                                 (1.0 + Rp * Cp);
-      w.densityNew = pressureNew / CS2;
-    }
-  }
-  w.flowRateNew = sum;
-  w.siteCount += (double)(le - lb);
-  if (w.centre_coupled) {
-    w.density = w.densityNew;
-    w.flowRateOld = w.flowRate;
-  }
+  ref.w->flowRateNew = sum;
+  ref.w->siteCount = (double)(ref.w->list_end - ref.w->list_begin);
 }
 
 }  // namespace
 
-hipError_t launch_wk_begin(const WkRef* refs, int n, int step, hipStream_t s) {
+hipError_t launch_wk_start(const WkRef* refs, int n, hipStream_t s) {
   if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(wk_begin, dim3((n + 255) / 256), dim3(256), 0, s, refs, n, step);
+  hipLaunchKernelGGL(wk_start, dim3((n + 255) / 256), dim3(256), 0, s, refs, n);
   return hipGetLastError();
 }
 
-hipError_t launch_wk_end(const WkRef* refs, int n, hipStream_t s) {
+hipError_t launch_wk_flush(const WkRef* refs, int n, int last, hipStream_t s) {
   if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(wk_end, dim3(n), dim3(kWkThreads), 0, s, refs);
+  hipLaunchKernelGGL(wk_flush, dim3(n), dim3(64), 0, s, refs, last);
   return hipGetLastError();
 }
 
@@ -747,7 +651,7 @@ template <int KN, bool NARROW>
 void launch_variant_fp64(const StepArgs& a, int variant, hipStream_t s) {
   const LaunchShape l = launch_shape(variant, false);
   const int per = shape_slabs(l);
-  const dim3 grid(shape_grid(l, (a.bt.nslab + per - 1) / per));
+  const dim3 grid(a.wk.groups + shape_grid(l, (a.bt.nslab + per - 1) / per));
   const unsigned lds = shape_lds(l);
 #define HLB_V(B, O, W)                                                                                   \
   if (l.nt)                                                                                              \
@@ -794,7 +698,7 @@ hipError_t launch_step_fp64(const StepArgs& a, int kernel, bool first, bool prop
   }
   // one-slab tiles in XCD order, the store policy of the variant
   const LaunchShape l{kSlab, kOrderXcd, 0, 1, launch_shape(variant, false).nt};
-  const dim3 grid(shape_grid(l, a.bt.nslab)), block(kSlab);
+  const dim3 grid(a.wk.groups + shape_grid(l, a.bt.nslab)), block(kSlab);
 #define HLB_LAUNCH(KN, FI, PR, NA)                                                                       \
   do {                                                                                                   \
     if (l.nt) hipLaunchKernelGGL((step_fp64<KN, FI, PR, kSlab, kOrderXcd, 0, NA, true>), grid, block, 0, s, a); \

@@ -197,6 +197,42 @@ struct GzsLink {
   double s, s2;     // iolet profile factors at x + c_INV[d] (mode 3): speed = vmax s + vmax2 s2
 };
 
+// Windkessel state of one iolet (InOutLetWK2.cc:13-18, InOutLetWK3.cc:13-18)
+// plus its constants; updated on the device between steps.
+struct WkIolet {
+  double density, densityNew, flowRate, flowRateOld, flowRateNew, siteCount;
+  double area, resistance, r_c, r_p, capacitance;
+  int32_t kind;            // HLB_IOLET_WK2 / HLB_IOLET_WK3, anything else: not a Windkessel
+  int32_t centre_coupled;  // the centre site is one of this iolet's coupling sites
+  int32_t list_begin, list_end;  // the iolet's coupling sites: positions in the coupling order
+};
+
+// A Windkessel iolet as the per-step kernels see it: its state and the
+// buffers of the lattice it belongs to.  Arrays of these let one launch
+// serve the Windkessel iolets of every lattice in a batch.
+struct WkRef {
+  WkIolet* w;
+  double* io_dens;        // the lattice's ghost-density rows (stride nio)
+  const double* contrib;  // the lattice's u.(-n) terms in the coupling order, even steps' and odd steps'
+  int64_t stride;         // from the first to the second
+  int32_t g, nio;         // iolet index in its lattice, row stride
+  int32_t ordered;        // 1: sum in the reference's site order (FP64 form); 0: tree (FP32-shifted form)
+  int32_t pad_;
+};
+
+// The Windkessel share of a launch (windkessel.h): its first `groups`
+// workgroups (a multiple of the XCD count), one of which serves each iolet.
+struct WkLaunch {
+  const WkRef* refs;
+  int32_t n;
+  uint32_t groups;
+  int32_t steps;  // of the sequence
+  int32_t pad_;
+};
+inline WkLaunch wk_launch(const WkRef* refs, int n, int64_t steps) {
+  return WkLaunch{refs, n, (uint32_t)((n + kXcds - 1) / kXcds * kXcds), (int32_t)steps, 0};
+}
+
 struct StepArgs {
   // Per-plane base pointers, passed as separate scalars so each access is one
   // SGPR base plus a 32-bit VGPR offset.
@@ -229,7 +265,8 @@ struct StepArgs {
   double half_omega_minus;
   double les_k;       // 18 sqrt(2) C_s^2 evaluated in the reference's order
   int32_t general_gather;  // 1: the steady step takes the general gather on any lattice
-  int32_t pad_;
+  int32_t step;            // of the sequence
+  WkLaunch wk;
   // LES sponge layer: vTau per slot (nullptr: none), this step's time (t
   // while t < lifetime, else -1), lifetime / 2 (integer division) and lifetime.
   const double* __restrict__ vtau;
@@ -265,7 +302,8 @@ struct Member32 {
   const double* io_vmax2;
   const uint32_t* wk_bit;
   const int32_t* wk_pos;
-  double* wk_contrib;
+  double* wk_contrib;     // even steps' terms, then wk_stride on the odd steps'
+  int64_t wk_stride;
   int64_t N, S, SB, SI;
   int32_t nio, n_in;
   int32_t kernel, inlet_bc, outlet_bc;
@@ -281,28 +319,6 @@ struct Member32 {
   const float* vtau;      // LES sponge layer (see StepArgs); nullptr: none
   const double* sp_t;     // rows of one per step of the launch sequence
   double sp_half, sp_life;
-};
-
-// Windkessel state of one iolet (InOutLetWK2.cc:13-18, InOutLetWK3.cc:13-18)
-// plus its constants; updated on the device between steps.
-struct WkIolet {
-  double density, densityNew, flowRate, flowRateOld, flowRateNew, siteCount;
-  double area, resistance, r_c, r_p, capacitance;
-  int32_t kind;            // HLB_IOLET_WK2 / HLB_IOLET_WK3, anything else: not a Windkessel
-  int32_t centre_coupled;  // the centre site is one of this iolet's coupling sites
-  int32_t list_begin, list_end;  // the iolet's coupling sites: positions in the coupling order
-};
-
-// A Windkessel iolet as the per-step kernels see it: its state and the
-// buffers of the lattice it belongs to.  Arrays of these let one launch
-// serve the Windkessel iolets of every lattice in a batch.
-struct WkRef {
-  WkIolet* w;
-  double* io_dens;        // the lattice's ghost-density rows (stride nio)
-  const double* contrib;  // the lattice's u.(-n) terms in the coupling order
-  int32_t g, nio;         // iolet index in its lattice, row stride
-  int32_t ordered;        // 1: sum in the reference's site order (FP64 form); 0: tree (FP32-shifted form)
-  int32_t pad_;
 };
 
 }  // namespace hlb
