@@ -149,7 +149,14 @@ int enqueue_sequence(hlb_batch* b, int64_t n) {
 // a captured graph when enabled.
 int launch_sequence(hlb_batch* b, int64_t n, int props_at) {
   if (n <= 0) return HLB_OK;
-  if (!b->use_graph) return enqueue_sequence(b, n);
+  // GZS walls add a launch per member and step, which a replay saves at any size
+  int64_t slabs = 0;
+  bool links = false;
+  for (const hlb_lattice* m : b->members) {
+    slabs += m->nslab;
+    links = links || !m->gz_links_host.empty();
+  }
+  if (!b->use_graph || !replay_pays(n, links ? 0 : slabs)) return enqueue_sequence(b, n);
   for (const auto& g : b->graphs)
     if (g.n == n && g.props_at == props_at) {
       HLB_CHECK(hipGraphLaunch(g.exec, b->stream));

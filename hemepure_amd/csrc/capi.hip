@@ -74,6 +74,15 @@ double cosine_density(const HostIolet& io, uint64_t t0) {
   return f * target + (1. - f) * io.minSimDensity;
 }
 
+// Points the arguments at the per-step values of step s of the sequence.
+void step_rows(const hlb_lattice* h, StepArgs& a, int64_t s) {
+  const int64_t nio = h->iolet_count();
+  a.io_dens = h->rows() + s * h->row();
+  a.io_vmax = a.io_dens + nio;
+  a.io_vmax2 = a.io_dens + 2 * nio;
+  a.sp_t = a.io_dens + 3 * nio;
+}
+
 StepArgs make_args(hlb_lattice* h, const double* ain, double* aout) {
   StepArgs a{};
   for (int j = 0; j < Q; ++j) {
@@ -94,9 +103,6 @@ StepArgs make_args(hlb_lattice* h, const double* ain, double* aout) {
   a.u = h->u.p;
   a.wss = h->wss.p;
   a.io_n = h->io_n.p;
-  a.io_dens = h->io_dens.p;
-  a.io_vmax = h->io_vmax.p;
-  a.io_vmax2 = h->io_vmax2.p;
   a.wk_bit = h->wk_bit.p;
   a.wk_pos = h->wk_pos.p;
   a.wk_contrib = h->wk_contrib.p;
@@ -114,7 +120,7 @@ StepArgs make_args(hlb_lattice* h, const double* ain, double* aout) {
   a.les_k = h->les_k;
   a.general_gather = h->general_gather ? 1 : 0;
   a.vtau = h->sponge_life > 0 ? h->vtau64.p : nullptr;
-  a.sp_t = h->io_sp.p;
+  step_rows(h, a, 0);
   a.sp_half = (double)(h->sponge_life / 2);
   a.sp_life = (double)h->sponge_life;
   return a;
@@ -533,8 +539,6 @@ int upload_lattice(hlb_lattice* h) {
     HLB_CHECK(h->A32[1].alloc((size_t)Q * S));
     HLB_CHECK(h->G32.alloc((size_t)Q * SI));
     HLB_CHECK(h->feq32.alloc(Q));
-    HLB_CHECK(h->mem.alloc(1));
-    HLB_CHECK(hipHostMalloc((void**)&h->h_mem, sizeof(Member32), hipHostMallocDefault));
     HLB_CHECK(hipMemsetAsync(h->A32[0].p, 0, sizeof(float) * Q * S, h->stream));
     HLB_CHECK(hipMemsetAsync(h->A32[1].p, 0, sizeof(float) * Q * S, h->stream));
     HLB_CHECK(hipMemsetAsync(h->G32.p, 0, sizeof(float) * Q * SI, h->stream));
@@ -553,7 +557,6 @@ int upload_lattice(hlb_lattice* h) {
   HLB_CHECK(h->rho.alloc((size_t)S));
   HLB_CHECK(h->u.alloc((size_t)3 * S));
   HLB_CHECK(h->wss.alloc((size_t)S));
-  HLB_CHECK(h->flag.alloc(1));
   HLB_CHECK(h->feq_vals.alloc(Q));
   // Holes are never written: keep the field arrays defined there.
   HLB_CHECK(hipMemsetAsync(h->rho.p, 0, sizeof(double) * S, h->stream));
@@ -622,7 +625,7 @@ int upload_lattice(hlb_lattice* h) {
                       hipMemcpyHostToDevice));
   // Per-iolet constants and the staging for per-step values.
   {
-    const int nio = std::max<int>(1, (int)h->iolets.size());
+    const int nio = h->iolet_count();
     std::vector<float> nf((size_t)3 * nio, 0.0f);
     std::vector<double> nd((size_t)3 * nio, 0.0);
     for (size_t g = 0; g < h->iolets.size(); ++g)
@@ -632,13 +635,11 @@ int upload_lattice(hlb_lattice* h) {
       }
     HLB_CHECK(h->io_nf.alloc(nf.size()));
     HLB_CHECK(h->io_n.alloc(nd.size()));
-    HLB_CHECK(h->io_dens.alloc((size_t)kChunk * nio));
-    HLB_CHECK(h->io_vmax.alloc((size_t)kChunk * nio));
-    HLB_CHECK(h->io_vmax2.alloc((size_t)kChunk * nio));
+    const size_t staged = (size_t)(kStageHead + kChunk * h->row());
+    HLB_CHECK(h->stage.alloc(staged));
     HLB_CHECK(hipMemcpy(h->io_nf.p, nf.data(), sizeof(float) * nf.size(), hipMemcpyHostToDevice));
     HLB_CHECK(hipMemcpy(h->io_n.p, nd.data(), sizeof(double) * nd.size(), hipMemcpyHostToDevice));
-    HLB_CHECK(h->io_sp.alloc((size_t)kChunk));
-    HLB_CHECK(hipHostMalloc((void**)&h->h_stage, sizeof(double) * (3 * nio + 1) * kChunk, hipHostMallocDefault));
+    HLB_CHECK(hipHostMalloc((void**)&h->h_stage, sizeof(double) * staged, hipHostMallocDefault));
     std::vector<uint32_t> bits(nio, 0u);
     for (size_t g = 0; g < h->iolets.size(); ++g)
       if (h->iolets[g].IsWK() && h->iolets[g].dirs0 != 0) bits[g] = 1u << (INV[h->iolets[g].dirs0] - 1);
@@ -657,7 +658,7 @@ int upload_lattice(hlb_lattice* h) {
     h->wk_refs_host.clear();
     for (size_t g = 0; g < h->iolets.size(); ++g)
       if (h->iolets[g].IsWK())
-        h->wk_refs_host.push_back(WkRef{h->wk.p + g, h->io_dens.p, h->wk_contrib.p, h->wk_stride(), (int32_t)g, nio,
+        h->wk_refs_host.push_back(WkRef{h->wk.p + g, h->rows(), h->wk_contrib.p, h->wk_stride(), (int32_t)g, (int32_t)h->row(),
                                         h->fp32() ? 0 : 1, 0});
     HLB_CHECK(h->wk_refs.alloc(std::max<size_t>(1, h->wk_refs_host.size())));
     if (!h->wk_refs_host.empty())
@@ -884,9 +885,9 @@ Member32 member_record(const hlb_lattice* h, int props_at) {
   m.wss = h->wss.p;
   m.io_nf = h->io_nf.p;
   m.io_n = h->io_n.p;
-  m.io_dens = h->io_dens.p;
-  m.io_vmax = h->io_vmax.p;
-  m.io_vmax2 = h->io_vmax2.p;
+  m.io_dens = h->rows();
+  m.io_vmax = m.io_dens + h->iolet_count();
+  m.io_vmax2 = m.io_dens + 2 * h->iolet_count();
   m.wk_bit = h->wk_bit.p;
   m.wk_pos = h->wk_pos.p;
   m.wk_contrib = h->wk_contrib.p;
@@ -895,7 +896,7 @@ Member32 member_record(const hlb_lattice* h, int props_at) {
   m.S = h->S;
   m.SB = h->SB;
   m.SI = h->SI;
-  m.nio = std::max<int>(1, (int)h->iolets.size());
+  m.row = (int32_t)h->row();
   m.n_in = h->n_in;
   m.kernel = h->params.kernel;
   m.inlet_bc = h->params.inlet_bc;
@@ -910,7 +911,7 @@ Member32 member_record(const hlb_lattice* h, int props_at) {
   m.half_omega_minus = (float)h->half_omega_minus;
   m.les_k = (float)h->les_k;
   m.vtau = h->sponge_life > 0 ? h->vtau32.p : nullptr;
-  m.sp_t = h->io_sp.p;
+  m.sp_t = m.io_dens + 3 * h->iolet_count();
   m.sp_half = (double)(h->sponge_life / 2);
   m.sp_life = (double)h->sponge_life;
   return m;
@@ -924,47 +925,61 @@ uint32_t member_grid(int64_t nslab, int variant) {
   return shape_grid(l, (nslab + per - 1) / per);
 }
 
-// Writes the member record through the pinned staging slot; the caller has
-// synchronised the stream, so the slot is free.
+// Writes the member record through the head of the pinned staging; the caller
+// has synchronised the stream, so the staging is free.
 int upload_member(hlb_lattice* h, int props_at) {
-  *h->h_mem = member_record(h, props_at);
-  HLB_CHECK(hipMemcpyAsync(h->mem.p, h->h_mem, sizeof(Member32), hipMemcpyHostToDevice, h->stream));
+  const Member32 m = member_record(h, props_at);
+  std::memcpy(h->h_stage, &m, sizeof m);
+  HLB_CHECK(hipMemcpyAsync(h->stage.p, h->h_stage, sizeof m, hipMemcpyHostToDevice, h->stream));
   return HLB_OK;
 }
 
-// Stages the per-step iolet values of steps t .. t+n-1 for the device.
+// Forms the rows of steps t .. t+n-1 in the pinned staging: per iolet the ghost
+// density and the two speed factors, then the sponge's time.
+int form_rows(hlb_lattice* h, int64_t t, int64_t n) {
+  const int64_t nio = h->iolet_count(), row = h->row();
+  for (int64_t s = 0; s < n; ++s) {
+    double* r = h->h_stage + kStageHead + s * row;
+    const int rc = iolet_values(h, t + s, r, r + nio, r + 2 * nio);
+    if (rc != HLB_OK) return rc;
+    // LBGKLESSpongeLayer::CalculateTau reads the 1-indexed step; past the
+    // lifetime the Smagorinsky time applies alone (-1).
+    r[3 * nio] = t + s < h->sponge_life ? (double)(t + s) : -1.0;
+  }
+  return HLB_OK;
+}
+
 }  // namespace
 
 int stage_iolet_values(hlb_lattice* h, int64_t t, int64_t n, hipStream_t stream) {
-  const int nio = std::max<int>(1, (int)h->iolets.size());
-  double* dens = h->h_stage;
-  double* vmax = h->h_stage + (size_t)kChunk * nio;
-  double* vmax2 = h->h_stage + (size_t)2 * kChunk * nio;
-  for (int64_t s = 0; s < n; ++s) {
-    const int rc = iolet_values(h, t + s, dens + s * nio, vmax + s * nio, vmax2 + s * nio);
-    if (rc != HLB_OK) return rc;
-  }
-  HLB_CHECK(hipMemcpyAsync(h->io_dens.p, dens, sizeof(double) * n * nio, hipMemcpyHostToDevice, stream));
-  HLB_CHECK(hipMemcpyAsync(h->io_vmax.p, vmax, sizeof(double) * n * nio, hipMemcpyHostToDevice, stream));
-  HLB_CHECK(hipMemcpyAsync(h->io_vmax2.p, vmax2, sizeof(double) * n * nio, hipMemcpyHostToDevice, stream));
-  if (h->sponge_life > 0) {
-    // LBGKLESSpongeLayer::CalculateTau reads the 1-indexed step; past the
-    // lifetime the Smagorinsky time applies alone (-1).
-    double* sp = h->h_stage + (size_t)3 * kChunk * nio;
-    for (int64_t s = 0; s < n; ++s) sp[s] = t + s < h->sponge_life ? (double)(t + s) : -1.0;
-    HLB_CHECK(hipMemcpyAsync(h->io_sp.p, sp, sizeof(double) * n, hipMemcpyHostToDevice, stream));
-  }
+  const int rc = form_rows(h, t, n);
+  if (rc != HLB_OK) return rc;
+  HLB_CHECK(hipMemcpyAsync(h->rows(), h->h_stage + kStageHead, sizeof(double) * n * h->row(), hipMemcpyHostToDevice,
+                           stream));
   return HLB_OK;
 }
 
 namespace {
+
+// Everything a sequence of n steps reads from the host, in one copy: the
+// member record (FP32 form) and the rows behind it.  The caller has
+// synchronised the stream.
+int stage_sequence(hlb_lattice* h, int64_t n, bool props_last) {
+  if (!h->fp32()) return stage_iolet_values(h, h->t, n, h->stream);
+  const int rc = form_rows(h, h->t, n);
+  if (rc != HLB_OK) return rc;
+  const Member32 m = member_record(h, props_last ? (int)(n - 1) : -1);
+  std::memcpy(h->h_stage, &m, sizeof m);
+  HLB_CHECK(hipMemcpyAsync(h->stage.p, h->h_stage, sizeof(double) * (kStageHead + n * h->row()), hipMemcpyHostToDevice,
+                           h->stream));
+  return HLB_OK;
+}
 
 // Enqueues the launches of n steps whose iolet values (and, in the FP32
 // form, member record) are staged: kernel launches only, so the sequence can
 // be captured into a graph.
 int enqueue_steps(hlb_lattice* h, int64_t n, bool props_last) {
   if (n <= 0) return HLB_OK;
-  const int nio = std::max<int>(1, (int)h->iolets.size());
   const int nwk = (int)h->wk_refs_host.size();
   const int variant = h->launch_variant();
   const WkLaunch wk = wk_launch(h->wk_refs.p, nwk, n);
@@ -972,8 +987,8 @@ int enqueue_steps(hlb_lattice* h, int64_t n, bool props_last) {
   if (h->fp32()) {
     const uint32_t grid = member_grid(h->nslab, variant);
     for (int64_t s = 0; s < n; ++s) {
-      HLB_CHECK(launch_step_fp32(h->mem.p, nullptr, grid, (int)s, wk, variant, h->stream));
-      HLB_CHECK(launch_gzs_fp32(h->mem.p, h->gz_links.p, (int)h->gz_links_host.size(), (int)s, h->stream));
+      HLB_CHECK(launch_step_fp32(h->member(), nullptr, grid, (int)s, wk, variant, h->stream));
+      HLB_CHECK(launch_gzs_fp32(h->member(), h->gz_links.p, (int)h->gz_links_host.size(), (int)s, h->stream));
     }
     HLB_CHECK(launch_wk_flush(h->wk_refs.p, nwk, (int)(n - 1), h->stream));
     advance_state(h, n);
@@ -985,10 +1000,7 @@ int enqueue_steps(hlb_lattice* h, int64_t n, bool props_last) {
     const double* ain = first ? h->F.p : h->A[h->cur].p;
     double* aout = first ? h->A[h->cur].p : h->A[h->cur ^ 1].p;
     StepArgs a = make_args(h, ain, aout);
-    a.io_dens = h->io_dens.p + s * nio;
-    a.io_vmax = h->io_vmax.p + s * nio;
-    a.io_vmax2 = h->io_vmax2.p + s * nio;
-    a.sp_t = h->io_sp.p + s;
+    step_rows(h, a, s);
     a.step = (int32_t)s;
     a.wk = wk;
     a.wk_contrib = h->wk_contrib.p + (s & 1) * h->wk_stride();
@@ -1061,15 +1073,11 @@ int replay_graph(hlb_lattice* h, int64_t n, bool props_last) {
   return HLB_OK;
 }
 
-// Launches n staged steps, from a graph (captured on first use) or eagerly
-// when the handle's graphs are off; the handle's state advances by n steps.
+// Launches n staged steps, from a graph (captured on first use) or eagerly;
+// the handle's state advances by n steps.
 int launch_steps(hlb_lattice* h, int64_t n, bool props_last) {
   if (n <= 0) return HLB_OK;
-  if (h->fp32()) {
-    const int rc = upload_member(h, props_last ? (int)(n - 1) : -1);
-    if (rc != HLB_OK) return rc;
-  }
-  if (!h->use_graph) return enqueue_steps(h, n, props_last);
+  if (!h->use_graph || !h->replays(n)) return enqueue_steps(h, n, props_last);
   const int rc = prepare_graph(h, n, props_last);
   if (rc != HLB_OK) return rc;
   return replay_graph(h, n, props_last);
@@ -1084,9 +1092,10 @@ int run_steps(hlb_lattice* h, int64_t nsteps, uint32_t flags) {
     // The staging buffers are reused per chunk: wait for the launches that
     // read the previous chunk's values.
     HLB_CHECK(hipStreamSynchronize(h->stream));
-    int rc = stage_iolet_values(h, h->t, chunk, h->stream);
+    const bool props_last = (flags & HLB_STEP_PROPERTIES) && done + chunk == nsteps;
+    int rc = stage_sequence(h, chunk, props_last);
     if (rc != HLB_OK) return rc;
-    rc = launch_steps(h, chunk, (flags & HLB_STEP_PROPERTIES) && done + chunk == nsteps);
+    rc = launch_steps(h, chunk, props_last);
     if (rc != HLB_OK) return rc;
     done += chunk;
   }
@@ -1101,7 +1110,7 @@ int materialise_f(hlb_lattice* h) {
     HLB_CHECK(hipStreamSynchronize(h->stream));
     int rc = upload_member(h, -1);
     if (rc != HLB_OK) return rc;
-    HLB_CHECK(launch_gather_fp32(h->mem.p, h->nslab, h->F32.p, h->stream));
+    HLB_CHECK(launch_gather_fp32(h->member(), h->nslab, h->F32.p, h->stream));
     return HLB_OK;
   }
   if (!h->F.p) HLB_CHECK(h->F.alloc((size_t)Q * h->S));
@@ -1337,18 +1346,14 @@ extern "C" int hlb_step_timed(hlb_handle h, int64_t nsteps, uint32_t flags, doub
   if (nsteps < 0 || nsteps > kChunk) return fail(HLB_EINVAL, "hlb_step_timed: 0 to 1024 steps per timed call");
   if (!h->f_valid) return fail(HLB_EINVAL, "hlb_step_timed: no initial condition");
   HLB_CHECK(hipStreamSynchronize(h->stream));
-  int rc = stage_iolet_values(h, h->t, nsteps, h->stream);
-  if (rc != HLB_OK) return rc;
   const bool props = (flags & HLB_STEP_PROPERTIES) != 0;
-  const bool graph = h->use_graph && nsteps > 0;
+  int rc = stage_sequence(h, nsteps, props);
+  if (rc != HLB_OK) return rc;
+  const bool graph = h->use_graph && nsteps > 0 && h->replays(nsteps);
   if (graph) {
     // Capture outside the timed region: a sequence not seen before is
     // recorded by a first call that runs nothing, then replayed below.
     rc = prepare_graph(h, nsteps, props);
-    if (rc != HLB_OK) return rc;
-  }
-  if (h->fp32()) {
-    rc = upload_member(h, props ? (int)(nsteps - 1) : -1);
     if (rc != HLB_OK) return rc;
   }
   HLB_CHECK(hipEventRecord(h->ev0, h->stream));
@@ -1474,13 +1479,15 @@ extern "C" int hlb_stability(hlb_handle h, int* stable) {
   if (!h->f_valid) return fail(HLB_EINVAL, "hlb_stability: no state");
   int rc = materialise_f(h);
   if (rc != HLB_OK) return rc;
-  HLB_CHECK(hipMemsetAsync(h->flag.p, 0, sizeof(int), h->stream));
-  if (h->fp32()) HLB_CHECK(launch_unstable_fp32(h->tables(), h->F32.p, h->S, h->flag.p, h->stream));
-  else HLB_CHECK(launch_unstable_fp64(h->tables(), h->F.p, h->S, h->flag.p, h->stream));
-  int flag = 0;
-  HLB_CHECK(hipMemcpyAsync(&flag, h->flag.p, sizeof(int), hipMemcpyDeviceToHost, h->stream));
+  // the scan writes its verdict straight into pinned host memory; earlier
+  // work on the stream (materialise_f's) has not touched it
+  volatile int* flag = reinterpret_cast<volatile int*>(h->result());
+  *flag = 0;
+  int* f = reinterpret_cast<int*>(h->result());
+  if (h->fp32()) HLB_CHECK(launch_unstable_fp32(h->tables(), h->F32.p, h->S, f, h->stream));
+  else HLB_CHECK(launch_unstable_fp64(h->tables(), h->F.p, h->S, f, h->stream));
   HLB_CHECK(hipStreamSynchronize(h->stream));
-  *stable = flag ? 0 : 1;
+  *stable = *flag ? 0 : 1;
   return HLB_OK;
 }
 
@@ -1489,11 +1496,11 @@ extern "C" int hlb_monitor(hlb_handle h, double out[4]) {
   if (!h->device_ready) return fail(HLB_EINVAL, "hlb_monitor: no state");
   if (!h->mon_scratch.p) {
     HLB_CHECK(h->mon_scratch.alloc(monitor_scratch(h->nslab)));
-    HLB_CHECK(h->mon_out.alloc(4));
   }
-  HLB_CHECK(launch_monitor(h->tables(), h->rho.p, h->u.p, h->S, h->mon_scratch.p, h->mon_out.p, h->stream));
-  HLB_CHECK(hipMemcpyAsync(out, h->mon_out.p, 4 * sizeof(double), hipMemcpyDeviceToHost, h->stream));
+  // the last pass writes the four results straight into pinned host memory
+  HLB_CHECK(launch_monitor(h->tables(), h->rho.p, h->u.p, h->S, h->mon_scratch.p, h->result(), h->stream));
   HLB_CHECK(hipStreamSynchronize(h->stream));
+  std::memcpy(out, h->result(), 4 * sizeof(double));
   return HLB_OK;
 }
 

@@ -43,6 +43,21 @@ hipError_t launch_cycle_delta(const double* u, float* prev, int64_t N, int64_t S
 inline constexpr double kPi = 3.14159265358979323846264338327950288;  // src/constants.h:17
 inline constexpr int64_t kChunk = 1024;  // steps of iolet values staged per upload
 
+inline constexpr int64_t kStageHead = 64;  // doubles ahead of them for the FP32 form's member record
+inline constexpr int64_t kStageResult = 56;  // where the pinned staging's head takes the monitors' results
+static_assert(sizeof(Member32) <= sizeof(double) * kStageResult, "the record fits the staging's head");
+
+// Whether a sequence of n one-launch steps over nslab slabs is replayed from a
+// captured graph rather than launched step by step.  A replay costs ~20 us to
+// start and, the first time, ~4 us a step to capture; a launch from the host
+// costs ~2.4 us, hidden behind the step before it, and ~0.6 us more between
+// kernels, which shows only while steps take a few us.  Graph / eager, us for n
+// steps (FP64): 6.5k sites n = 8 68 / 67, n = 16 111 / 117, n = 300 1636 / 1880;
+// 30k sites n = 16 120 / 124, n = 300 1801 / 2021; 67k sites (~1.4k slabs) n =
+// 16 159 / 153, n = 300 2443 / 2541; 127k sites (~2.5k slabs) n = 16 197 / 190,
+// n = 300 3208 / 3218; 430k sites n = 8 226 / 217, n = 300 7471 / 7468.
+inline bool replay_pays(int64_t n, int64_t nslab) { return n >= 16 && nslab <= 2048; }
+
 inline int64_t round_up(int64_t v, int64_t m) { return (v + m - 1) / m * m; }
 
 struct HostIolet {
@@ -113,12 +128,11 @@ struct hlb_lattice {
   std::vector<int32_t> bsite;  // reference index of boundary slot b
   std::vector<int32_t> isite;  // reference index of iolet slot i
   int64_t S = 0, NB = 0, SB = 0, NI = 0, SI = 0;
-  hlb::DevBuf<double> A[2], F, G, ladd_s, rho, u, wss, io_n, io_dens, io_vmax, io_vmax2, feq_vals;
+  hlb::DevBuf<double> A[2], F, G, ladd_s, rho, u, wss, io_n, feq_vals;
   hlb::DevBuf<hlb::BndRec> bnd;  // boundary records
   hlb::DevBuf<hlb::SlabRec> rec;  // slab records
   hlb::DevBuf<float> bq, bnrm, io_nf;
   hlb::DevBuf<int32_t> dinv;      // inv on the device (transfer.hip)
-  hlb::DevBuf<int> flag;
   // Guo-Zheng-Shi walls (params.wall_bc == HLB_WALL_GZS).
   std::vector<hlb::GzsLink> gz_links_host;
   std::vector<uint64_t> h_pmask;
@@ -132,12 +146,8 @@ struct hlb_lattice {
   hlb::DevBuf<float> P32, GW32;
   hlb::DevBuf<char> mon_scratch;  // monitor partials, allocated on first use
   hlb::DevBuf<double> stress;     // 17 stress planes, allocated on first use
-  hlb::DevBuf<double> mon_out;
-  // FP32-shifted storage (params.precision == HLB_FP32_SHIFTED): float A, F,
-  // G and the one-member table the member-table kernel reads.
+  // FP32-shifted storage (params.precision == HLB_FP32_SHIFTED): float A, F, G.
   hlb::DevBuf<float> A32[2], F32, G32, feq32;
-  hlb::DevBuf<hlb::Member32> mem;
-  hlb::Member32* h_mem = nullptr;  // pinned staging of the member record
   // Windkessel iolets: device state, coupling bit per iolet, per-site terms,
   // coupling sites per iolet in the reference's site order.
   bool any_wk = false;
@@ -157,9 +167,20 @@ struct hlb_lattice {
   int64_t sponge_life = 0;
   double sponge_ratio = 1.0, sponge_width = 0.0;
   std::vector<double> h_vtau;
-  hlb::DevBuf<double> vtau64, io_sp;
+  hlb::DevBuf<double> vtau64;
   hlb::DevBuf<float> vtau32;
-  double* h_stage = nullptr;  // pinned staging for per-step iolet values (and sponge times)
+  // What a sequence of steps reads from the host, and its pinned staging: the
+  // one-member table the FP32 kernel reads (kStageHead doubles), then a row per
+  // step (per iolet the ghost density, then the two speed factors, then the
+  // sponge's time).
+  hlb::DevBuf<double> stage;
+  double* h_stage = nullptr;
+  int iolet_count() const { return iolets.empty() ? 1 : (int)iolets.size(); }
+  int64_t row() const { return 3 * (int64_t)iolet_count() + 1; }
+  double* rows() const { return stage.p + hlb::kStageHead; }
+  // Pinned doubles the monitors' kernels write their results to.
+  double* result() const { return h_stage + hlb::kStageResult; }
+  hlb::Member32* member() const { return reinterpret_cast<hlb::Member32*>(stage.p); }
   int cur = 0;                // A[cur] holds the latest post-collision values
   bool have_post = false;     // false: the next step reads the pre-collision F
   bool f_valid = false;
@@ -185,6 +206,8 @@ struct hlb_lattice {
   };
   std::vector<StepGraph> graphs;
   bool use_graph = true;
+  // GZS walls add a launch per step, which a replay saves at any size.
+  bool replays(int64_t n) const { return hlb::replay_pays(n, gz_links_host.empty() ? nslab : 0); }
   void drop_graphs() {
     for (StepGraph& g : graphs) (void)hipGraphExecDestroy(g.exec);
     graphs.clear();
@@ -199,7 +222,6 @@ struct hlb_lattice {
     if (ev0) (void)hipEventDestroy(ev0);
     if (ev1) (void)hipEventDestroy(ev1);
     if (h_stage) (void)hipHostFree(h_stage);
-    if (h_mem) (void)hipHostFree(h_mem);
     if (device_ready) hlb::transfer_close();
   }
   bool fp32() const { return params.precision == HLB_FP32_SHIFTED; }

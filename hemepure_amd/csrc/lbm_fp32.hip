@@ -207,7 +207,7 @@ struct IoletIn32 {
   uint32_t wk;
 };
 __device__ __forceinline__ IoletIn32 load_iolet32(const Member32& m, int step, uint32_t gi) {
-  const double dens = ldp(m.io_dens + (int64_t)step * m.nio, gi);
+  const double dens = ldp(m.io_dens + (int64_t)step * m.row, gi);
   return IoletIn32{(float)dens,
                    (float)(dens - 1.0),
                    {ldp(m.io_nf, 3u * gi), ldp(m.io_nf, 3u * gi + 1), ldp(m.io_nf, 3u * gi + 2)},
@@ -273,7 +273,7 @@ __device__ __forceinline__ void iolet_links32(const Member32& m, int step, const
     const float usq15 = 1.5f * (gx * gx + gy * gy + gz * gz) * inv;
     nash_links32(m, r, io.drho, inv, usq15, gx, gy, gz);
   } else {
-    const int64_t row = (int64_t)step * m.nio;
+    const int64_t row = (int64_t)step * m.row;
     ladd_groups32(m, r, LaddIn32{ldp(m.io_vmax + row, r.gi), ldp(m.io_vmax2 + row, r.gi), {io.n[0], io.n[1], io.n[2]}},
                   rho, gpost);
   }
@@ -363,7 +363,7 @@ __device__ __forceinline__ Collision32 collide32(const Member32& m, int step, ui
     const float root = __builtin_amdgcn_sqrtf(__builtin_fmaf(m.les_k, __builtin_amdgcn_sqrtf(q2), m.tau * m.tau));
     c.tau = 0.5f * (m.tau + root);
     if (m.vtau != nullptr) {
-      const double t = ldp(m.sp_t, (uint32_t)step);
+      const double t = ldp(m.sp_t + (int64_t)step * m.row, 0);
       if (t >= 0.0) {
         const float vt = ldp(m.vtau, d);
         if (t <= m.sp_half) c.tau = vt == m.tau ? c.tau : vt;
@@ -528,8 +528,8 @@ __global__ __launch_bounds__(kBlock) void gzs_links_fp32(const Member32* __restr
 #pragma unroll
     for (int j = 0; j < Q; ++j) gneq[j] = q * gneq[j] + (1.0f - q) * (h[j] - heq[j]);
   } else if (lk.mode == 3) {
-    const double* vmax = m.io_vmax + (int64_t)step * m.nio;
-    const double* vmax2 = m.io_vmax2 + (int64_t)step * m.nio;
+    const double* vmax = m.io_vmax + (int64_t)step * m.row;
+    const double* vmax2 = m.io_vmax2 + (int64_t)step * m.row;
     const float sp = (float)(ldp(vmax, (uint32_t)lk.gi) * lk.s + ldp(vmax2, (uint32_t)lk.gi) * lk.s2);
 #pragma unroll
     for (int c = 0; c < 3; ++c) {

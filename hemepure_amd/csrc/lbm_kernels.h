@@ -212,10 +212,10 @@ struct WkIolet {
 // serve the Windkessel iolets of every lattice in a batch.
 struct WkRef {
   WkIolet* w;
-  double* io_dens;        // the lattice's ghost-density rows (stride nio)
+  double* io_dens;        // the lattice's rows of per-step values, ghost densities first
   const double* contrib;  // the lattice's u.(-n) terms in the coupling order, even steps' and odd steps'
   int64_t stride;         // from the first to the second
-  int32_t g, nio;         // iolet index in its lattice, row stride
+  int32_t g, row;         // iolet index in its lattice, row stride
   int32_t ordered;        // 1: sum in the reference's site order (FP64 form); 0: tree (FP32-shifted form)
   int32_t pad_;
 };
@@ -297,7 +297,7 @@ struct Member32 {
   double* wss;
   const float* io_nf;
   const double* io_n;
-  const double* io_dens;  // rows of nio per step of the launch sequence
+  const double* io_dens;  // one value per iolet, a row per step of the launch sequence
   const double* io_vmax;
   const double* io_vmax2;
   const uint32_t* wk_bit;
@@ -305,7 +305,7 @@ struct Member32 {
   double* wk_contrib;     // even steps' terms, then wk_stride on the odd steps'
   int64_t wk_stride;
   int64_t N, S, SB, SI;
-  int32_t nio, n_in;
+  int32_t row, n_in;      // row stride of the per-step values
   int32_t kernel, inlet_bc, outlet_bc;
   int32_t cur0;           // A[cur0] holds the latest values when the sequence starts
   int32_t first0;         // 1: step 0 of the sequence reads F (pre-collision)
@@ -317,7 +317,7 @@ struct Member32 {
   float* P;
   const float* GW;
   const float* vtau;      // LES sponge layer (see StepArgs); nullptr: none
-  const double* sp_t;     // rows of one per step of the launch sequence
+  const double* sp_t;     // one value, a row per step of the launch sequence
   double sp_half, sp_life;
 };
 

@@ -127,7 +127,7 @@ __device__ __forceinline__ void wk_advance(const WkRef& ref, int step, bool last
   w.flowRate = flow;
   w.flowRateNew = 0.0;
   w.siteCount = 0.0;
-  if (!last) ref.io_dens[(int64_t)(step + 1) * ref.nio + ref.g] = next;
+  if (!last) ref.io_dens[(int64_t)(step + 1) * ref.row + ref.g] = next;
 }
 
 // True for the launch's leading workgroups, which serve the Windkessel iolets.

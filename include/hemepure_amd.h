@@ -229,10 +229,10 @@ int hlb_autotune(hlb_handle h, int64_t trial_steps, int* variant, double* ms_per
  * event, so the timed region holds the replay only. */
 int hlb_step_timed(hlb_handle h, int64_t nsteps, uint32_t flags, double* ms);
 /* No counterpart in the reference (its steps are host loops over site
- * ranges).  Step sequences of up to 1024 steps are captured into HIP graphs
- * on first use and replayed (the default, enable = 1), so small lattices are
- * not bound by per-launch host cost; enable = 0 launches every kernel
- * eagerly.  Results are bit-identical either way.  Changing it, or tau via
+ * ranges).  Step sequences (16 to 1024 steps) of small lattices are captured
+ * into HIP graphs on first use and replayed (the default, enable = 1), so they
+ * are not bound by per-launch cost; short sequences and lattices whose steps
+ * hide it, and with enable = 0 every sequence, are launched step by step.  Results are bit-identical either way.  Changing it, or tau via
  * hlb_set_params, drops the captured graphs. */
 int hlb_set_graphs(hlb_handle h, int enable);
 /* Blocks until the handle's stream is idle. */
@@ -370,7 +370,7 @@ int hlb_batch_step(hlb_batch_handle b, int64_t nsteps, uint32_t flags);
 /* Like hlb_batch_step for at most 1024 steps; blocks and returns the device
  * milliseconds of the launches (HIP events on the batch's stream). */
 int hlb_batch_step_timed(hlb_batch_handle b, int64_t nsteps, uint32_t flags, double* ms);
-/* Step sequences are captured into HIP graphs and replayed (default on). */
+/* As hlb_set_graphs, for the batch's sequences (default on). */
 int hlb_batch_set_graphs(hlb_batch_handle b, int enable);
 /* Launch variant, as for hlb_set_variant of an FP32-shifted lattice (0..215). */
 int hlb_batch_set_variant(hlb_batch_handle b, int variant);
