@@ -235,27 +235,41 @@ void device_order(hlb_lattice* h, int order) {
                 ntz = ((int64_t)L.blocks[2] * L.bs + 7) / 8;
   auto tile_of = [&](int64_t x, int64_t y, int64_t z) { return (x * nty + y) * ntz + z; };
   std::vector<int32_t> brickOf((size_t)(ntx * nty * ntz), -1);
-  for (int64_t k = 0; k < N; ++k)
-    brickOf[tile_of(L.coords[3 * k] >> 3, L.coords[3 * k + 1] >> 3, L.coords[3 * k + 2] >> 3)] = 0;
+  parallel_ranges(N, [&](int, int64_t lo, int64_t hi) {
+    for (int64_t k = lo; k < hi; ++k) {
+      int32_t* b = &brickOf[(size_t)tile_of(L.coords[3 * k] >> 3, L.coords[3 * k + 1] >> 3, L.coords[3 * k + 2] >> 3)];
+      if (__atomic_load_n(b, __ATOMIC_RELAXED) != 0) __atomic_store_n(b, 0, __ATOMIC_RELAXED);
+    }
+  });
   std::vector<int64_t> brickTile;
   for (size_t t = 0; t < brickOf.size(); ++t)
-    if (brickOf[t] >= 0) brickTile.push_back((int64_t)t);
-  for (size_t i = 0; i < brickTile.size(); ++i) brickOf[(size_t)brickTile[i]] = (int32_t)i;
+    if (brickOf[t] >= 0) {
+      brickOf[t] = (int32_t)brickTile.size();
+      brickTile.push_back((int64_t)t);
+    }
   const int64_t NBr = (int64_t)brickTile.size();
   h->nbrick = NBr;
+  constexpr int64_t kBrickGrain = kGrain / kBrickSites;
   // the site at each position of each brick
-  std::vector<int32_t> at((size_t)NBr * kBrickSites, -1);
-  for (int64_t k = 0; k < N; ++k) {
-    const int32_t x = L.coords[3 * k], y = L.coords[3 * k + 1], z = L.coords[3 * k + 2];
-    const int64_t brick = brickOf[tile_of(x >> 3, y >> 3, z >> 3)];
-    at[(size_t)brick * kBrickSites + ((x & 7) * 8 + (y & 7)) * 8 + (z & 7)] = (int32_t)k;
-  }
+  RawVector<int32_t> at;
+  at.resize((size_t)NBr * kBrickSites);
+  parallel_ranges(NBr, [&](int, int64_t lo, int64_t hi) {
+    std::fill(at.begin() + lo * kBrickSites, at.begin() + hi * kBrickSites, -1);
+  }, kBrickGrain);
+  parallel_ranges(N, [&](int, int64_t lo, int64_t hi) {
+    for (int64_t k = lo; k < hi; ++k) {
+      const int32_t x = L.coords[3 * k], y = L.coords[3 * k + 1], z = L.coords[3 * k + 2];
+      const int64_t brick = brickOf[(size_t)tile_of(x >> 3, y >> 3, z >> 3)];
+      at[(size_t)brick * kBrickSites + ((x & 7) * 8 + (y & 7)) * 8 + (z & 7)] = (int32_t)k;
+    }
+  });
   // fluid masks of every layer of every brick
   std::vector<uint64_t> fmAll((size_t)NBr * 8, 0);
-  for (int64_t k = 0; k < NBr; ++k)
-    for (int x = 0; x < 8; ++x)
+  parallel_ranges(NBr * 8, [&](int, int64_t lo, int64_t hi) {
+    for (int64_t i = lo; i < hi; ++i)
       for (int lane = 0; lane < kSlab; ++lane)
-        if (at[(size_t)k * kBrickSites + x * kSlab + lane] >= 0) fmAll[(size_t)k * 8 + x] |= 1ull << lane;
+        if (at[(size_t)i * kSlab + lane] >= 0) fmAll[(size_t)i] |= 1ull << lane;
+  }, 8 * kBrickGrain);
   h->slab_order = order;
   if (order == HLB_ORDER_AUTO) {
     // median slab distance from a brick to its y neighbour in TILE order
@@ -302,8 +316,6 @@ void device_order(hlb_lattice* h, int order) {
   h->S = round_up(std::max<int64_t>(next, 1), 64);
   h->perm.assign((size_t)h->S, -1);
   h->inv.assign((size_t)N, -1);
-  h->bsite.clear();
-  h->isite.clear();
   h->h_rec.assign((size_t)std::max<int64_t>(h->nslab, 1), SlabRec{});
   // the slab at layer x + dx of the brick at (dy, dz) from brick k, or -1
   auto reach = [&](int64_t k, int x, int dx, int dy, int dz) -> int32_t {
@@ -315,36 +327,57 @@ void device_order(hlb_lattice* h, int order) {
     const int32_t nb = brickOf[tile_of(tx, ty, tz)];
     return nb < 0 ? -1 : slabOf[(size_t)nb * 8 + (xx & 7)];
   };
-  for (int64_t r = 0; r < h->nslab; ++r) {
-    const int64_t k = h->h_slab[r] >> 3;
-    const int x = h->h_slab[r] & 7;
-    SlabRec& R = h->h_rec[r];
-    std::memset(&R, 0, sizeof R);
-    R.sid = h->h_slab[r];
-    R.bbase = (int32_t)h->bsite.size();
-    for (int dx = -1; dx <= 1; ++dx)
-      for (int dy = -1; dy <= 1; ++dy)
-        for (int dz = -1; dz <= 1; ++dz) {
-          if (dx != 0 && dy != 0 && dz != 0) continue;  // no such link in D3Q19
-          const int e = reach_entry(dx, dy, dz);
-          const int32_t q = reach(k, x, dx, dy, dz);
-          R.fm[e] = q < 0 ? 0 : h->h_fmask[q];
-          R.base[e] = q < 0 ? 0 : h->h_sbase[q];
-        }
-    uint32_t slot = (uint32_t)h->h_sbase[r];
-    for (int lane = 0; lane < kSlab; ++lane) {
-      const int32_t site = at[(size_t)k * kBrickSites + x * kSlab + lane];
-      if (site < 0) continue;
-      h->perm[slot] = site;
-      h->inv[site] = (int32_t)slot;
-      ++slot;
-      if (site >= L.off[1]) {
-        R.bmask |= 1ull << lane;
-        h->bsite.push_back(site);
+  // per slab its boundary and iolet sites, then where their numbering starts
+  std::vector<int32_t> firstB((size_t)h->nslab + 1, 0), firstI((size_t)h->nslab + 1, 0);
+  constexpr int64_t kSlabGrain = kGrain / kSlab;
+  parallel_ranges(h->nslab, [&](int, int64_t lo, int64_t hi) {
+    for (int64_t r = lo; r < hi; ++r) {
+      const int32_t* sites = &at[(size_t)h->h_slab[r] * kSlab];
+      for (int lane = 0; lane < kSlab; ++lane) {
+        if (sites[lane] >= L.off[1]) firstB[(size_t)r + 1]++;
+        if (sites[lane] >= L.off[2]) firstI[(size_t)r + 1]++;
       }
-      if (site >= L.off[2]) h->isite.push_back(site);
     }
+  }, kSlabGrain);
+  for (int64_t r = 0; r < h->nslab; ++r) {
+    firstB[(size_t)r + 1] += firstB[(size_t)r];
+    firstI[(size_t)r + 1] += firstI[(size_t)r];
   }
+  h->bsite.resize((size_t)firstB.back());
+  h->isite.resize((size_t)firstI.back());
+  parallel_ranges(h->nslab, [&](int, int64_t lo, int64_t hi) {
+    for (int64_t r = lo; r < hi; ++r) {
+      const int64_t k = h->h_slab[r] >> 3;
+      const int x = h->h_slab[r] & 7;
+      SlabRec& R = h->h_rec[r];
+      std::memset(&R, 0, sizeof R);
+      R.sid = h->h_slab[r];
+      R.bbase = firstB[(size_t)r];
+      for (int dx = -1; dx <= 1; ++dx)
+        for (int dy = -1; dy <= 1; ++dy)
+          for (int dz = -1; dz <= 1; ++dz) {
+            if (dx != 0 && dy != 0 && dz != 0) continue;  // no such link in D3Q19
+            const int e = reach_entry(dx, dy, dz);
+            const int32_t q = reach(k, x, dx, dy, dz);
+            R.fm[e] = q < 0 ? 0 : h->h_fmask[q];
+            R.base[e] = q < 0 ? 0 : h->h_sbase[q];
+          }
+      int32_t nb = firstB[(size_t)r], ni = firstI[(size_t)r];
+      uint32_t slot = (uint32_t)h->h_sbase[r];
+      for (int lane = 0; lane < kSlab; ++lane) {
+        const int32_t site = at[(size_t)h->h_slab[r] * kSlab + lane];
+        if (site < 0) continue;
+        h->perm[slot] = site;
+        h->inv[site] = (int32_t)slot;
+        ++slot;
+        if (site >= L.off[1]) {
+          R.bmask |= 1ull << lane;
+          h->bsite[(size_t)nb++] = site;
+        }
+        if (site >= L.off[2]) h->isite[(size_t)ni++] = site;
+      }
+    }
+  }, kSlabGrain);
   h->NB = (int64_t)h->bsite.size();
   h->NI = (int64_t)h->isite.size();
   h->SB = round_up(std::max<int64_t>(h->NB, 1), 64);
@@ -534,34 +567,26 @@ int upload_sponge(hlb_lattice* h) {
 int upload_lattice(hlb_lattice* h) {
   const HostLattice& L = h->L;
   const int64_t N = L.N, S = h->S, SB = h->SB, SI = h->SI, NB = h->NB;
+  DevPack pack;
+  // the two distribution sets are one allocation, the field arrays another
   if (h->fp32()) {
-    HLB_CHECK(h->A32[0].alloc((size_t)Q * S));
-    HLB_CHECK(h->A32[1].alloc((size_t)Q * S));
-    HLB_CHECK(h->G32.alloc((size_t)Q * SI));
-    HLB_CHECK(h->feq32.alloc(Q));
-    HLB_CHECK(hipMemsetAsync(h->A32[0].p, 0, sizeof(float) * Q * S, h->stream));
-    HLB_CHECK(hipMemsetAsync(h->A32[1].p, 0, sizeof(float) * Q * S, h->stream));
-    HLB_CHECK(hipMemsetAsync(h->G32.p, 0, sizeof(float) * Q * SI, h->stream));
+    HLB_CHECK(h->a_mem.alloc(sizeof(float) * 2 * Q * S));
+    for (int c = 0; c < 2; ++c) h->A32[c].view(h->a_mem.p + sizeof(float) * Q * S * c, (size_t)Q * S);
+    pack.add(h->G32, (const float*)nullptr, (size_t)Q * SI);
+    pack.add(h->feq32, (const float*)nullptr, (size_t)Q);
   } else {
-    HLB_CHECK(h->A[0].alloc((size_t)Q * S));
-    HLB_CHECK(h->A[1].alloc((size_t)Q * S));
-    HLB_CHECK(h->G.alloc((size_t)Q * SI));
-    HLB_CHECK(hipMemsetAsync(h->A[0].p, 0, sizeof(double) * Q * S, h->stream));
-    HLB_CHECK(hipMemsetAsync(h->A[1].p, 0, sizeof(double) * Q * S, h->stream));
-    HLB_CHECK(hipMemsetAsync(h->G.p, 0, sizeof(double) * Q * SI, h->stream));
+    HLB_CHECK(h->a_mem.alloc(sizeof(double) * 2 * Q * S));
+    for (int c = 0; c < 2; ++c) h->A[c].view(h->a_mem.p + sizeof(double) * Q * S * c, (size_t)Q * S);
+    pack.add(h->G, (const double*)nullptr, (size_t)Q * SI);
   }
-  HLB_CHECK(h->bnd.alloc((size_t)SB));
-  HLB_CHECK(h->bq.alloc((size_t)18 * SB));
-  HLB_CHECK(h->bnrm.alloc((size_t)3 * SB));
-  HLB_CHECK(h->ladd_s.alloc((size_t)36 * SI));
-  HLB_CHECK(h->rho.alloc((size_t)S));
-  HLB_CHECK(h->u.alloc((size_t)3 * S));
-  HLB_CHECK(h->wss.alloc((size_t)S));
-  HLB_CHECK(h->feq_vals.alloc(Q));
+  HLB_CHECK(hipMemsetAsync(h->a_mem.p, 0, h->a_mem.n, h->stream));
   // Holes are never written: keep the field arrays defined there.
-  HLB_CHECK(hipMemsetAsync(h->rho.p, 0, sizeof(double) * S, h->stream));
-  HLB_CHECK(hipMemsetAsync(h->u.p, 0, sizeof(double) * 3 * S, h->stream));
-  HLB_CHECK(hipMemsetAsync(h->wss.p, 0, sizeof(double) * S, h->stream));
+  HLB_CHECK(h->fields_mem.alloc(sizeof(double) * 5 * S));
+  HLB_CHECK(hipMemsetAsync(h->fields_mem.p, 0, h->fields_mem.n, h->stream));
+  h->rho.view(h->fields_mem.p, (size_t)S);
+  h->u.view(h->fields_mem.p + sizeof(double) * S, (size_t)3 * S);
+  h->wss.view(h->fields_mem.p + sizeof(double) * 4 * S, (size_t)S);
+  pack.add(h->feq_vals, (const double*)nullptr, (size_t)Q);
 
   // Guo-Zheng-Shi tables.
   {
@@ -569,16 +594,11 @@ int upload_lattice(hlb_lattice* h) {
     if (rc != HLB_OK) return rc;
     if (!h->gz_links_host.empty()) {
       const size_t nl = h->gz_links_host.size();
-      HLB_CHECK(h->gz_links.alloc(nl));
-      HLB_CHECK(hipMemcpy(h->gz_links.p, h->gz_links_host.data(), sizeof(GzsLink) * nl, hipMemcpyHostToDevice));
-      HLB_CHECK(h->pmask.alloc(h->h_pmask.size()));
-      HLB_CHECK(hipMemcpy(h->pmask.p, h->h_pmask.data(), sizeof(uint64_t) * h->h_pmask.size(), hipMemcpyHostToDevice));
-      HLB_CHECK(h->pbase.alloc(h->h_pbase.size()));
-      HLB_CHECK(hipMemcpy(h->pbase.p, h->h_pbase.data(), sizeof(int32_t) * h->h_pbase.size(), hipMemcpyHostToDevice));
-      HLB_CHECK(h->bgz.alloc((size_t)SB));
-      HLB_CHECK(hipMemcpy(h->bgz.p, h->h_bgz.data(), sizeof(uint32_t) * SB, hipMemcpyHostToDevice));
-      HLB_CHECK(h->bgzbase.alloc((size_t)SB));
-      HLB_CHECK(hipMemcpy(h->bgzbase.p, h->h_bgzbase.data(), sizeof(int32_t) * SB, hipMemcpyHostToDevice));
+      pack.add(h->gz_links, h->gz_links_host);
+      pack.add(h->pmask, h->h_pmask);
+      pack.add(h->pbase, h->h_pbase);
+      pack.add(h->bgz, reinterpret_cast<const uint32_t*>(h->h_bgz.data()), (size_t)SB);
+      pack.add(h->bgzbase, h->h_bgzbase.data(), (size_t)SB);
       if (h->fp32()) {
         HLB_CHECK(h->P32.alloc((size_t)Q * h->SP));
         HLB_CHECK(h->GW32.alloc(nl));
@@ -588,42 +608,43 @@ int upload_lattice(hlb_lattice* h) {
       }
     }
   }
-  // Slab records.
-  HLB_CHECK(h->rec.alloc(h->h_rec.size()));
-  HLB_CHECK(hipMemcpy(h->rec.p, h->h_rec.data(), sizeof(SlabRec) * h->h_rec.size(), hipMemcpyHostToDevice));
+  // Slab records and the site -> slot index.
+  pack.add(h->rec, h->h_rec);
+  pack.add(h->dinv, h->inv.data(), h->inv.size());
   // Boundary arrays in device order.
+  std::vector<BndRec> rec(SB, BndRec{0, 0, 0, 0});
+  std::vector<float> q((size_t)18 * SB, 0.0f), nr((size_t)3 * SB, 0.0f);
   {
     std::vector<int32_t> iolIndex(N, -1);
     for (int64_t i = 0; i < h->NI; ++i) iolIndex[h->isite[i]] = (int32_t)i;
-    std::vector<BndRec> rec(SB, BndRec{0, 0, 0, 0});
-    std::vector<float> q((size_t)18 * SB, 0.0f), nr((size_t)3 * SB, 0.0f);
-    for (int64_t b = 0; b < NB; ++b) {
-      const int64_t k = h->bsite[b];
-      BndRec& R = rec[b];
-      const uint32_t wm = L.wall[k];
-      R.iolet = L.iolet[k];
-      if (wm != 0) R.far |= 1u << 31;
-      // BouzidiFirdaousLallemandDelegate.h:44-93: a wall link whose opposite is
-      // no wall interpolates, with the site's own opposite value from q = 1/2 on
-      for (int j = 1; j < Q && h->params.wall_bc == HLB_WALL_BFL; ++j) {
-        const int ib = INV[j];
-        if (!((wm >> (ib - 1)) & 1u) || ((wm >> (j - 1)) & 1u)) continue;
-        (L.q[k * 18 + ib - 1] < 0.5f ? R.near : R.far) |= 1u << (j - 1);
+    parallel_ranges(NB, [&](int, int64_t lo, int64_t hi) {
+      for (int64_t b = lo; b < hi; ++b) {
+        const int64_t k = h->bsite[b];
+        BndRec& R = rec[b];
+        const uint32_t wm = L.wall[k];
+        R.iolet = L.iolet[k];
+        if (wm != 0) R.far |= 1u << 31;
+        // BouzidiFirdaousLallemandDelegate.h:44-93: a wall link whose opposite is
+        // no wall interpolates, with the site's own opposite value from q = 1/2 on
+        for (int j = 1; j < Q && h->params.wall_bc == HLB_WALL_BFL; ++j) {
+          const int ib = INV[j];
+          if (!((wm >> (ib - 1)) & 1u) || ((wm >> (j - 1)) & 1u)) continue;
+          (L.q[k * 18 + ib - 1] < 0.5f ? R.near : R.far) |= 1u << (j - 1);
+        }
+        if (k >= L.off[2]) {
+          R.near |= (uint32_t)side_iolet(h, k) << 18;
+          R.ii = (uint32_t)iolIndex[k];
+        }
+        for (int d = 0; d < 18; ++d) q[(size_t)d * SB + b] = L.q[k * 18 + d];
+        for (int a = 0; a < 3; ++a) nr[(size_t)a * SB + b] = L.nrm[k * 3 + a];
       }
-      if (k >= L.off[2]) {
-        R.near |= (uint32_t)side_iolet(h, k) << 18;
-        R.ii = (uint32_t)iolIndex[k];
-      }
-      for (int d = 0; d < 18; ++d) q[(size_t)d * SB + b] = L.q[k * 18 + d];
-      for (int a = 0; a < 3; ++a) nr[(size_t)a * SB + b] = L.nrm[k * 3 + a];
-    }
-    HLB_CHECK(hipMemcpy(h->bnd.p, rec.data(), sizeof(BndRec) * SB, hipMemcpyHostToDevice));
-    HLB_CHECK(hipMemcpy(h->bq.p, q.data(), sizeof(float) * q.size(), hipMemcpyHostToDevice));
-    HLB_CHECK(hipMemcpy(h->bnrm.p, nr.data(), sizeof(float) * nr.size(), hipMemcpyHostToDevice));
+    });
   }
-  HLB_CHECK(hipMemcpy(h->ladd_s.p, h->h_ladd_s.data(), sizeof(double) * h->h_ladd_s.size(),
-                      hipMemcpyHostToDevice));
-  // Per-iolet constants and the staging for per-step values.
+  pack.add(h->bnd, rec);
+  pack.add(h->bq, q);
+  pack.add(h->bnrm, nr);
+  pack.add(h->ladd_s, h->h_ladd_s);
+  // Per-iolet constants and what the per-step values are copied to.
   {
     const int nio = h->iolet_count();
     std::vector<float> nf((size_t)3 * nio, 0.0f);
@@ -633,37 +654,30 @@ int upload_lattice(hlb_lattice* h) {
         nf[3 * g + a] = h->iolets[g].nf[a];
         nd[3 * g + a] = h->iolets[g].n[a];
       }
-    HLB_CHECK(h->io_nf.alloc(nf.size()));
-    HLB_CHECK(h->io_n.alloc(nd.size()));
-    const size_t staged = (size_t)(kStageHead + kChunk * h->row());
-    HLB_CHECK(h->stage.alloc(staged));
-    HLB_CHECK(hipMemcpy(h->io_nf.p, nf.data(), sizeof(float) * nf.size(), hipMemcpyHostToDevice));
-    HLB_CHECK(hipMemcpy(h->io_n.p, nd.data(), sizeof(double) * nd.size(), hipMemcpyHostToDevice));
-    HLB_CHECK(hipHostMalloc((void**)&h->h_stage, sizeof(double) * staged, hipHostMallocDefault));
     std::vector<uint32_t> bits(nio, 0u);
     for (size_t g = 0; g < h->iolets.size(); ++g)
       if (h->iolets[g].IsWK() && h->iolets[g].dirs0 != 0) bits[g] = 1u << (INV[h->iolets[g].dirs0] - 1);
-    HLB_CHECK(h->wk_bit.alloc(nio));
-    HLB_CHECK(hipMemcpy(h->wk_bit.p, bits.data(), sizeof(uint32_t) * nio, hipMemcpyHostToDevice));
-    HLB_CHECK(h->wk.alloc(h->wk_host.size()));
-    HLB_CHECK(hipMemcpy(h->wk.p, h->wk_host.data(), sizeof(WkIolet) * h->wk_host.size(), hipMemcpyHostToDevice));
-    // the coupling terms, written by the step in the coupling order
-    const size_t ncoup = 2 * (size_t)h->wk_stride();
-    HLB_CHECK(h->wk_contrib.alloc(ncoup));
-    HLB_CHECK(hipMemsetAsync(h->wk_contrib.p, 0, sizeof(double) * ncoup, h->stream));
     std::vector<int32_t> pos((size_t)std::max<int64_t>(1, SI), -1);
     for (size_t e = 0; e < h->wk_list.size(); ++e) pos[(size_t)h->wk_list[e]] = (int32_t)e;
-    HLB_CHECK(h->wk_pos.alloc(pos.size()));
-    HLB_CHECK(hipMemcpy(h->wk_pos.p, pos.data(), sizeof(int32_t) * pos.size(), hipMemcpyHostToDevice));
+    pack.add(h->io_nf, nf);
+    pack.add(h->io_n, nd);
+    pack.add(h->stage, (const double*)nullptr, (size_t)h->stage_doubles());
+    pack.add(h->wk_bit, bits);
+    pack.add(h->wk, h->wk_host);
+    // the coupling terms, written by the step in the coupling order
+    pack.add(h->wk_contrib, (const double*)nullptr, 2 * (size_t)h->wk_stride());
+    pack.add(h->wk_pos, pos);
+    HLB_CHECK(pack.commit(h->arena, h->stream));
     h->wk_refs_host.clear();
     for (size_t g = 0; g < h->iolets.size(); ++g)
       if (h->iolets[g].IsWK())
-        h->wk_refs_host.push_back(WkRef{h->wk.p + g, h->rows(), h->wk_contrib.p, h->wk_stride(), (int32_t)g, (int32_t)h->row(),
-                                        h->fp32() ? 0 : 1, 0});
-    HLB_CHECK(h->wk_refs.alloc(std::max<size_t>(1, h->wk_refs_host.size())));
-    if (!h->wk_refs_host.empty())
+        h->wk_refs_host.push_back(WkRef{h->wk.p + g, h->rows(), h->wk_contrib.p, h->wk_stride(), (int32_t)g,
+                                        (int32_t)h->row(), h->fp32() ? 0 : 1, 0});
+    if (!h->wk_refs_host.empty()) {
+      HLB_CHECK(h->wk_refs.alloc(h->wk_refs_host.size()));
       HLB_CHECK(hipMemcpy(h->wk_refs.p, h->wk_refs_host.data(), sizeof(WkRef) * h->wk_refs_host.size(),
                           hipMemcpyHostToDevice));
+    }
   }
   {
     const int rc = upload_sponge(h);
@@ -694,12 +708,18 @@ int ensure_device(hlb_lattice* h) {
     const char* force = std::getenv("HLB_FP64_GENERAL_GATHER");
     h->general_gather = force && force[0] == '1';
   }
-  HLB_CHECK(hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking));
-  HLB_CHECK(hipEventCreate(&h->ev0));
-  HLB_CHECK(hipEventCreate(&h->ev1));
-  int rc = upload_lattice(h);
-  if (rc == HLB_OK) rc = transfer_open(h);
+  int rc = HLB_OK;
+  if (!h->stream) {
+    rc = take_lane(h->device, (size_t)h->stage_doubles(), h->lane);
+    if (rc != HLB_OK) return rc;
+    h->stream = h->lane.stream;
+    h->ev0 = h->lane.ev0;
+    h->ev1 = h->lane.ev1;
+    h->h_stage = h->lane.stage;
+  }
+  rc = upload_lattice(h);
   if (rc != HLB_OK) return rc;
+  transfer_open();
   h->device_ready = true;
   return HLB_OK;
 }
@@ -1522,7 +1542,7 @@ extern "C" int hlb_neighbour_tables(hlb_handle h, int64_t* push, uint32_t* pull)
   if (!h) return fail(HLB_EINVAL, "hlb_neighbour_tables: null handle");
   if (push) push_table(h->L, push);
   if (pull && !h->device_ready) {
-    std::memcpy(pull, h->L.pull.data(), sizeof(uint32_t) * h->L.pull.size());
+    pull_table(h->L, pull);
   } else if (pull) {
     // The slots the device kernels gather from, computed by the same code
     // on the device, expressed in the reference's order (a padding slot reads as

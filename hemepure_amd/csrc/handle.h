@@ -79,21 +79,65 @@ template <typename T>
 struct DevBuf {
   T* p = nullptr;
   size_t n = 0;
+  bool owned = true;  // false: a part of another allocation
   DevBuf() = default;
   DevBuf(const DevBuf&) = delete;
   DevBuf& operator=(const DevBuf&) = delete;
-  ~DevBuf() {
-    if (p) (void)hipFree(p);
+  ~DevBuf() { release(); }
+  void release() {
+    if (p && owned) (void)hipFree(p);
+    p = nullptr;
+    owned = true;
   }
   hipError_t alloc(size_t count) {
-    if (p) {
-      (void)hipFree(p);
-      p = nullptr;
-    }
+    release();
     n = count;
     if (count == 0) return hipSuccess;
     return hipMalloc(&p, sizeof(T) * count);
   }
+  void view(void* part, size_t count) {
+    release();
+    p = static_cast<T*>(part);
+    n = count;
+    owned = false;
+  }
+};
+
+// Device arrays made together: those up to kPackBytes are laid out in one
+// allocation and filled with one copy (an allocation costs ~11 us, its release
+// ~29 us and a blocking copy ~46 us whatever their size), larger ones get their
+// own.  add() keeps a pointer to `data` (null: zeros) until commit().
+class DevPack {
+ public:
+  template <typename T>
+  void add(DevBuf<T>& buf, const T* data, size_t count) {
+    items_.push_back({&buf, data, sizeof(T), count, [](void* b, void* part, size_t n) {
+                        auto* d = static_cast<DevBuf<T>*>(b);
+                        if (part) {
+                          d->view(part, n);
+                          return hipSuccess;
+                        }
+                        return d->alloc(n);
+                      },
+                      [](void* b) { return (void*)static_cast<DevBuf<T>*>(b)->p; }});
+  }
+  template <typename T>
+  void add(DevBuf<T>& buf, const std::vector<T>& data) {
+    add(buf, data.data(), data.size());
+  }
+  // Allocates and fills everything (zeros asynchronously on s).
+  hipError_t commit(DevBuf<char>& arena, hipStream_t s);
+
+ private:
+  static constexpr size_t kPackBytes = size_t(1) << 20, kAlign = 256;
+  struct Item {
+    void* buf;
+    const void* data;
+    size_t size, count;
+    hipError_t (*place)(void*, void*, size_t);
+    void* (*where)(void*);
+  };
+  std::vector<Item> items_;
 };
 
 inline int dev_fail(hipError_t e, const char* what) {
@@ -109,11 +153,13 @@ inline int dev_fail(hipError_t e, const char* what) {
 }  // namespace hlb
 
 struct hlb_lattice {
+  hlb::DevBuf<char> arena, fields_mem, a_mem;  // what the arrays below are parts of
   hlb::HostLattice L;
   hlb_params params{};
   std::vector<hlb::HostIolet> iolets;  // inlets then outlets
   int n_in = 0, n_out = 0;
   int device = 0;
+  hlb::HostLane lane;  // the stream, events and pinned staging below
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   // Device slots (compact slab layout): perm[slot] = reference index or -1
@@ -177,6 +223,7 @@ struct hlb_lattice {
   double* h_stage = nullptr;
   int iolet_count() const { return iolets.empty() ? 1 : (int)iolets.size(); }
   int64_t row() const { return 3 * (int64_t)iolet_count() + 1; }
+  int64_t stage_doubles() const { return hlb::kStageHead + hlb::kChunk * row(); }
   double* rows() const { return stage.p + hlb::kStageHead; }
   // Pinned doubles the monitors' kernels write their results to.
   double* result() const { return h_stage + hlb::kStageResult; }
@@ -217,11 +264,8 @@ struct hlb_lattice {
     if (stream) {
       (void)hipStreamSynchronize(stream);
       drop_graphs();
-      (void)hipStreamDestroy(stream);
     }
-    if (ev0) (void)hipEventDestroy(ev0);
-    if (ev1) (void)hipEventDestroy(ev1);
-    if (h_stage) (void)hipHostFree(h_stage);
+    hlb::give_lane(lane);
     if (device_ready) hlb::transfer_close();
   }
   bool fp32() const { return params.precision == HLB_FP32_SHIFTED; }

@@ -17,9 +17,11 @@
 // writers and are rejected.
 #include "lattice.h"
 
+#include <atomic>
 #include <cmath>
 #include <limits>
 #include <string>
+#include <unordered_set>
 
 #include "d3q19.h"
 #include "errors.h"
@@ -54,6 +56,49 @@ void normalise_float(float v[3]) {
   v[2] /= mag;
 }
 
+// The first inconsistent record, in input order, of a geometry known to hold
+// one.
+int site_map_error(const hlb_geometry& g) {
+  const int64_t SX = (int64_t)g.blocks[0] * g.block_size, SY = (int64_t)g.blocks[1] * g.block_size,
+                SZ = (int64_t)g.blocks[2] * g.block_size;
+  std::unordered_set<int64_t> seen;
+  for (int64_t i = 0; i < g.n_sites; ++i) {
+    const int64_t x = g.coords[3 * i], y = g.coords[3 * i + 1], z = g.coords[3 * i + 2];
+    if (x < 0 || y < 0 || z < 0 || x >= SX || y >= SY || z >= SZ)
+      return fail(HLB_EGEOMETRY, "hlb_create: site outside the block grid");
+    if (!seen.insert((x * SY + y) * SZ + z).second) return fail(HLB_EGEOMETRY, "hlb_create: duplicate fluid site");
+  }
+  return HLB_OK;
+}
+
+// The link type of contiguous site k in direction d (1..18).
+uint8_t link_of(const HostLattice& L, int64_t k, int d) {
+  if ((L.wall[k] >> (d - 1)) & 1u) return HLB_LINK_WALL;
+  if ((L.iolet[k] >> (d - 1)) & 1u) return HLB_LINK_INLET;
+  return HLB_LINK_NONE;
+}
+
+// The lowest site (and its lowest direction) of a lattice known to hold a
+// distribution with no writer or two.
+int one_writer_error(const HostLattice& L) {
+  for (int64_t k = 0; k < L.N; ++k) {
+    const int64_t x = L.coords[3 * k], y = L.coords[3 * k + 1], z = L.coords[3 * k + 2];
+    for (int j = 1; j < Q; ++j) {
+      const int ib = INV[j];
+      const int64_t src = L.site_at(x - CX[j], y - CY[j], z - CZ[j]);
+      const bool plain = link_of(L, k, ib) == HLB_LINK_NONE;
+      const bool srcPushes = src >= 0 && link_of(L, src, j) == HLB_LINK_NONE;
+      if (plain != srcPushes)
+        return fail(HLB_EGEOMETRY, "hlb_create: link type disagrees with neighbour fluidity at site (" +
+                                       std::to_string(x) + "," + std::to_string(y) + "," + std::to_string(z) +
+                                       ") direction " + std::to_string(ib) +
+                                       " (the push step would write that distribution " + (plain ? "zero" : "two") +
+                                       " times)");
+    }
+  }
+  return HLB_OK;
+}
+
 }  // namespace
 
 int build_lattice(const hlb_geometry& g, HostLattice& L) {
@@ -72,145 +117,209 @@ int build_lattice(const hlb_geometry& g, HostLattice& L) {
   const int64_t SX = BX * bs, SY = BY * bs, SZ = BZ * bs;
   const int64_t n = g.n_sites;
 
-  // Site map over the input records.
-  L.blockSlot.assign(BX * BY * BZ, -1);
-  std::vector<int64_t> slotInput;
-  for (int64_t i = 0; i < n; ++i) {
-    const int64_t x = g.coords[3 * i], y = g.coords[3 * i + 1], z = g.coords[3 * i + 2];
-    if (x < 0 || y < 0 || z < 0 || x >= SX || y >= SY || z >= SZ)
-      return fail(HLB_EGEOMETRY, "hlb_create: site outside the block grid");
-    const int64_t b = ((x / bs) * BY + (y / bs)) * BZ + (z / bs);
-    if (L.blockSlot[b] < 0) {
-      L.blockSlot[b] = (int64_t)(slotInput.size() / spb);
-      slotInput.resize(slotInput.size() + spb, -1);
+  // Site map over the input records: the occupied blocks, numbered in block
+  // order, then each record's cell in its block.
+  std::atomic<bool> bad{false};
+  L.blockSlot.assign((size_t)(BX * BY * BZ), -1);
+  parallel_ranges(n, [&](int, int64_t lo, int64_t hi) {
+    for (int64_t i = lo; i < hi; ++i) {
+      const int32_t x = g.coords[3 * i], y = g.coords[3 * i + 1], z = g.coords[3 * i + 2];
+      if (x < 0 || y < 0 || z < 0 || x >= SX || y >= SY || z >= SZ) {
+        bad.store(true, std::memory_order_relaxed);
+        return;
+      }
+      int64_t& slot = L.blockSlot[(size_t)(((x / (int32_t)bs) * BY + (y / (int32_t)bs)) * BZ + (z / (int32_t)bs))];
+      if (__atomic_load_n(&slot, __ATOMIC_RELAXED) != 0) __atomic_store_n(&slot, int64_t(0), __ATOMIC_RELAXED);
     }
-    int64_t& cell = slotInput[L.blockSlot[b] * spb + (((x % bs) * bs) + (y % bs)) * bs + (z % bs)];
-    if (cell >= 0) return fail(HLB_EGEOMETRY, "hlb_create: duplicate fluid site");
-    cell = i;
-  }
+  });
+  if (bad.load()) return site_map_error(g);
+  std::vector<int64_t> slotBlock;
+  for (int64_t b = 0; b < BX * BY * BZ; ++b)
+    if (L.blockSlot[(size_t)b] == 0) {
+      L.blockSlot[(size_t)b] = (int64_t)slotBlock.size();
+      slotBlock.push_back(b);
+    }
+  const int64_t nslot = (int64_t)slotBlock.size();
+  const int64_t slotGrain = std::max<int64_t>(1, kGrain / spb);
+  RawVector<int32_t> cellInput;
+  cellInput.resize((size_t)(nslot * spb));
+  parallel_ranges(nslot, [&](int, int64_t lo, int64_t hi) {
+    std::fill(cellInput.begin() + lo * spb, cellInput.begin() + hi * spb, -1);
+  }, slotGrain);
+  parallel_ranges(n, [&](int, int64_t lo, int64_t hi) {
+    const int32_t b = (int32_t)bs;
+    for (int64_t i = lo; i < hi; ++i) {
+      const int32_t x = g.coords[3 * i], y = g.coords[3 * i + 1], z = g.coords[3 * i + 2];
+      const int64_t slot = L.blockSlot[(size_t)(((x / b) * BY + (y / b)) * BZ + (z / b))];
+      int32_t* cell = &cellInput[(size_t)(slot * spb + (((x % b) * b) + (y % b)) * b + (z % b))];
+      if (__atomic_exchange_n(cell, (int32_t)i, __ATOMIC_RELAXED) >= 0) {
+        bad.store(true, std::memory_order_relaxed);
+        return;
+      }
+    }
+  });
+  if (bad.load()) return site_map_error(g);
 
   // Classification of every input record.
-  std::vector<uint32_t> wall(n, 0), iol(n, 0);
-  std::vector<int32_t> ioletId(n, -1), type(n, kFluidType);
-  std::vector<uint8_t> cls(n, 0);
-  std::vector<uint8_t> badLink((size_t)host_workers(n), 0);
-  parallel_ranges(n, [&](int w, int64_t lo, int64_t hi) {
+  RawVector<uint32_t> wall, iol;
+  RawVector<int32_t> ioletId, type;
+  RawVector<uint8_t> cls;
+  wall.resize((size_t)n);
+  iol.resize((size_t)n);
+  ioletId.resize((size_t)n);
+  type.resize((size_t)n);
+  cls.resize((size_t)n);
+  parallel_ranges(n, [&](int, int64_t lo, int64_t hi) {
     for (int64_t i = lo; i < hi; ++i) {
       bool hadInlet = false, hadOutlet = false;
+      uint32_t w = 0, io = 0;
+      int32_t id = -1;
       for (int d = 1; d < Q; ++d) {
         const uint8_t t = g.link_type[i * 18 + d - 1];
+        if (t == HLB_LINK_NONE) continue;
         if (t > HLB_LINK_OUTLET) {
-          badLink[(size_t)w] = 1;
+          bad.store(true, std::memory_order_relaxed);
           return;
         }
-        if (t == HLB_LINK_WALL) wall[i] |= 1u << (d - 1);
-        else if (t == HLB_LINK_INLET || t == HLB_LINK_OUTLET) iol[i] |= 1u << (d - 1);
-        if (t == HLB_LINK_INLET) {
-          ioletId[i] = g.link_iolet[i * 18 + d - 1];
-          hadInlet = true;
-        } else if (t == HLB_LINK_OUTLET) {
-          ioletId[i] = g.link_iolet[i * 18 + d - 1];
-          hadOutlet = true;
+        if (t == HLB_LINK_WALL) {
+          w |= 1u << (d - 1);
+          continue;
         }
+        io |= 1u << (d - 1);
+        id = g.link_iolet[i * 18 + d - 1];
+        (t == HLB_LINK_INLET ? hadInlet : hadOutlet) = true;
       }
+      wall[i] = w;
+      iol[i] = io;
+      ioletId[i] = id;
       type[i] = hadInlet ? kInletType : (hadOutlet ? kOutletType : kFluidType);
-      const bool wl = wall[i] != 0;
+      const bool wl = w != 0;
       cls[i] = type[i] == kFluidType ? (wl ? 1 : 0) : type[i] == kInletType ? (wl ? 4 : 2) : (wl ? 5 : 3);
     }
   });
-  for (uint8_t b : badLink)
-    if (b) return fail(HLB_EGEOMETRY, "hlb_create: unknown link type");
+  if (bad.load()) return fail(HLB_EGEOMETRY, "hlb_create: unknown link type");
 
-  // Class-major contiguous order.
-  int64_t count[6] = {0, 0, 0, 0, 0, 0};
-  for (int64_t i = 0; i < n; ++i) count[cls[i]]++;
-  L.off[0] = 0;
-  for (int c = 0; c < 6; ++c) L.off[c + 1] = L.off[c] + count[c];
+  // Class-major contiguous order: per block and class the first index, then
+  // every cell's.  cellLinks: a cell's wall and iolet links, bit 31 where it is
+  // fluid.
+  constexpr uint32_t kFluid = 1u << 31;
+  std::vector<int64_t> next((size_t)nslot * 6, 0);
+  parallel_ranges(nslot, [&](int, int64_t lo, int64_t hi) {
+    for (int64_t s = lo; s < hi; ++s)
+      for (int64_t c = s * spb; c < (s + 1) * spb; ++c)
+        if (cellInput[(size_t)c] >= 0) next[(size_t)(s * 6 + cls[(size_t)cellInput[(size_t)c]])]++;
+  }, slotGrain);
   L.N = n;
-  int64_t next[6];
-  for (int c = 0; c < 6; ++c) next[c] = L.off[c];
-  std::vector<int64_t> contigOf(n, -1);
-  L.slotSites.assign(slotInput.size(), -1);
-  for (int64_t b = 0; b < BX * BY * BZ; ++b) {
-    const int64_t slot = L.blockSlot[b];
-    if (slot < 0) continue;
-    for (int64_t s = 0; s < spb; ++s) {
-      const int64_t i = slotInput[slot * spb + s];
-      if (i < 0) continue;
-      const int64_t k = next[cls[i]]++;
-      contigOf[i] = k;
-      L.slotSites[slot * spb + s] = (int32_t)k;
+  int64_t k = 0;
+  for (int c = 0; c < 6; ++c) {
+    L.off[c] = k;
+    for (int64_t s = 0; s < nslot; ++s) {
+      const int64_t count = next[(size_t)(s * 6 + c)];
+      next[(size_t)(s * 6 + c)] = k;
+      k += count;
     }
   }
-
-  L.coords.assign(n * 3, 0);
-  L.wall.assign(n, 0);
-  L.iolet.assign(n, 0);
-  L.ioletId.assign(n, -1);
-  L.siteType.assign(n, kFluidType);
-  L.q.assign(n * 18, -1.0f);
-  L.nrm.assign(n * 3, 0.0f);
-  parallel_ranges(n, [&](int, int64_t lo, int64_t hi) {
-    for (int64_t i = lo; i < hi; ++i) {
-      const int64_t k = contigOf[i];
-      for (int a = 0; a < 3; ++a) L.coords[3 * k + a] = g.coords[3 * i + a];
-      L.wall[k] = wall[i];
-      L.iolet[k] = iol[i];
-      L.ioletId[k] = ioletId[i];
-      L.siteType[k] = type[i];
-      for (int d = 0; d < 18; ++d) L.q[k * 18 + d] = g.link_dist[i * 18 + d];
-      float v[3];
-      if (g.normal_avail[i]) {
-        for (int a = 0; a < 3; ++a) v[a] = g.normal[3 * i + a];
-        normalise_float(v);
-      } else {
-        v[0] = v[1] = v[2] = std::numeric_limits<float>::infinity();  // float(NO_VALUE)
+  L.off[6] = k;
+  RawVector<uint32_t> cellLinks;
+  cellLinks.resize((size_t)(nslot * spb));
+  L.slotSites.resize((size_t)(nslot * spb));
+  L.coords.resize((size_t)n * 3);
+  L.wall.resize((size_t)n);
+  L.iolet.resize((size_t)n);
+  L.ioletId.resize((size_t)n);
+  L.siteType.resize((size_t)n);
+  L.q.resize((size_t)n * 18);
+  L.nrm.resize((size_t)n * 3);
+  parallel_ranges(nslot, [&](int, int64_t lo, int64_t hi) {
+    for (int64_t s = lo; s < hi; ++s)
+      for (int64_t c = s * spb; c < (s + 1) * spb; ++c) {
+        const int64_t i = cellInput[(size_t)c];
+        if (i < 0) {
+          L.slotSites[(size_t)c] = -1;
+          cellLinks[(size_t)c] = 0;
+          continue;
+        }
+        const int64_t to = next[(size_t)(s * 6 + cls[(size_t)i])]++;
+        L.slotSites[(size_t)c] = (int32_t)to;
+        cellLinks[(size_t)c] = wall[(size_t)i] | iol[(size_t)i] | kFluid;
+        for (int a = 0; a < 3; ++a) L.coords[(size_t)(3 * to + a)] = g.coords[3 * i + a];
+        L.wall[(size_t)to] = wall[(size_t)i];
+        L.iolet[(size_t)to] = iol[(size_t)i];
+        L.ioletId[(size_t)to] = ioletId[(size_t)i];
+        L.siteType[(size_t)to] = type[(size_t)i];
+        for (int d = 0; d < 18; ++d) L.q[(size_t)(to * 18 + d)] = g.link_dist[i * 18 + d];
+        float v[3];
+        if (g.normal_avail[i]) {
+          for (int a = 0; a < 3; ++a) v[a] = g.normal[3 * i + a];
+          normalise_float(v);
+        } else {
+          v[0] = v[1] = v[2] = std::numeric_limits<float>::infinity();  // float(NO_VALUE)
+        }
+        for (int a = 0; a < 3; ++a) L.nrm[(size_t)(3 * to + a)] = v[a];
       }
-      for (int a = 0; a < 3; ++a) L.nrm[3 * k + a] = v[a];
-    }
-  });
+  }, slotGrain);
 
-  // Pull table and the one-writer check.  Each worker stops at its first
-  // inconsistent (site, direction); the error names the lowest such site.
-  L.pull.assign((size_t)18 * n, 0);
-  auto linkOf = [&](int64_t k, int d) -> uint8_t {
-    // link type of contiguous site k in direction d (1..18)
-    if ((L.wall[k] >> (d - 1)) & 1u) return HLB_LINK_WALL;
-    if ((L.iolet[k] >> (d - 1)) & 1u) return HLB_LINK_INLET;
-    return HLB_LINK_NONE;
-  };
-  struct Bad {
-    int64_t k = -1;
-    int ib = 0;
-    bool plain = false;
-  };
-  std::vector<Bad> bad((size_t)host_workers(n));
-  parallel_ranges(n, [&](int w, int64_t lo, int64_t hi) {
+  // The one-writer check, cell by cell: a plain link's neighbour must be
+  // fluid with a plain link back, any other link's must not push here.
+  parallel_ranges(nslot, [&](int, int64_t lo, int64_t hi) {
+    for (int64_t s = lo; s < hi; ++s) {
+      const int64_t b = slotBlock[(size_t)s], bx = b / (BY * BZ), by = (b / BZ) % BY, bz = b % BZ;
+      const uint32_t* around[27];  // the 3 x 3 x 3 blocks' cells
+      for (int e = 0; e < 27; ++e) {
+        const int64_t x = bx + e / 9 - 1, y = by + (e / 3) % 3 - 1, z = bz + e % 3 - 1;
+        const bool in = x >= 0 && y >= 0 && z >= 0 && x < BX && y < BY && z < BZ;
+        const int64_t t = in ? L.blockSlot[(size_t)((x * BY + y) * BZ + z)] : -1;
+        around[e] = t < 0 ? nullptr : &cellLinks[(size_t)(t * spb)];
+      }
+      const uint32_t* own = around[13];
+      for (int64_t c = 0; c < spb; ++c) {
+        const uint32_t here = own[c];
+        if (!(here & kFluid)) continue;
+        const int64_t x = c / (bs * bs), y = (c / bs) % bs, z = c % bs;
+        const bool inner = x > 0 && y > 0 && z > 0 && x < bs - 1 && y < bs - 1 && z < bs - 1;
+        for (int j = 1; j < Q; ++j) {
+          uint32_t src = 0;
+          if (inner) {
+            src = own[c - ((CX[j] * bs + CY[j]) * bs + CZ[j])];
+          } else {
+            int64_t p[3] = {x - CX[j], y - CY[j], z - CZ[j]};
+            int e = 13;
+            const int step[3] = {9, 3, 1};
+            for (int a = 0; a < 3; ++a) {
+              if (p[a] < 0) {
+                p[a] += bs;
+                e -= step[a];
+              } else if (p[a] >= bs) {
+                p[a] -= bs;
+                e += step[a];
+              }
+            }
+            if (around[e]) src = around[e][(p[0] * bs + p[1]) * bs + p[2]];
+          }
+          const bool plain = !((here >> (INV[j] - 1)) & 1u);
+          const bool srcPushes = (src & kFluid) && !((src >> (j - 1)) & 1u);
+          if (plain != srcPushes) {
+            bad.store(true, std::memory_order_relaxed);
+            return;
+          }
+        }
+      }
+    }
+  }, slotGrain);
+  return bad.load() ? one_writer_error(L) : HLB_OK;
+}
+
+void pull_table(const HostLattice& L, uint32_t* out) {
+  const int64_t n = L.N;
+  parallel_ranges(n, [&](int, int64_t lo, int64_t hi) {
     for (int64_t k = lo; k < hi; ++k) {
       const int64_t x = L.coords[3 * k], y = L.coords[3 * k + 1], z = L.coords[3 * k + 2];
       for (int j = 1; j < Q; ++j) {
-        const int ib = INV[j];
-        const int64_t src = L.site_at(x - CX[j], y - CY[j], z - CZ[j]);
-        const bool plain = linkOf(k, ib) == HLB_LINK_NONE;
-        const bool srcPushes = src >= 0 && linkOf(src, j) == HLB_LINK_NONE;
-        if (plain != srcPushes) {
-          bad[(size_t)w] = Bad{k, ib, plain};
-          return;
-        }
-        L.pull[(size_t)(j - 1) * n + k] = (uint32_t)(plain ? src : k);
+        const bool plain = link_of(L, k, INV[j]) == HLB_LINK_NONE;
+        out[(size_t)(j - 1) * n + k] = (uint32_t)(plain ? L.site_at(x - CX[j], y - CY[j], z - CZ[j]) : k);
       }
     }
   });
-  for (const Bad& b : bad)
-    if (b.k >= 0) {
-      const int64_t x = L.coords[3 * b.k], y = L.coords[3 * b.k + 1], z = L.coords[3 * b.k + 2];
-      return fail(HLB_EGEOMETRY, "hlb_create: link type disagrees with neighbour fluidity at site (" +
-                                     std::to_string(x) + "," + std::to_string(y) + "," + std::to_string(z) +
-                                     ") direction " + std::to_string(b.ib) +
-                                     " (the push step would write that distribution " +
-                                     (b.plain ? "zero" : "two") + " times)");
-    }
-  return HLB_OK;
 }
 
 void push_table(const HostLattice& L, int64_t* out) {

@@ -57,7 +57,7 @@ struct Request {
   double t_submit = 0, t_admit = -1, t_done = -1;
   float* prev = nullptr;  // device snapshot of u at the last cycle end (3 planes of S)
   int bypassed = 0;       // later requests admitted while this one waited at the head
-  std::vector<double> rho, u, wss;
+  RawVector<double> rho, u, wss;  // filled when the request is retired
   std::string error;
 };
 
@@ -81,6 +81,7 @@ struct hlb_server {
   unsigned* d_delta = nullptr;
   std::chrono::steady_clock::time_point t0 = std::chrono::steady_clock::now();
 
+  hlb_server() { hlb::transfer_open(); }
   double now() const {
     return std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
   }
@@ -91,6 +92,7 @@ struct hlb_server {
     }
     if (batch) hlb_batch_destroy(batch);
     if (d_delta) (void)hipFree(d_delta);
+    hlb::transfer_close();
   }
 };
 

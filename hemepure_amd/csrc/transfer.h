@@ -2,6 +2,9 @@
 // site records (the reference's site order).
 #pragma once
 
+#include <hip/hip_runtime.h>
+
+#include <cstddef>
 #include <cstdint>
 
 struct hlb_lattice;
@@ -18,9 +21,22 @@ struct TransferPart {
   double* host;
 };
 
-// The device copy of the site -> slot index and the handle's share of the
-// pinned chunks; closed once when the handle goes.
-int transfer_open(hlb_lattice* h);
+// A stream with two timing events and pinned staging, which a lattice has from
+// its first use to its end.  Making one costs ~0.6 ms and dropping it ~0.4 ms,
+// so idle ones are kept (up to kIdleLanes, none once no user is left).
+struct HostLane {
+  hipStream_t stream = nullptr;
+  hipEvent_t ev0 = nullptr, ev1 = nullptr;
+  double* stage = nullptr;  // pinned
+  size_t doubles = 0;
+  int device = -1;
+};
+int take_lane(int device, size_t doubles, HostLane& out);
+void give_lane(HostLane& lane);  // the stream is idle
+
+// A user of the pinned chunks and lanes (a lattice with a device state, a
+// server, whose lattices come and go); closed once when it goes.
+void transfer_open();
 void transfer_close();
 
 // Both follow the work queued on the handle's stream and return when the host
