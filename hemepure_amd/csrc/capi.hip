@@ -228,6 +228,23 @@ int side_iolet(const hlb_lattice* h, int64_t k) {
 // fast or faster there.
 constexpr int64_t kL2WindowSlabs = 431;
 
+// Why sections: in XCD order each XCD takes one eighth of the slabs.  In tile
+// order (x slowest) the eighths of a vessel that runs along z or y are slices
+// along it: those at its sides are mostly boundary slabs, which take about
+// twice as long, and the XCDs in the middle wait.  AUTO therefore enumerates
+// such a vessel in sections of kSectionBricks bricks along its longest axis,
+// tile order within, where XCD order is what a lattice is launched in and its
+// steps are long enough for it to show: distributions between a quarter of the
+// Infinity Cache and all of it.  Measured on MI355X, tile order / sections: the
+// 0.70M-site Y-bifurcation (z) FP64 44.9 / 41.6-42.1 us, FP32 27.0 / 25.8-26.1;
+// beyond the cache nothing or a loss (3.0M-site tree 206.6 / 206.5, 1.9M-site
+// pipe 119.0 / 119.2, 20-pipe ensemble 67.7 / 69.7).
+constexpr int64_t kSectionBricks = 8;
+bool sections_pay(int64_t sites, bool fp32) {
+  const int64_t bytes = distribution_bytes(sites, fp32);
+  return bytes > kInfinityCacheBytes / 4 && bytes <= kInfinityCacheBytes;
+}
+
 void device_order(hlb_lattice* h, int order) {
   const HostLattice& L = h->L;
   const int64_t N = L.N;
@@ -243,10 +260,24 @@ void device_order(hlb_lattice* h, int order) {
   });
   std::vector<int64_t> brickTile;
   for (size_t t = 0; t < brickOf.size(); ++t)
-    if (brickOf[t] >= 0) {
-      brickOf[t] = (int32_t)brickTile.size();
-      brickTile.push_back((int64_t)t);
-    }
+    if (brickOf[t] >= 0) brickTile.push_back((int64_t)t);
+  if (order == HLB_ORDER_AUTO && sections_pay(N, h->params.precision == HLB_FP32_SHIFTED)) {
+    int64_t lo[3] = {ntx, nty, ntz}, hi[3] = {-1, -1, -1};
+    auto axis_of = [&](int64_t t, int a) { return a == 0 ? t / (nty * ntz) : a == 1 ? (t / ntz) % nty : t % ntz; };
+    for (const int64_t t : brickTile)
+      for (int a = 0; a < 3; ++a) {
+        lo[a] = std::min(lo[a], axis_of(t, a));
+        hi[a] = std::max(hi[a], axis_of(t, a));
+      }
+    int along = 0;
+    for (int a = 1; a < 3; ++a)
+      if (hi[a] - lo[a] > hi[along] - lo[along]) along = a;
+    if (along != 0)
+      std::stable_sort(brickTile.begin(), brickTile.end(), [&](int64_t s, int64_t t) {
+        return axis_of(s, along) / kSectionBricks < axis_of(t, along) / kSectionBricks;
+      });
+  }
+  for (size_t i = 0; i < brickTile.size(); ++i) brickOf[(size_t)brickTile[i]] = (int32_t)i;
   const int64_t NBr = (int64_t)brickTile.size();
   h->nbrick = NBr;
   constexpr int64_t kBrickGrain = kGrain / kBrickSites;
@@ -1168,6 +1199,7 @@ extern "C" int hlb_create(const hlb_geometry* geom, const hlb_params* params, co
     auto h = std::make_unique<hlb_lattice>();
     rc = build_lattice(*geom, h->L);
     if (rc != HLB_OK) return rc;
+    h->params.precision = p.precision;  // the automatic order goes by the size of the distributions
     device_order(h.get(), p.slab_order);
     if (h->S > (int64_t(1) << 29))
       return fail(HLB_EINVAL, "hlb_create: the geometry needs " + std::to_string(h->S) +

@@ -70,7 +70,9 @@ extern "C" {
  * launch order each XCD then walks one layer, and a slab's y neighbours,
  * which share the cache lines of its face lanes, come within its L2 window.
  * AUTO (0): LAYER when the median distance from a slab to its y neighbour in
- * TILE order exceeds that window (431 slabs), else TILE.  No effect on
+ * TILE order exceeds that window (431 slabs), else TILE; lattices whose
+ * distributions take 64 to 256 MB and run along y or z enumerate their tiles in
+ * sections of 8 tiles along that axis first.  No effect on
  * results; hlb_get_params reports the order chosen. */
 #define HLB_ORDER_AUTO 0
 #define HLB_ORDER_TILE 1
