@@ -163,7 +163,7 @@ __device__ __forceinline__ void gather_site32(const float* in, int64_t S, const 
 
 // The boundary delegates of one gathered site, as boundary_fixup in the FP64
 // pass (SimpleBounceBackDelegate.h:36-44, BouzidiFirdaousLallemandDelegate.h:
-// 44-93, iolet values from G).
+// 44-93).
 __device__ __forceinline__ void boundary_fixup32(const Member32& m, const float* in, uint32_t d, uint32_t b,
                                                  const Bnd& r, float* g) {
   float q[Q], own[Q];
@@ -175,10 +175,11 @@ __device__ __forceinline__ void boundary_fixup32(const Member32& m, const float*
       for (int j = 1; j < Q; ++j) own[j] = ldp(uplane(in, m.S, j), d);
     }
   }
-  if (r.iolet != 0) {
+  const uint32_t aside = r.far & r.iolet;
+  if (aside != 0) {
 #pragma unroll
     for (int j = 1; j < Q; ++j)
-      if (r.iolet & (1u << (INV[j] - 1))) g[j] = ldp(plane(m.G, m.SI, j), r.ii);
+      if (aside & (1u << (INV[j] - 1))) g[j] = ldp(plane(m.G, m.SI, j), r.ii);
   }
   if (m.gz.bgz != nullptr && r.wall) {
     const uint32_t gzm = ldp(m.gz.bgz, b);
@@ -215,12 +216,12 @@ __device__ __forceinline__ IoletIn32 load_iolet32(const Member32& m, int step, u
 }
 
 template <int D = 1>
-__device__ __forceinline__ void nash_links32(const Member32& m, const Bnd& r, float drg, float inv, float usq15,
-                                             float gx, float gy, float gz) {
+__device__ __forceinline__ void nash_links32(const Member32& m, float* out, uint32_t slot, const Bnd& r, float drg,
+                                             float inv, float usq15, float gx, float gy, float gz) {
   if constexpr (D < Q) {
     if (r.iolet & (1u << (D - 1)))
-      stp(plane(m.G, m.SI, INV[D]), r.ii, geq_dir<INV[D]>(drg, inv, usq15, gx, gy, gz));
-    nash_links32<D + 1>(m, r, drg, inv, usq15, gx, gy, gz);
+      stp(iolet_place(D, uplane(out, m.S, D), slot, m.G, m.SI, r), 0, geq_dir<INV[D]>(drg, inv, usq15, gx, gy, gz));
+    nash_links32<D + 1>(m, out, slot, r, drg, inv, usq15, gx, gy, gz);
   }
 }
 
@@ -230,23 +231,24 @@ struct LaddIn32 {
 };
 
 template <int D0, int D = D0>
-__device__ __forceinline__ void ladd_links32(const Member32& m, const Bnd& r, const LaddIn32& io, const double* s,
-                                             const double* s2, float rho, const float* gpost) {
+__device__ __forceinline__ void ladd_links32(const Member32& m, float* out, uint32_t slot, const Bnd& r,
+                                             const LaddIn32& io, const double* s, const double* s2, float rho,
+                                             const float* gpost) {
   if constexpr (D < Q && D < D0 + kLaddGroup) {
     if (r.iolet & (1u << (D - 1))) {
       const float v = (float)(io.vmax * s[D - D0] + io.vmax2 * s2[D - D0]);
       const float wx = io.n[0] * v * rho, wy = io.n[1] * v * rho, wz = io.n[2] * v * rho;
       const float correction = 2.0f * wf(D) * cdotf<D>(wx, wy, wz) * 3.0f;
-      stp(plane(m.G, m.SI, INV[D]), r.ii, gpost[D] - correction);
+      stp(iolet_place(D, uplane(out, m.S, D), slot, m.G, m.SI, r), 0, gpost[D] - correction);
     }
-    ladd_links32<D0, D + 1>(m, r, io, s, s2, rho, gpost);
+    ladd_links32<D0, D + 1>(m, out, slot, r, io, s, s2, rho, gpost);
   }
 }
 
 // The profile factors of kLaddGroup links at a time, then their values.
 template <int D0 = 1>
-__device__ __forceinline__ void ladd_groups32(const Member32& m, const Bnd& r, const LaddIn32& io, float rho,
-                                              const float* gpost) {
+__device__ __forceinline__ void ladd_groups32(const Member32& m, float* out, uint32_t slot, const Bnd& r,
+                                              const LaddIn32& io, float rho, const float* gpost) {
   if constexpr (D0 < Q) {
     double s[kLaddGroup], s2[kLaddGroup];
 #pragma unroll
@@ -255,8 +257,8 @@ __device__ __forceinline__ void ladd_groups32(const Member32& m, const Bnd& r, c
       s[e] = ldp(m.ladd_s + (int64_t)(D0 + e - 1) * m.SI, r.ii);
       s2[e] = ldp(m.ladd_s2 + (int64_t)(D0 + e - 1) * m.SI, r.ii);
     }
-    ladd_links32<D0>(m, r, io, s, s2, rho, gpost);
-    ladd_groups32<D0 + kLaddGroup>(m, r, io, rho, gpost);
+    ladd_links32<D0>(m, out, slot, r, io, s, s2, rho, gpost);
+    ladd_groups32<D0 + kLaddGroup>(m, out, slot, r, io, rho, gpost);
   }
 }
 
@@ -264,18 +266,20 @@ __device__ __forceinline__ void ladd_groups32(const Member32& m, const Bnd& r, c
 // each iolet link (NashZerothOrderPressureDelegate.h:36-76,
 // LaddIoletDelegate.h:37-86), in shifted form, and the Windkessel coupling
 // site's flux term.
-__device__ __forceinline__ void iolet_links32(const Member32& m, int step, const Bnd& r, const IoletIn32& io, float rho,
-                                              float vx, float vy, float vz, const float* gpost) {
+__device__ __forceinline__ void iolet_links32(const Member32& m, float* out, uint32_t slot, int step, const Bnd& r,
+                                              const IoletIn32& io, float rho, float vx, float vy, float vz,
+                                              const float* gpost) {
   if (((int)r.gi < m.n_in ? m.inlet_bc : m.outlet_bc) == HLB_IOLET_NASH) {
     const float component = vx * io.n[0] + vy * io.n[1] + vz * io.n[2];
     const float gx = io.n[0] * component * io.rho, gy = io.n[1] * component * io.rho, gz = io.n[2] * component * io.rho;
     const float inv = 1.0f / io.rho;
     const float usq15 = 1.5f * (gx * gx + gy * gy + gz * gz) * inv;
-    nash_links32(m, r, io.drho, inv, usq15, gx, gy, gz);
+    nash_links32(m, out, slot, r, io.drho, inv, usq15, gx, gy, gz);
   } else {
     const int64_t row = (int64_t)step * m.row;
-    ladd_groups32(m, r, LaddIn32{ldp(m.io_vmax + row, r.gi), ldp(m.io_vmax2 + row, r.gi), {io.n[0], io.n[1], io.n[2]}},
-                  rho, gpost);
+    ladd_groups32(m, out, slot, r,
+                  LaddIn32{ldp(m.io_vmax + row, r.gi), ldp(m.io_vmax2 + row, r.gi), {io.n[0], io.n[1], io.n[2]}}, rho,
+                  gpost);
   }
   if (r.iolet & io.wk) {
     const double c = (double)vx * -ldp(m.io_n, 3u * r.gi) + (double)vy * -ldp(m.io_n, 3u * r.gi + 1) +
@@ -438,7 +442,7 @@ __device__ __forceinline__ void site_finish32(const Member32& m, const Planes& P
   const Collision32 cs = collide32(m, step, d, g, gpost);
   store_row32<NT>(m, P.out, d, gpost);
 
-  if (bnd.iolet != 0) iolet_links32(m, step, bnd, io, cs.rho, cs.ux, cs.uy, cs.uz, gpost);
+  if (bnd.iolet != 0) iolet_links32(m, P.out, d, step, bnd, io, cs.rho, cs.ux, cs.uy, cs.uz, gpost);
   if (step == m.props_at) {
     stp(m.rho, d, 1.0 + (double)cs.drho);
     stp(m.u, d, (double)cs.ux);

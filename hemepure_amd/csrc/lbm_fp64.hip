@@ -62,9 +62,11 @@ __device__ __forceinline__ void gather_site(const StepArgs& a, const Lane& L, do
   gather_up<NARROW>(a, L, own, f);
 }
 
-// The boundary delegates of one gathered site: f[j] already holds the site's
-// own post-collision value for every wall or iolet link INV[j], which is all
-// SimpleBounceBackDelegate.h:36-44 does.
+// The boundary delegates of one gathered site: f[j] already holds what the
+// site's own slot has in plane INV[j] for every wall or iolet link INV[j]: the
+// post-collision value at a wall link, which is all
+// SimpleBounceBackDelegate.h:36-44 does, and the iolet delegate's value at an
+// iolet link (iolet_links).
 //
 // A wave with boundary lanes is bound by instructions and by the chain of
 // loads it waits for, not by bytes.  So what each direction does is worked out
@@ -86,10 +88,11 @@ __device__ __forceinline__ void boundary_fixup(const StepArgs& a, uint32_t d, ui
       for (int j = 1; j < Q; ++j) own[j] = ldp(a.ain[j], d);
     }
   }
-  if (r.iolet != 0) {
+  const uint32_t aside = r.far & r.iolet;
+  if (aside != 0) {
 #pragma unroll
     for (int j = 1; j < Q; ++j)
-      if (r.iolet & (1u << (INV[j] - 1))) f[j] = ldp(plane(a.G, a.SI, j), r.ii);
+      if (aside & (1u << (INV[j] - 1))) f[j] = ldp(plane(a.G, a.SI, j), r.ii);
   }
   if (a.gz.bgz != nullptr && r.wall) {
     // GuoZhengShiDelegate: the link kernel's values.
@@ -127,26 +130,27 @@ __device__ __forceinline__ IoletIn load_iolet(const StepArgs& a, uint32_t gi) {
 }
 
 template <int D = 1>
-__device__ __forceinline__ void nash_links(const StepArgs& a, const Bnd& r, const FeqPre& p, double gx, double gy,
-                                           double gz) {
+__device__ __forceinline__ void nash_links(const StepArgs& a, uint32_t slot, const Bnd& r, const FeqPre& p, double gx,
+                                           double gy, double gz) {
   if constexpr (D < Q) {
-    if (r.iolet & (1u << (D - 1))) stp(plane(a.G, a.SI, INV[D]), r.ii, feq_dir<INV[D]>(p, gx, gy, gz));
-    nash_links<D + 1>(a, r, p, gx, gy, gz);
+    if (r.iolet & (1u << (D - 1))) stp(iolet_place(D, a.aout[D], slot, a.G, a.SI, r), 0, feq_dir<INV[D]>(p, gx, gy, gz));
+    nash_links<D + 1>(a, slot, r, p, gx, gy, gz);
   }
 }
 
-// Iolet delegates of one site: the value each iolet link k hands to the next
-// step in direction INV[k].  Nash: f_eq of the ghost state, one per site
-// (NashZerothOrderPressureDelegate.h:36-76; the normal is its float copy).
-// Ladd: bounce-back minus the moving-wall correction (LaddIoletDelegate.h:37-86).
-__device__ __forceinline__ void iolet_links(const StepArgs& a, const Bnd& r, const IoletIn& io, int bc, double rho,
-                                            double vx, double vy, double vz, const double* fpost) {
+// Iolet delegates of one site, after its row's stores: the value each iolet
+// link k hands to the next step in direction INV[k].  Nash: f_eq of the ghost
+// state, one per site (NashZerothOrderPressureDelegate.h:36-76; the normal is
+// its float copy).  Ladd: bounce-back minus the moving-wall correction
+// (LaddIoletDelegate.h:37-86).
+__device__ __forceinline__ void iolet_links(const StepArgs& a, uint32_t slot, const Bnd& r, const IoletIn& io, int bc,
+                                            double rho, double vx, double vy, double vz, const double* fpost) {
   if (bc == HLB_IOLET_NASH) {
     const double rg = io.dens;
     const double nx = (double)(float)io.n[0], ny = (double)(float)io.n[1], nz = (double)(float)io.n[2];
     const double component = vx * nx + vy * ny + vz * nz;
     const double gx = nx * component * rg, gy = ny * component * rg, gz = nz * component * rg;
-    nash_links(a, r, feq_pre(rg, gx, gy, gz), gx, gy, gz);
+    nash_links(a, slot, r, feq_pre(rg, gx, gy, gz), gx, gy, gz);
   } else {
     const double vmax = a.io_vmax[r.gi], vmax2 = a.io_vmax2[r.gi];
 #pragma unroll
@@ -167,7 +171,7 @@ __device__ __forceinline__ void iolet_links(const StepArgs& a, const Bnd& r, con
         const double wx = io.n[0] * m * rho, wy = io.n[1] * m * rho, wz = io.n[2] * m * rho;
         const double correction =
             2. * Wt(d) * (wx * (double)CX[d] + wy * (double)CY[d] + wz * (double)CZ[d]) / CS2;
-        stp(plane(a.G, a.SI, INV[d]), r.ii, fpost[d] - correction);
+        stp(iolet_place(d, a.aout[d], slot, a.G, a.SI, r), 0, fpost[d] - correction);
       }
     }
   }
@@ -314,7 +318,7 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(W > 0 ? W : 1
 
   if (bnd.iolet != 0) {
     const int bc = (int)bnd.gi < a.n_in ? a.inlet_bc : a.outlet_bc;
-    iolet_links(a, bnd, io, bc, rho, ux, uy, uz, fpost);
+    iolet_links(a, d, bnd, io, bc, rho, ux, uy, uz, fpost);
     // InOutLetWK*::DoPreStreamCoupling: the coupling site's velocity.Dot(-normal).
     if (bnd.iolet & io.wk) {
       const double c = ux * -io.n[0] + uy * -io.n[1] + uz * -io.n[2];

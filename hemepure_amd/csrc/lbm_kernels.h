@@ -28,9 +28,10 @@
 //          (collision classes 1-5) are numbered in slot order.
 //   boundary arrays (NB boundary sites, stride SB): one BndRec, 18 planes of
 //          float link distances, 3 planes of float wall normals.
-//   iolet arrays (NI sites with iolet links, slot order, stride SI): G, 19
-//          planes of the values the site's iolet delegates computed for the
-//          next step, and 18 planes of Ladd profile factors.
+//   iolet arrays (NI sites with iolet links, slot order, stride SI): 18 planes
+//          of Ladd profile factors, and G, 19 planes of values the site's iolet
+//          delegates computed for the next step where they cannot take the
+//          place of a post-collision one (iolet_place).
 #pragma once
 
 #include <cstdint>
@@ -289,7 +290,7 @@ struct Member32 {
   const BndRec* bnd;
   const float* bq;
   const float* bnrm;
-  float* G;               // iolet values for the next step, 19 planes of SI
+  float* G;               // 19 planes of SI (see iolet_place)
   const double* ladd_s;
   const double* ladd_s2;
   double* rho;
