@@ -578,6 +578,8 @@ __global__ __launch_bounds__(kBlock) void monitor_pass2(const Mon* __restrict__ 
     out[1] = t.hi;
     out[2] = t.umax;
     out[3] = t.mass;
+    // a host that sees out[4] set has the four before it
+    __hip_atomic_store(out + 4, 1.0, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
 
