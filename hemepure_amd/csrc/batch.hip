@@ -31,6 +31,7 @@ struct hlb_batch {
   int variant = hlb::kFp32DefaultVariant;
   bool variant_chosen = false;  // set by hlb_batch_set_variant / autotune; else default_variant
   int launch = hlb::kFp32DefaultVariant;  // the variant steps are launched in, as of the last rebuild
+  bool inner = false;                     // a member has links between fluid sites, likewise
   bool use_graph = true;
   bool dirty = true;  // member set or variant changed: rebuild tables, drop graphs
   uint32_t grid = 0;
@@ -99,6 +100,9 @@ int rebuild(hlb_batch* b) {
   } else {
     b->launch = b->variant;
   }
+  b->inner = false;
+  for (const hlb_lattice* m : b->members) b->inner = b->inner || m->inner_links();
+  if (b->inner) b->launch = inner_launch(b->launch);
   const LaunchShape shape = launch_shape(b->launch, true);
   const int64_t per = shape_slabs(shape);
   std::vector<int32_t> map;
@@ -134,7 +138,7 @@ int enqueue_sequence(hlb_batch* b, int64_t n) {
   const WkLaunch wk = wk_launch(b->refs.p, b->nwk, n);
   HLB_CHECK(launch_wk_start(b->refs.p, b->nwk, b->stream));
   for (int64_t s = 0; s < n; ++s) {
-    HLB_CHECK(launch_step_fp32(b->mem.p, b->wg_member.p, b->grid, (int)s, wk, b->launch, b->stream));
+    HLB_CHECK(launch_step_fp32(b->mem.p, b->wg_member.p, b->grid, (int)s, wk, b->launch, b->inner, b->stream));
     for (size_t i = 0; i < b->members.size(); ++i) {  // GZS walls, per member
       const hlb_lattice* m = b->members[i];
       if (!m->gz_links_host.empty())

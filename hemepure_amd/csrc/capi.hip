@@ -648,6 +648,7 @@ int upload_lattice(hlb_lattice* h) {
   // Boundary arrays in device order.
   std::vector<BndRec> rec(SB, BndRec{0, 0, 0, 0});
   std::vector<float> q((size_t)18 * SB, 0.0f), nr((size_t)3 * SB, 0.0f);
+  std::vector<uint32_t> inner(h->inner_links() ? (size_t)SB : 0, 0);
   {
     std::vector<int32_t> iolIndex(N, -1);
     for (int64_t i = 0; i < h->NI; ++i) iolIndex[h->isite[i]] = (int32_t)i;
@@ -658,6 +659,7 @@ int upload_lattice(hlb_lattice* h) {
         const uint32_t wm = L.wall[k];
         R.iolet = L.iolet[k];
         if (wm != 0) R.far |= 1u << 31;
+        if (!inner.empty() && (inner[(size_t)b] = L.inner[(size_t)k]) != 0) R.far |= kInnerLinks;
         // BouzidiFirdaousLallemandDelegate.h:44-93: a wall link whose opposite is
         // no wall interpolates, with the site's own opposite value from q = 1/2 on
         for (int j = 1; j < Q && h->params.wall_bc == HLB_WALL_BFL; ++j) {
@@ -677,6 +679,7 @@ int upload_lattice(hlb_lattice* h) {
   pack.add(h->bnd, rec);
   pack.add(h->bq, q);
   pack.add(h->bnrm, nr);
+  pack.add(h->inner, inner);
   pack.add(h->ladd_s, h->h_ladd_s);
   // Per-iolet constants and what the per-step values are copied to.
   {
@@ -1044,7 +1047,7 @@ int enqueue_steps(hlb_lattice* h, int64_t n, bool props_last) {
   if (h->fp32()) {
     const uint32_t grid = member_grid(h->nslab, variant);
     for (int64_t s = 0; s < n; ++s) {
-      HLB_CHECK(launch_step_fp32(h->member(), nullptr, grid, (int)s, wk, variant, h->stream));
+      HLB_CHECK(launch_step_fp32(h->member(), nullptr, grid, (int)s, wk, variant, h->inner_links(), h->stream));
       HLB_CHECK(launch_gzs_fp32(h->member(), h->gz_links.p, (int)h->gz_links_host.size(), (int)s, h->stream));
     }
     HLB_CHECK(launch_wk_flush(h->wk_refs.p, nwk, (int)(n - 1), h->stream));
@@ -1612,7 +1615,9 @@ extern "C" int hlb_neighbour_tables(hlb_handle h, int64_t* push, uint32_t* pull)
     HLB_CHECK(hipStreamSynchronize(h->stream));
     for (int j = 0; j < 18; ++j)
       for (int64_t k = 0; k < N; ++k) {
-        const uint32_t v = tmp[(size_t)j * S + h->inv[k]];
+        uint32_t v = tmp[(size_t)j * S + h->inv[k]];
+        // the boundary delegates replace what a link between fluid sites gathered
+        if (h->inner_links() && ((h->L.inner[(size_t)k] >> (INV[j + 1] - 1)) & 1u)) v = (uint32_t)h->inv[k];
         pull[(size_t)j * N + k] = v < (uint32_t)S ? (uint32_t)h->perm[v] : 0xffffffffu;
       }
   }

@@ -212,9 +212,11 @@ __device__ __forceinline__ uint32_t upstream_pos(const Lane& L, uint64_t& fluid_
 // where the upstream position is not fluid (a wall or iolet link ib = INV[J])
 // the lane reads its own value in plane ib -- the bounce-back value, which SBB
 // keeps, BFL keeps or interpolates from and iolet and GZS links replace -- so
-// no boundary delegate loads it.  The pair's plane offset is folded into the
-// scalar bases, and own[k] (the own slot in the k-th plane of a pair) into two
-// values a lane forms once, so the choice costs one select.
+// no boundary delegate loads it, except for a link between two fluid sites
+// (kInnerLinks), where the upstream position is fluid.  The pair's plane
+// offset is folded into the scalar bases, and own[k] (the own slot in the k-th
+// plane of a pair) into two values a lane forms once, so the choice costs one
+// select.
 template <int J, typename T>
 __device__ __forceinline__ T gather_bb(const T* lower, uint32_t S, const Lane& L, const uint32_t (&own)[2]) {
   constexpr bool upper = J > INV[J];
@@ -236,16 +238,17 @@ __device__ __forceinline__ Bnd no_bnd() { return Bnd{0, 0, 0, 0, 0, false}; }
 __device__ __forceinline__ Bnd load_bnd(const BndRec* rec, uint32_t b) {
   typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
   const u32x4 v = *(const HLB_GLOBAL u32x4*)(rec + b);
-  return Bnd{v.x & kLinkBits, v.y & kLinkBits, v.z, v.y >> 18, v.w, (v.x >> 31) != 0};
+  return Bnd{v.x & (kLinkBits | kInnerLinks), v.y & kLinkBits, v.z, v.y >> 18, v.w, (v.x >> 31) != 0};
 }
 
 // Where the value of iolet link d goes, which is what the next step gathers in
-// direction INV[d]: into the site's own post-collision row, plane d.  No site
-// lies downstream of an iolet link, so nothing but the site's own bounce-back
-// gather (gather_bb) reads it there, and the next step has no load of its own
-// for it.  BFL's interpolation with the site's own value (a wall link opposite
-// the iolet link, far bit d) needs the post-collision value in that place; the
-// iolet's then goes to G.
+// direction INV[d]: into the site's own post-collision row, plane d.  Nothing but
+// the site's own bounce-back gather (gather_bb) reads it there: no site lies
+// downstream of an iolet link, or one that does has the link from its side too
+// and replaces what it gathered (kInnerLinks).  So the next step has no load
+// of its own for it.  BFL's interpolation with the site's own value (a wall link
+// opposite the iolet link, far bit d) needs the post-collision value in that
+// place; the iolet's then goes to G.
 // With every value in G the waves of an iolet layer, which decide a small
 // lattice's step, had one more round of loads (boundary record, iolet index, G)
 // ahead of the collision: 30k-site cylinder FP64 5.98 -> 5.50 us a step, FP32

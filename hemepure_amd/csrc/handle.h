@@ -31,7 +31,7 @@ hipError_t launch_unstable_fp64(const BrickTables& bt, const double* F, int64_t 
 hipError_t launch_wk_start(const WkRef* refs, int n, hipStream_t s);
 hipError_t launch_wk_flush(const WkRef* refs, int n, int last, hipStream_t s);
 hipError_t launch_step_fp32(const Member32* members, const int32_t* wg_member, uint32_t grid, int step,
-                            const WkLaunch& wk, int variant, hipStream_t s);
+                            const WkLaunch& wk, int variant, bool inner, hipStream_t s);
 hipError_t launch_gather_fp32(const Member32* members, int64_t nslab, float* F, hipStream_t s);
 hipError_t launch_fill_fp32(float* F, int64_t N, int64_t S, const float* vals, hipStream_t s);
 hipError_t launch_unstable_fp32(const BrickTables& bt, const float* F, int64_t S, int* flag, hipStream_t s);
@@ -187,7 +187,7 @@ struct hlb_lattice {
   hlb::DevBuf<hlb::GzsLink> gz_links;
   hlb::DevBuf<uint64_t> pmask;
   hlb::DevBuf<int32_t> pbase, bgzbase;
-  hlb::DevBuf<uint32_t> bgz;
+  hlb::DevBuf<uint32_t> bgz, inner;  // inner: L.inner per boundary site
   hlb::DevBuf<double> P64, GW64;
   hlb::DevBuf<float> P32, GW32;
   hlb::DevBuf<char> mon_scratch;  // monitor partials, allocated on first use
@@ -248,8 +248,10 @@ struct hlb_lattice {
   bool variant_chosen = false;              // set by hlb_set_variant / hlb_autotune; else default_variant
   // The variant steps are launched in.
   int launch_variant() const {
-    return variant_chosen ? variant : hlb::default_launch(hlb::distribution_bytes(S, fp32()), fp32());
+    const int v = variant_chosen ? variant : hlb::default_launch(hlb::distribution_bytes(S, fp32()), fp32());
+    return fp32() && inner_links() ? hlb::inner_launch(v) : v;
   }
+  bool inner_links() const { return !L.inner.empty(); }  // links between fluid sites
   bool general_gather = false;  // HLB_FP64_GENERAL_GATHER=1 when the device state was made
   // Step sequences captured into HIP graphs and replayed: one per (length,
   // property flag, first-step flag, buffer parity, launch shape); the FP32
@@ -278,8 +280,9 @@ struct hlb_lattice {
   }
   bool fp32() const { return params.precision == HLB_FP32_SHIFTED; }
   hlb::GzsTables gz_tables() const {
-    if (gz_links_host.empty()) return hlb::GzsTables{nullptr, nullptr, nullptr, nullptr, 0};
-    return hlb::GzsTables{pmask.p, pbase.p, bgz.p, bgzbase.p, SP};
+    const uint32_t* in = inner_links() ? inner.p : nullptr;
+    if (gz_links_host.empty()) return hlb::GzsTables{nullptr, nullptr, nullptr, nullptr, in, 0};
+    return hlb::GzsTables{pmask.p, pbase.p, bgz.p, bgzbase.p, in, SP};
   }
   hlb::BrickTables tables() const {
     return hlb::BrickTables{rec.p, nslab};

@@ -13,8 +13,9 @@
 // boundary delegate of site k itself writes it (SimpleBounceBack, BFL, Nash,
 // Ladd all write fNew[k*19 + INV[d]] for their link d).  Each (site, j) slot
 // must have exactly one writer in the reference's push step; geometries where
-// a link's type disagrees with its neighbour's fluidity give zero or two
-// writers and are rejected.
+// the two sides of a link disagree give zero or two writers and are rejected.  A
+// link that is a wall or an iolet from both sides has one writer whether or not
+// there is fluid beyond it: two sites with a wall of no thickness between them.
 #include "lattice.h"
 
 #include <atomic>
@@ -261,7 +262,9 @@ int build_lattice(const hlb_geometry& g, HostLattice& L) {
 
   // The one-writer check, cell by cell: a plain link's neighbour must be
   // fluid with a plain link back, any other link's must not push here.
+  std::atomic<bool> inner{false};
   parallel_ranges(nslot, [&](int, int64_t lo, int64_t hi) {
+    uint32_t found = 0;  // what lies beyond wall and iolet links
     for (int64_t s = lo; s < hi; ++s) {
       const int64_t b = slotBlock[(size_t)s], bx = b / (BY * BZ), by = (b / BZ) % BY, bz = b % BZ;
       const uint32_t* around[27];  // the 3 x 3 x 3 blocks' cells
@@ -302,11 +305,26 @@ int build_lattice(const hlb_geometry& g, HostLattice& L) {
             bad.store(true, std::memory_order_relaxed);
             return;
           }
+          found |= plain ? 0 : src;
         }
       }
     }
+    if (found & kFluid) inner.store(true, std::memory_order_relaxed);
   }, slotGrain);
-  return bad.load() ? one_writer_error(L) : HLB_OK;
+  if (bad.load()) return one_writer_error(L);
+  if (inner.load()) {
+    L.inner.resize((size_t)n);
+    parallel_ranges(n, [&](int, int64_t lo, int64_t hi) {
+      for (int64_t k = lo; k < hi; ++k) {
+        L.inner[(size_t)k] = 0;
+        for (int d = 1; d < Q; ++d)
+          if (link_of(L, k, d) != HLB_LINK_NONE &&
+              L.site_at(L.coords[3 * k] + CX[d], L.coords[3 * k + 1] + CY[d], L.coords[3 * k + 2] + CZ[d]) >= 0)
+            L.inner[(size_t)k] |= 1u << (d - 1);
+      }
+    });
+  }
+  return HLB_OK;
 }
 
 void pull_table(const HostLattice& L, uint32_t* out) {

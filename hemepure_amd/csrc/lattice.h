@@ -23,6 +23,9 @@ struct HostLattice {
   RawVector<uint32_t> iolet;   // N, bit d-1 set for an inlet/outlet link d
   RawVector<int32_t> ioletId;  // N
   RawVector<int32_t> siteType; // N
+  // N, bit d-1 set for a wall or iolet link d that leads to a fluid site; empty
+  // when no link does.
+  RawVector<uint32_t> inner;
   RawVector<float> q;          // N*18 link distances as read
   RawVector<float> nrm;        // N*3 wall normal normalised in float (+inf if none)
   // Site map: per block a slot (or -1), per slot the block's contiguous indices (or -1).

@@ -163,7 +163,8 @@ __device__ __forceinline__ void gather_site32(const float* in, int64_t S, const 
 
 // The boundary delegates of one gathered site, as boundary_fixup in the FP64
 // pass (SimpleBounceBackDelegate.h:36-44, BouzidiFirdaousLallemandDelegate.h:
-// 44-93).
+// 44-93).  INNER: the lattice may have links between fluid sites (kInnerLinks).
+template <bool INNER>
 __device__ __forceinline__ void boundary_fixup32(const Member32& m, const float* in, uint32_t d, uint32_t b,
                                                  const Bnd& r, float* g) {
   float q[Q], own[Q];
@@ -173,6 +174,14 @@ __device__ __forceinline__ void boundary_fixup32(const Member32& m, const float*
     if (r.far != 0) {
 #pragma unroll
       for (int j = 1; j < Q; ++j) own[j] = ldp(uplane(in, m.S, j), d);
+      if constexpr (INNER) {
+        if (r.far & kInnerLinks) {
+          const uint32_t links = ldp(m.gz.inner, b);
+#pragma unroll
+          for (int j = 1; j < Q; ++j)
+            if (links & (1u << (INV[j] - 1))) g[j] = own[INV[j]];
+        }
+      }
     }
   }
   const uint32_t aside = r.far & r.iolet;
@@ -456,7 +465,7 @@ __device__ __forceinline__ void site_finish32(const Member32& m, const Planes& P
 // B threads per workgroup tile, each wavefront SPT consecutive slabs (the
 // gathers of all of them issued before any is waited for); ORDER: the tile
 // order (TileOrder); NT: non-temporal stores of the post-collision rows.
-template <int B, int ORDER, int W = 0, int SPT = 1, bool NT = false>
+template <int B, int ORDER, int W = 0, int SPT = 1, bool NT = false, bool INNER = false>
 __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(W > 0 ? W : 1))) void step_fp32(
     const Member32* __restrict__ members, const int32_t* __restrict__ wg_member, int step, WkLaunch wk) {
   if (wk_workgroup(wk, step)) return;
@@ -478,7 +487,7 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(W > 0 ? W : 1
       for (int j = 0; j < Q; ++j) g[j] = ldp(uplane(P.in, m.S, j), L.slot);
     } else {
       gather_site32(P.in, m.S, L, g);
-      if (L.boundary) boundary_fixup32(m, P.in, L.slot, L.b, bnd, g);
+      if (L.boundary) boundary_fixup32<INNER>(m, P.in, L.slot, L.b, bnd, g);
     }
     site_finish32<NT>(m, P, step, L, bnd, g);
   } else {
@@ -488,7 +497,7 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(W > 0 ? W : 1
 #pragma unroll
     for (int k = 0; k < SPT; ++k) {
       if (!s[k].ok) continue;
-      if (!P.first && s[k].L.boundary) boundary_fixup32(m, P.in, s[k].L.slot, s[k].L.b, s[k].bnd, s[k].g);
+      if (!P.first && s[k].L.boundary) boundary_fixup32<INNER>(m, P.in, s[k].L.slot, s[k].L.b, s[k].bnd, s[k].g);
       site_finish32<NT>(m, P, step, s[k].L, s[k].bnd, s[k].g);
     }
   }
@@ -570,7 +579,7 @@ __global__ __launch_bounds__(kBlock) void gather_fp32(const Member32* __restrict
   if (L.boundary) bnd = load_bnd(m.bnd, L.b);
   float g[Q];
   gather_site32(in, m.S, L, g);
-  if (L.boundary) boundary_fixup32(m, in, L.slot, L.b, bnd, g);
+  if (L.boundary) boundary_fixup32<true>(m, in, L.slot, L.b, bnd, g);
 #pragma unroll
   for (int j = 0; j < Q; ++j) stp(plane(F, m.S, j), L.slot, g[j]);
 }
@@ -670,12 +679,22 @@ unsigned shape_lds(const LaunchShape& l) {
 }
 
 // `grid` workgroup tiles of the variant's size, padded as shape_grid pads
-// them (padding tiles map to member -1).
+// them (padding tiles map to member -1).  inner: a member has links between
+// fluid sites, and the variant is an inner_launch one.
 hipError_t launch_step_fp32(const Member32* members, const int32_t* wg_member, uint32_t grid, int step,
-                            const WkLaunch& wk, int variant, hipStream_t s) {
+                            const WkLaunch& wk, int variant, bool inner, hipStream_t s) {
   if (grid == 0) return hipSuccess;
   grid += wk.groups;
   const LaunchShape l = launch_shape(variant, true);
+  if (inner) {
+    if (l.nt)
+      hipLaunchKernelGGL((step_fp32<kSlab, kOrderXcd, 0, 1, true, true>), dim3(grid), dim3(kSlab), 0, s, members,
+                         wg_member, step, wk);
+    else
+      hipLaunchKernelGGL((step_fp32<kSlab, kOrderXcd, 0, 1, false, true>), dim3(grid), dim3(kSlab), 0, s, members,
+                         wg_member, step, wk);
+    return hipGetLastError();
+  }
   const unsigned lds = shape_lds(l);
 #define HLB_VN(B, O, W, NT)                                                                                  \
   if (l.spt == 2)                                                                                            \

@@ -66,7 +66,8 @@ __device__ __forceinline__ void gather_site(const StepArgs& a, const Lane& L, do
 // site's own slot has in plane INV[j] for every wall or iolet link INV[j]: the
 // post-collision value at a wall link, which is all
 // SimpleBounceBackDelegate.h:36-44 does, and the iolet delegate's value at an
-// iolet link (iolet_links).
+// iolet link (iolet_links).  Where such a link leads to a fluid site it holds the
+// neighbour's value, and the site's own takes its place (kInnerLinks).
 //
 // A wave with boundary lanes is bound by instructions and by the chain of
 // loads it waits for, not by bytes.  So what each direction does is worked out
@@ -86,6 +87,12 @@ __device__ __forceinline__ void boundary_fixup(const StepArgs& a, uint32_t d, ui
     if (r.far != 0) {
 #pragma unroll
       for (int j = 1; j < Q; ++j) own[j] = ldp(a.ain[j], d);
+      if (r.far & kInnerLinks) {
+        const uint32_t links = ldp(a.gz.inner, b);
+#pragma unroll
+        for (int j = 1; j < Q; ++j)
+          if (links & (1u << (INV[j] - 1))) f[j] = own[INV[j]];
+      }
     }
   }
   const uint32_t aside = r.far & r.iolet;

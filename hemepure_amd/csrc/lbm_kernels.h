@@ -16,8 +16,10 @@
 // site's upstream neighbour is found arithmetically from the fluid masks and
 // bases of the slabs around it, which the slab's record lists, so no
 // per-site neighbour table is read.  A link whose upstream position is not
-// fluid (a wall or iolet link) reads the site's own slot instead, and the
-// boundary delegates overwrite the value.
+// fluid reads the site's own slot instead, which holds what a wall or iolet link
+// hands back; a wall or iolet link to a position that is fluid (no thickness
+// between two sites) is marked (kInnerLinks) and its value replaced by the
+// boundary delegates.
 //
 // HBM layout (S = compact slots rounded up to 64):
 //   A[2]   post-collision distributions, 19 planes of S (double, or float
@@ -74,13 +76,20 @@ static_assert(sizeof(SlabRec) == 256, "slab record is four 64-byte scalar loads"
 // Bits are links (d - 1) or pull directions (j - 1); direction j's value is
 // written by link INV[j].
 struct BndRec {
-  uint32_t far;    // directions BFL interpolates with the site's own value (q >= 1/2); bit 31: a wall site
+  uint32_t far;    // directions BFL interpolates with the site's own value (q >= 1/2); kInnerLinks; bit 31: a wall site
   uint32_t near;   // directions BFL interpolates with the streamed value (q < 1/2); bits 18..: global iolet index
   uint32_t iolet;  // iolet links
   uint32_t ii;     // compact iolet index (sites with iolet links)
 };
 static_assert(sizeof(BndRec) == 16, "one 16-byte load");
 constexpr uint32_t kLinkBits = (1u << 18) - 1u;
+// Bit of BndRec::far at sites with a wall or iolet link to a fluid site (a wall of
+// no thickness).  FP64 lattices without such links do no more than test the bit
+// where BFL loads a site's own row, which cost nothing measurable.  In the FP32
+// step any form of the test did on a 6k-site pipe, whose step is one chain of
+// loads (6.6 us: 1.3 to 2.3%, a null pointer tested beside the GZS tables' 1.4%),
+// so its kernels are compiled without it and once with it (inner_launch).
+constexpr uint32_t kInnerLinks = 1u << 30;
 
 // The brick tables of one lattice.
 struct BrickTables {
@@ -176,6 +185,11 @@ inline int default_launch(int64_t dist_bytes, bool fp32, bool batch = false) {
   return (fp32 ? kFp32Shapes : kFp64Shapes) + (chunks ? chunk64 : 1);
 }
 
+// The FP32 variant launched in place of `variant` when a lattice or a member of a
+// batch has links between fluid sites: one-slab tiles in XCD order with its store
+// policy, the one shape compiled for them.
+inline int inner_launch(int variant) { return (launch_shape(variant, true).nt ? kFp32Shapes : 0) + 5; }
+
 // Guo-Zheng-Shi wall links (GuoZhengShiDelegate.h:123-294).  Sites whose
 // pre-collision f the link kernel needs (GZS wall sites and the next fluid
 // site out along a link) store it in P during the step; the link kernel
@@ -185,6 +199,7 @@ struct GzsTables {
   const int32_t* pbase;   // per active slab: P index of the first such lane
   const uint32_t* bgz;    // per boundary site: wall links whose value comes from GW
   const int32_t* bgzbase; // per boundary site: GW index of its first GZS link
+  const uint32_t* inner;  // per boundary site: wall and iolet links to a fluid site (any wall delegate; see kInnerLinks)
   int64_t SP;             // P plane stride
 };
 
