@@ -745,17 +745,17 @@ int ensure_device(hlb_lattice* h) {
     const char* force = std::getenv("HLB_FP64_GENERAL_GATHER");
     h->general_gather = force && force[0] == '1';
   }
-  int rc = HLB_OK;
-  if (!h->stream) {
-    rc = take_lane(h->device, (size_t)h->stage_doubles(), h->lane);
-    if (rc != HLB_OK) return rc;
-    h->stream = h->lane.stream;
-    h->ev0 = h->lane.ev0;
-    h->ev1 = h->lane.ev1;
-    h->h_stage = h->lane.stage;
-  }
-  rc = upload_lattice(h);
+  int rc = take_lane(h->device, (size_t)h->stage_doubles(), h->lane);
   if (rc != HLB_OK) return rc;
+  h->use_lane();
+  rc = upload_lattice(h);
+  if (rc != HLB_OK) {
+    // without a state the iolets, which size the staging, may still change
+    (void)hipStreamSynchronize(h->stream);
+    give_lane(h->lane);
+    h->use_lane();
+    return rc;
+  }
   transfer_open();
   h->device_ready = true;
   return HLB_OK;

@@ -159,9 +159,15 @@ struct hlb_lattice {
   std::vector<hlb::HostIolet> iolets;  // inlets then outlets
   int n_in = 0, n_out = 0;
   int device = 0;
-  hlb::HostLane lane;  // the stream, events and pinned staging below
+  hlb::HostLane lane;  // the stream, events and pinned staging below, while there is a device state
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
+  void use_lane() {
+    stream = lane.stream;
+    ev0 = lane.ev0;
+    ev1 = lane.ev1;
+    h_stage = lane.stage;
+  }
   // Device slots (compact slab layout): perm[slot] = reference index or -1
   // for padding, inv[k] = slot of reference index k.
   std::vector<int32_t> perm, inv;
