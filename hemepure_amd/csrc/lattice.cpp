@@ -36,8 +36,7 @@ int64_t HostLattice::site_at(int64_t x, int64_t y, int64_t z) const {
   const int64_t b = ((x / bs) * blocks[1] + (y / bs)) * blocks[2] + (z / bs);
   const int64_t slot = blockSlot[b];
   if (slot < 0) return -1;
-  const int64_t s = (((x % bs) * bs) + (y % bs)) * bs + (z % bs);
-  return slotSites[slot * (int64_t)bs * bs * bs + s];
+  return slotSites[slot * (int64_t)bs * bs * bs + cell_in_block<int64_t>(x, y, z, bs)];
 }
 
 int HostLattice::collision_class(int64_t k) const {
@@ -152,7 +151,7 @@ int build_lattice(const hlb_geometry& g, HostLattice& L) {
     for (int64_t i = lo; i < hi; ++i) {
       const int32_t x = g.coords[3 * i], y = g.coords[3 * i + 1], z = g.coords[3 * i + 2];
       const int64_t slot = L.blockSlot[(size_t)(((x / b) * BY + (y / b)) * BZ + (z / b))];
-      int32_t* cell = &cellInput[(size_t)(slot * spb + (((x % b) * b) + (y % b)) * b + (z % b))];
+      int32_t* cell = &cellInput[(size_t)(slot * spb + cell_in_block(x, y, z, b))];
       if (__atomic_exchange_n(cell, (int32_t)i, __ATOMIC_RELAXED) >= 0) {
         bad.store(true, std::memory_order_relaxed);
         return;

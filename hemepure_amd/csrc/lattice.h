@@ -13,6 +13,13 @@ namespace hlb {
 // SiteType (src/geometry/SiteType.h:17-24).
 enum : int32_t { kSolidType = 0, kFluidType = 1, kInletType = 2, kOutletType = 3 };
 
+// Cell of position (x, y, z) within its block of side bs, z fastest; the cells of
+// a block of side 1291 no longer fit 32 bits.
+template <typename T>
+int64_t cell_in_block(T x, T y, T z, T bs) {
+  return ((int64_t)(x % bs) * bs + y % bs) * bs + z % bs;
+}
+
 struct HostLattice {
   int32_t blocks[3] = {0, 0, 0};
   int32_t bs = 8;
