@@ -1653,10 +1653,12 @@ int64_t device_bytes(const hlb_lattice* h) {
   const int64_t fsz = h->fp32() ? 4 : 8;
   int64_t b = 3 * Q * fsz * S + Q * fsz * SI;        // A[2], F, G
   b += (int64_t)sizeof(SlabRec) * std::max<int64_t>(h->nslab, 1);  // slab records
-  b += (4 * 4 + 18 * 4 + 3 * 4) * SB;                 // boundary masks, ids, q, normals
-  b += 36 * 8 * SI + 12 * SI;                         // Ladd factors, Windkessel terms and places
-  b += 5 * 8 * S;                                     // rho, u, wss
-  b += (int64_t)(3 * kChunk + 8) * 8 * std::max<int64_t>(1, (int64_t)h->iolets.size());  // iolet rows
+  b += (16 + 18 * 4 + 3 * 4 + (h->inner_links() ? 4 : 0)) * SB;  // boundary records, q, normals, marked links
+  b += 36 * 8 * SI + 4 * SI + 16 * h->wk_stride();    // Ladd factors, Windkessel places and two sets of terms
+  b += 5 * 8 * S + 4 * h->L.N;                        // rho, u, wss, the site -> slot index
+  b += 8 * h->stage_doubles();                        // member record and per-step rows
+  b += (12 + 24 + 4 + (int64_t)(sizeof(WkIolet) + sizeof(WkRef))) * h->iolet_count();  // per-iolet constants and state
+  b += 32 * 256;                                      // alignment of the small arrays in their allocation
   return b;
 }
 
