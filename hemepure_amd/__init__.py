@@ -165,6 +165,7 @@ _SIGS = {
     "hlb_noalloc_scratch_bytes": (C.c_int64, []),
     "hlb_set_variant": (C.c_int, [C.c_void_p, C.c_int]),
     "hlb_set_graphs": (C.c_int, [C.c_void_p, C.c_int]),
+    "hlb_captured_graphs": (C.c_int, [C.c_void_p]),
     "hlb_variant": (C.c_int, [C.c_void_p]),
     "hlb_autotune": (C.c_int, [C.c_void_p, C.c_int64, C.POINTER(C.c_int), C.POINTER(C.c_double)]),
     "hlb_set_params": (C.c_int, [C.c_void_p, C.POINTER(Params)]),
@@ -191,6 +192,7 @@ _SIGS = {
     "hlb_batch_step": (C.c_int, [C.c_void_p, C.c_int64, C.c_uint32]),
     "hlb_batch_step_timed": (C.c_int, [C.c_void_p, C.c_int64, C.c_uint32, C.POINTER(C.c_double)]),
     "hlb_batch_set_graphs": (C.c_int, [C.c_void_p, C.c_int]),
+    "hlb_batch_captured_graphs": (C.c_int, [C.c_void_p]),
     "hlb_batch_set_variant": (C.c_int, [C.c_void_p, C.c_int]),
     "hlb_batch_variant": (C.c_int, [C.c_void_p]),
     "hlb_batch_autotune": (C.c_int, [C.c_void_p, C.c_int64, C.POINTER(C.c_int), C.POINTER(C.c_double)]),
@@ -563,6 +565,10 @@ class Lattice:
         """Replay captured step sequences (True, the default) or launch eagerly."""
         _check(lib().hlb_set_graphs(self._h, 1 if enable else 0))
 
+    def captured_graphs(self) -> int:
+        """Captured step sequences held for replay."""
+        return int(lib().hlb_captured_graphs(self._h))
+
     def variant(self) -> int:
         return int(lib().hlb_variant(self._h))
 
@@ -711,6 +717,10 @@ class Batch:
 
     def set_graphs(self, enable: bool):
         _check(lib().hlb_batch_set_graphs(self._h, 1 if enable else 0))
+
+    def captured_graphs(self) -> int:
+        """Captured step sequences held for replay."""
+        return int(lib().hlb_batch_captured_graphs(self._h))
 
     def set_variant(self, variant: int):
         _check(lib().hlb_batch_set_variant(self._h, variant))

@@ -291,6 +291,8 @@ extern "C" int hlb_batch_set_graphs(hlb_batch_handle b, int enable) {
   return HLB_OK;
 }
 
+extern "C" int hlb_batch_captured_graphs(hlb_batch_handle b) { return b ? (int)b->graphs.size() : -1; }
+
 extern "C" int hlb_batch_set_variant(hlb_batch_handle b, int variant) {
   if (!b) return fail(HLB_EINVAL, "hlb_batch_set_variant: null batch");
   if (variant < 0 || variant >= kFp32Variants) return fail(HLB_EINVAL, "hlb_batch_set_variant: no such variant");

@@ -1317,6 +1317,8 @@ extern "C" int hlb_set_graphs(hlb_handle h, int enable) {
   return HLB_OK;
 }
 
+extern "C" int hlb_captured_graphs(hlb_handle h) { return h ? (int)h->graphs.size() : -1; }
+
 extern "C" int hlb_set_iolets(hlb_handle h, const hlb_iolet_desc* inlets, int n_inlets, const hlb_iolet_desc* outlets,
                               int n_outlets) {
   if (!h) return fail(HLB_EINVAL, "hlb_set_iolets: null handle");

@@ -237,6 +237,8 @@ int hlb_step_timed(hlb_handle h, int64_t nsteps, uint32_t flags, double* ms);
  * hide it, and with enable = 0 every sequence, are launched step by step.  Results are bit-identical either way.  Changing it, or tau via
  * hlb_set_params, drops the captured graphs. */
 int hlb_set_graphs(hlb_handle h, int enable);
+/* Captured sequences the handle holds (at most 8), -1 for a null handle. */
+int hlb_captured_graphs(hlb_handle h);
 /* Blocks until the handle's stream is idle. */
 int hlb_synchronize(hlb_handle h);
 
@@ -374,6 +376,7 @@ int hlb_batch_step(hlb_batch_handle b, int64_t nsteps, uint32_t flags);
 int hlb_batch_step_timed(hlb_batch_handle b, int64_t nsteps, uint32_t flags, double* ms);
 /* As hlb_set_graphs, for the batch's sequences (default on). */
 int hlb_batch_set_graphs(hlb_batch_handle b, int enable);
+int hlb_batch_captured_graphs(hlb_batch_handle b);
 /* Launch variant, as for hlb_set_variant of an FP32-shifted lattice (0..215). */
 int hlb_batch_set_variant(hlb_batch_handle b, int variant);
 int hlb_batch_variant(hlb_batch_handle b);
