@@ -149,24 +149,28 @@ int enqueue_sequence(hlb_batch* b, int64_t n) {
   return HLB_OK;
 }
 
-// Launches n steps whose iolet values and member records are staged, from
-// a captured graph when enabled.
-int launch_sequence(hlb_batch* b, int64_t n, int props_at) {
-  if (n <= 0) return HLB_OK;
-  // GZS walls add a launch per member and step, which a replay saves at any size
+// Whether an n-step sequence is replayed.  GZS walls add a launch per member and
+// step, which a replay saves at any size.
+bool replays(const hlb_batch* b, int64_t n) {
   int64_t slabs = 0;
   bool links = false;
   for (const hlb_lattice* m : b->members) {
     slabs += m->nslab;
     links = links || !m->gz_links_host.empty();
   }
-  if (!b->use_graph || !replay_pays(n, links ? 0 : slabs)) return enqueue_sequence(b, n);
+  return b->use_graph && replay_pays(n, links ? 0 : slabs);
+}
+
+// Launches n steps whose iolet values and member records are staged, from
+// a captured graph or one by one.
+int launch_sequence(hlb_batch* b, int64_t n, int props_at, bool graph) {
+  if (n <= 0) return HLB_OK;
+  if (!graph) return enqueue_sequence(b, n);
   for (const auto& g : b->graphs)
     if (g.n == n && g.props_at == props_at) {
       HLB_CHECK(hipGraphLaunch(g.exec, b->stream));
       return HLB_OK;
     }
-  hipGraph_t graph = nullptr;
   HLB_CHECK(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
   const int rc = enqueue_sequence(b, n);
   hipGraph_t captured = nullptr;
@@ -176,10 +180,9 @@ int launch_sequence(hlb_batch* b, int64_t n, int props_at) {
     return rc;
   }
   HLB_CHECK(end);
-  graph = captured;
   hipGraphExec_t exec = nullptr;
-  const hipError_t inst = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
-  (void)hipGraphDestroy(graph);
+  const hipError_t inst = hipGraphInstantiate(&exec, captured, nullptr, nullptr, 0);
+  (void)hipGraphDestroy(captured);
   HLB_CHECK(inst);
   b->graphs.push_back({n, props_at, exec});
   HLB_CHECK(hipGraphLaunch(exec, b->stream));
@@ -214,8 +217,8 @@ int stage_chunk(hlb_batch* b, int64_t n, int props_at) {
 }
 
 // Launches a staged chunk and advances the members' host state.
-int launch_chunk(hlb_batch* b, int64_t n, int props_at) {
-  const int rc = launch_sequence(b, n, props_at);
+int launch_chunk(hlb_batch* b, int64_t n, int props_at, bool graph) {
+  const int rc = launch_sequence(b, n, props_at, graph);
   if (rc != HLB_OK) return rc;
   for (hlb_lattice* m : b->members) advance_state(m, n);
   return HLB_OK;
@@ -314,16 +317,18 @@ extern "C" int hlb_batch_step(hlb_batch_handle b, int64_t nsteps, uint32_t flags
     const int64_t n = std::min<int64_t>(kChunk, nsteps - done);
     const int props_at = ((flags & HLB_STEP_PROPERTIES) && done + n == nsteps) ? (int)(n - 1) : -1;
     rc = stage_chunk(b, n, props_at);
-    if (rc == HLB_OK) rc = launch_chunk(b, n, props_at);
+    if (rc == HLB_OK) rc = launch_chunk(b, n, props_at, replays(b, n));
     if (rc != HLB_OK) return rc;
     done += n;
   }
   return release_members(b);
 }
 
-extern "C" int hlb_batch_step_timed(hlb_batch_handle b, int64_t nsteps, uint32_t flags, double* ms) {
-  if (!b || !ms) return fail(HLB_EINVAL, "hlb_batch_step_timed: null argument");
-  if (nsteps < 0 || nsteps > kChunk) return fail(HLB_EINVAL, "hlb_batch_step_timed: 0 to 1024 steps per timed call");
+namespace hlb {
+namespace {
+
+// nsteps timed steps; replayed if sequences of `like` steps are.
+int timed_steps(hlb_batch* b, int64_t nsteps, uint32_t flags, int64_t like, double* ms) {
   int rc = prepare(b, "hlb_batch_step_timed");
   if (rc != HLB_OK) return rc;
   if (b->members.empty()) {
@@ -336,7 +341,7 @@ extern "C" int hlb_batch_step_timed(hlb_batch_handle b, int64_t nsteps, uint32_t
   if (rc != HLB_OK) return rc;
   HLB_CHECK(hipStreamSynchronize(b->stream));
   HLB_CHECK(hipEventRecord(b->ev0, b->stream));
-  rc = launch_chunk(b, nsteps, props_at);
+  rc = launch_chunk(b, nsteps, props_at, replays(b, like));
   if (rc != HLB_OK) return rc;
   HLB_CHECK(hipEventRecord(b->ev1, b->stream));
   HLB_CHECK(hipEventSynchronize(b->ev1));
@@ -344,6 +349,15 @@ extern "C" int hlb_batch_step_timed(hlb_batch_handle b, int64_t nsteps, uint32_t
   HLB_CHECK(hipEventElapsedTime(&e, b->ev0, b->ev1));
   *ms = e;
   return release_members(b);
+}
+
+}  // namespace
+}  // namespace hlb
+
+extern "C" int hlb_batch_step_timed(hlb_batch_handle b, int64_t nsteps, uint32_t flags, double* ms) {
+  if (!b || !ms) return fail(HLB_EINVAL, "hlb_batch_step_timed: null argument");
+  if (nsteps < 0 || nsteps > kChunk) return fail(HLB_EINVAL, "hlb_batch_step_timed: 0 to 1024 steps per timed call");
+  return timed_steps(b, nsteps, flags, nsteps, ms);
 }
 
 // Times every launch shape on the live batch (the trial steps are real steps
@@ -357,9 +371,10 @@ extern "C" int hlb_batch_autotune(hlb_batch_handle b, int64_t trial_steps, int* 
     int rc = hlb_batch_set_variant(b, v);
     if (rc != HLB_OK) return rc;
     double ms = 0.0;
-    rc = hlb_batch_step_timed(b, trial_steps, 0, &ms);  // first call captures the graph
+    const int64_t like = std::max(trial_steps, kReplaySteps);  // what a solve's sequences run
+    rc = timed_steps(b, trial_steps, 0, like, &ms);  // the first call captures the graph
     if (rc != HLB_OK) return rc;
-    rc = hlb_batch_step_timed(b, trial_steps, 0, &ms);
+    rc = timed_steps(b, trial_steps, 0, like, &ms);
     if (rc != HLB_OK) return rc;
     if (ms < best_ms) {
       best_ms = ms;

@@ -1405,15 +1405,16 @@ extern "C" int hlb_step(hlb_handle h, int64_t nsteps, uint32_t flags) {
   return run_steps(h, nsteps, flags);
 }
 
-extern "C" int hlb_step_timed(hlb_handle h, int64_t nsteps, uint32_t flags, double* ms) {
-  if (!h || !ms) return fail(HLB_EINVAL, "hlb_step_timed: null argument");
-  if (nsteps < 0 || nsteps > kChunk) return fail(HLB_EINVAL, "hlb_step_timed: 0 to 1024 steps per timed call");
+namespace hlb {
+namespace {
+
+// nsteps timed steps, replayed from a graph or launched one by one.
+int timed_steps(hlb_lattice* h, int64_t nsteps, uint32_t flags, bool graph, double* ms) {
   if (!h->f_valid) return fail(HLB_EINVAL, "hlb_step_timed: no initial condition");
   HLB_CHECK(hipStreamSynchronize(h->stream));
   const bool props = (flags & HLB_STEP_PROPERTIES) != 0;
   int rc = stage_sequence(h, nsteps, props);
   if (rc != HLB_OK) return rc;
-  const bool graph = h->use_graph && nsteps > 0 && h->replays(nsteps);
   if (graph) {
     // Capture outside the timed region: a sequence not seen before is
     // recorded by a first call that runs nothing, then replayed below.
@@ -1429,6 +1430,15 @@ extern "C" int hlb_step_timed(hlb_handle h, int64_t nsteps, uint32_t flags, doub
   HLB_CHECK(hipEventElapsedTime(&elapsed, h->ev0, h->ev1));
   *ms = elapsed;
   return HLB_OK;
+}
+
+}  // namespace
+}  // namespace hlb
+
+extern "C" int hlb_step_timed(hlb_handle h, int64_t nsteps, uint32_t flags, double* ms) {
+  if (!h || !ms) return fail(HLB_EINVAL, "hlb_step_timed: null argument");
+  if (nsteps < 0 || nsteps > kChunk) return fail(HLB_EINVAL, "hlb_step_timed: 0 to 1024 steps per timed call");
+  return timed_steps(h, nsteps, flags, h->use_graph && nsteps > 0 && h->replays(nsteps), ms);
 }
 
 extern "C" int hlb_set_variant(hlb_handle h, int variant) {
@@ -1450,11 +1460,14 @@ extern "C" int hlb_autotune(hlb_handle h, int64_t trial_steps, int* variant, dou
   h->variant_chosen = true;
   double best_ms = 1e300;
   const int nvar = h->fp32() ? kFp32Variants : kFp64Variants;
+  // trials too short to be replayed by themselves still time what a solve's
+  // sequences run
+  const bool graph = h->use_graph && h->replays(std::max(trial_steps, kReplaySteps));
   for (int v = 0; v < nvar; ++v) {
     h->variant = v;
     double ms = 0.0;
-    int rc = hlb_step_timed(h, trial_steps, 0, &ms);  // the first launch of a shape warms it
-    if (rc == HLB_OK) rc = hlb_step_timed(h, trial_steps, 0, &ms);
+    int rc = timed_steps(h, trial_steps, 0, graph, &ms);  // the first launch of a shape warms it
+    if (rc == HLB_OK) rc = timed_steps(h, trial_steps, 0, graph, &ms);
     if (rc != HLB_OK) return rc;
     if (ms < best_ms) {
       best_ms = ms;

@@ -56,7 +56,8 @@ static_assert(sizeof(Member32) <= sizeof(double) * kStageResult, "the record fit
 // 30k sites n = 16 120 / 124, n = 300 1801 / 2021; 67k sites (~1.4k slabs) n =
 // 16 159 / 153, n = 300 2443 / 2541; 127k sites (~2.5k slabs) n = 16 197 / 190,
 // n = 300 3208 / 3218; 430k sites n = 8 226 / 217, n = 300 7471 / 7468.
-inline bool replay_pays(int64_t n, int64_t nslab) { return n >= 16 && nslab <= 2048; }
+inline constexpr int64_t kReplaySteps = 16;
+inline bool replay_pays(int64_t n, int64_t nslab) { return n >= kReplaySteps && nslab <= 2048; }
 
 inline int64_t round_up(int64_t v, int64_t m) { return (v + m - 1) / m * m; }
 

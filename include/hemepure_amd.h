@@ -220,15 +220,17 @@ int hlb_step(hlb_handle h, int64_t nsteps, uint32_t flags);
  * non-temporal stores (faster where the arrays are far larger than the
  * caches, slower where they fit the Infinity Cache).
  * No counterpart in the reference.  hlb_autotune times every variant over
- * trial_steps real steps of the lattice (they advance it) and keeps the
- * fastest; results do not depend on the variant. */
+ * trial_steps real steps of the lattice (they advance it; replayed where the
+ * lattice's long sequences are) and keeps the fastest; results do not depend on
+ * the variant. */
 int hlb_set_variant(hlb_handle h, int variant);
 int hlb_variant(hlb_handle h);
 int hlb_autotune(hlb_handle h, int64_t trial_steps, int* variant, double* ms_per_step);
 /* Like hlb_step, timing the launches with HIP events recorded on the handle's
- * stream; blocks until done and returns the elapsed milliseconds.  A step
- * sequence not seen before is captured into its graph before the first
- * event, so the timed region holds the replay only. */
+ * stream; blocks until done and returns the elapsed milliseconds.  A
+ * sequence that hlb_step would replay (hlb_set_graphs) and that was not seen
+ * before is captured ahead of the first event, so the timed region holds the
+ * replay only; any other is launched step by step within it. */
 int hlb_step_timed(hlb_handle h, int64_t nsteps, uint32_t flags, double* ms);
 /* No counterpart in the reference (its steps are host loops over site
  * ranges).  Step sequences (16 to 1024 steps) of small lattices are captured

@@ -126,3 +126,28 @@ def test_windkessel_fp32_replayed_eager_and_batched():
         assert a.captured_graphs() == 3 and b.captured_graphs() == 0
     assert batch.captured_graphs() == 3
     batch.close()
+
+
+@pytest.mark.parametrize("precision", [H.FP64, H.FP32_SHIFTED])
+def test_autotuner_times_what_a_solve_runs(precision):
+    """Trials of a small lattice are replays, whatever their length, as its solve's
+    sequences are; launched eagerly where graphs are off."""
+    case = windkessel_cylinder_case(radius=4.6, length=17, box_xy=24)
+    for graphs in (True, False):
+        lat = case.product(precision=precision)
+        lat.set_graphs(graphs)
+        lat.init_equilibrium(1.0)
+        lat.autotune(3)
+        assert lat.captured_graphs() == (8 if graphs else 0)
+        lat.step_timed(3)  # times what step(3) runs
+        assert lat.captured_graphs() == (8 if graphs else 0)
+    if precision == H.FP32_SHIFTED:
+        for graphs in (True, False):
+            members = [case.product(precision=precision) for _ in range(2)]
+            for lat in members:
+                lat.init_equilibrium(1.0)
+            batch = H.Batch(members)
+            batch.set_graphs(graphs)
+            batch.autotune(3)
+            assert batch.captured_graphs() == (1 if graphs else 0)  # the last variant's
+            batch.close()
