@@ -1456,7 +1456,9 @@ extern "C" int hlb_variant(hlb_handle h) { return h ? h->variant : -1; }
 extern "C" int hlb_autotune(hlb_handle h, int64_t trial_steps, int* variant, double* ms_per_step) {
   if (!h) return fail(HLB_EINVAL, "hlb_autotune: null handle");
   if (trial_steps < 1 || trial_steps > kChunk) return fail(HLB_EINVAL, "hlb_autotune: 1 to 1024 trial steps");
-  int best = h->variant;
+  const int before = h->variant;
+  const bool chosen = h->variant_chosen;
+  int best = before;
   h->variant_chosen = true;
   double best_ms = 1e300;
   const int nvar = h->fp32() ? kFp32Variants : kFp64Variants;
@@ -1468,7 +1470,11 @@ extern "C" int hlb_autotune(hlb_handle h, int64_t trial_steps, int* variant, dou
     double ms = 0.0;
     int rc = timed_steps(h, trial_steps, 0, graph, &ms);  // the first launch of a shape warms it
     if (rc == HLB_OK) rc = timed_steps(h, trial_steps, 0, graph, &ms);
-    if (rc != HLB_OK) return rc;
+    if (rc != HLB_OK) {
+      h->variant = before;
+      h->variant_chosen = chosen;
+      return rc;
+    }
     if (ms < best_ms) {
       best_ms = ms;
       best = v;
