@@ -17,10 +17,22 @@
 // 16 outlets 255 -> 251 us.
 //
 // FP64 form: the terms are added in the reference's site order
-// (InOutLetWK3.cc:33-52 accumulates flowRateNew += u.(-n) site by site), one
-// wavefront reading 64 at a time a chunk ahead of its chain of dependent
-// additions, about 7 ns a term.  FP32-shifted form: no order, so 256 strided
-// partial sums of four each, combined across lanes in a fixed order, in FP64.
+// (InOutLetWK3.cc:33-52 accumulates flowRateNew += u.(-n) site by site) by one
+// wavefront, a chain of dependent additions that bounds the step of a wide
+// outlet.  A term costs one broadcast within its row of 16 lanes and the
+// addition, 5.2 ns; taken from its lane through two scalar registers it cost
+// 10.1 ns, from LDS in a launch of its own 7.4 ns.  FP32-shifted form: no order,
+// so 256 strided partial sums of four each, combined across lanes in a fixed
+// order, in FP64; the one wavefront has all 16 loads of 1024 terms in flight, for
+// with four at a time a wide outlet's sum outlasted the step.
+//   us a step, outlet of 11,300 sites (0.27M-site pipe) FP64 115.5 -> 59.2,
+//   31,400 sites (0.75M) FP64 316 -> 162, FP32 50 -> 27.5; 5,000 sites FP64 56
+//   -> 33; 1,260 sites FP64 15.9 -> 8.8.
+//
+// No intrinsic with a side effect belongs here (raised wave priority): the
+// compiler takes it for a write to memory and reads the slab records of every
+// wave of the step with vector loads instead of scalar ones (FP32 ensemble 26.8
+// -> 31.2 ms a pass, 7.6M-site tree 84 -> 94).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -39,21 +51,36 @@ __device__ __forceinline__ double lane_value(double v, int lane) {
   return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
 }
 
-// 0 + t[0] + t[1] + ... + t[n - 1], in that order, by one wavefront.
+// s + v of lane 0 + v of lane 1 + ... + v of lane 15 of each lane's row of 16, in
+// that order: one broadcast within the row and one addition a term.
+template <int K = 0>
+__device__ __forceinline__ double row_chain(double s, double v) {
+  if constexpr (K < 16) return row_chain<K + 1>(s + __builtin_amdgcn_mov_dpp(v, 0x150 + K, 0xf, 0xf, true), v);
+  else return s;
+}
+
+// 0 + t[0] + t[1] + ... + t[n - 1], in that order, by one wavefront: 64 terms a
+// load, kChainAhead loads ahead of the additions.
+constexpr int kChainAhead = 4;
 __device__ __forceinline__ double chain_sum(const double* t, int n) {
   const int lane = threadIdx.x & 63;
-  double sum = 0.0;
-  double next = lane < n ? ldp(t, (uint32_t)lane) : 0.0;
-  for (int i = 0; i < n; i += 64) {
-    const double v = next;
-    if (i + 64 + lane < n) next = ldp(t, (uint32_t)(i + 64 + lane));
-    if (n - i >= 64) {
+  double ahead[kChainAhead];
 #pragma unroll
-      for (int k = 0; k < 64; ++k) sum += lane_value(v, k);
-    } else {
-      for (int k = 0; k < n - i; ++k) sum += lane_value(v, k);
-    }
+  for (int a = 0; a < kChainAhead; ++a) ahead[a] = 64 * a + lane < n ? ldp(t, (uint32_t)(64 * a + lane)) : 0.0;
+  double sum = 0.0;
+  int i = 0;
+  for (; i + 64 <= n; i += 64) {
+    const double v = ahead[0];
+#pragma unroll
+    for (int a = 1; a < kChainAhead; ++a) ahead[a - 1] = ahead[a];
+    const int e = i + 64 * kChainAhead + lane;
+    if (e < n) ahead[kChainAhead - 1] = ldp(t, (uint32_t)e);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) sum = lane_value(row_chain(sum, v), 16 * r);
   }
+  int k = 0;
+  for (; i + k + 16 <= n; k += 16) sum = lane_value(row_chain(sum, ahead[0]), k);
+  for (; i + k < n; ++k) sum += lane_value(ahead[0], k);
   return sum;
 }
 
@@ -64,22 +91,35 @@ __device__ __forceinline__ double wave_sum(double v) {
 }
 
 // The sum of t[0 .. n - 1] by one wavefront, as four wavefronts of strided
-// shares would form it.
+// shares with four partial sums a lane would form it; all 16 loads of a round are
+// in flight together.
 __device__ __forceinline__ double tree_sum(const double* t, int n) {
   constexpr int T = 256;
+  const int lane = threadIdx.x & 63;
+  double p[4][4] = {};
+  int base = 0;
+  for (; base + 4 * T <= n; base += 4 * T) {
+    double v[4][4];
+#pragma unroll
+    for (int w = 0; w < 4; ++w)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) v[w][k] = ldp(t, (uint32_t)(base + k * T + 64 * w + lane));
+#pragma unroll
+    for (int w = 0; w < 4; ++w)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) p[w][k] += v[w][k];
+  }
   double part[4];
 #pragma unroll
   for (int w = 0; w < 4; ++w) {
-    double p0 = 0.0, p1 = 0.0, p2 = 0.0, p3 = 0.0;
-    int e = 64 * w + (int)(threadIdx.x & 63);
-    for (; e + 3 * T < n; e += 4 * T) {
-      p0 += ldp(t, (uint32_t)e);
-      p1 += ldp(t, (uint32_t)(e + T));
-      p2 += ldp(t, (uint32_t)(e + 2 * T));
-      p3 += ldp(t, (uint32_t)(e + 3 * T));
+    int e = base + 64 * w + lane;
+    if (e + 3 * T < n) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) p[w][k] += ldp(t, (uint32_t)(e + k * T));
+      e += 4 * T;
     }
-    for (; e < n; e += T) p0 += ldp(t, (uint32_t)e);
-    part[w] = wave_sum((p0 + p1) + (p2 + p3));
+    for (; e < n; e += T) p[w][0] += ldp(t, (uint32_t)e);
+    part[w] = wave_sum((p[w][0] + p[w][1]) + (p[w][2] + p[w][3]));
   }
   return 0.0 + ((part[0] + part[1]) + (part[2] + part[3]));
 }
