@@ -248,6 +248,32 @@ bool sections_pay(int64_t sites, bool fp32) {
   return bytes > kInfinityCacheBytes / 4 && bytes <= kInfinityCacheBytes;
 }
 
+// m's positions moved by BY, for those that stay within the slab.
+template <int BY>
+uint64_t moved(uint64_t m) {
+  if constexpr (BY >= 64 || BY <= -64) return 0;
+  else if constexpr (BY >= 0) return m >> BY;
+  else return m << -BY;
+}
+
+// Fluid upstream positions of a slab's sites in directions J and up, from the
+// masks of the reachable slabs (upstream_pos on the host).
+template <int J = 1>
+int fluid_neighbours(const SlabRec& R) {
+  if constexpr (J == Q) {
+    return 0;
+  } else {
+    constexpr int ox = -CX[J], oy = -CY[J], oz = -CZ[J], by = 8 * oy + oz;
+    constexpr uint64_t Y = oy == 0 ? 0 : oy > 0 ? 0xffull << 56 : 0xffull;
+    constexpr uint64_t Z = oz == 0 ? 0 : oz > 0 ? 0x8080808080808080ull : 0x0101010101010101ull;
+    uint64_t f = moved<by>(R.fm[reach_entry(ox, 0, 0)]) & ~(Y | Z);
+    if constexpr (oy != 0) f |= moved<by - 64 * oy>(R.fm[reach_entry(ox, oy, 0)]) & Y & ~Z;
+    if constexpr (oz != 0) f |= moved<by - 8 * oz>(R.fm[reach_entry(ox, 0, oz)]) & Z & ~Y;
+    if constexpr (oy != 0 && oz != 0) f |= moved<by - 64 * oy - 8 * oz>(R.fm[reach_entry(ox, oy, oz)]) & Y & Z;
+    return __builtin_popcountll(f & R.fm[reach_entry(0, 0, 0)]) + fluid_neighbours<J + 1>(R);
+  }
+}
+
 void device_order(hlb_lattice* h, int order) {
   const HostLattice& L = h->L;
   const int64_t N = L.N;
@@ -379,7 +405,12 @@ void device_order(hlb_lattice* h, int order) {
   }
   h->bsite.resize((size_t)firstB.back());
   h->isite.resize((size_t)firstI.back());
+  // fluid neighbours of all sites: as many as plain links, unless wall or iolet
+  // links lead to fluid sites (counted here, 64 sites at a time, because the same
+  // test per link takes 7% of hlb_create)
+  std::atomic<int64_t> neighbours{0};
   parallel_ranges(h->nslab, [&](int, int64_t lo, int64_t hi) {
+    int64_t count = 0;
     for (int64_t r = lo; r < hi; ++r) {
       const int64_t k = h->h_slab[r] >> 3;
       const int x = h->h_slab[r] & 7;
@@ -410,8 +441,11 @@ void device_order(hlb_lattice* h, int order) {
         }
         if (site >= L.off[2]) h->isite[(size_t)ni++] = site;
       }
+      count += fluid_neighbours(R);
     }
+    neighbours.fetch_add(count, std::memory_order_relaxed);
   }, kSlabGrain);
+  if (neighbours.load() != (Q - 1) * N - L.links) mark_inner_links(h->L);
   h->NB = (int64_t)h->bsite.size();
   h->NI = (int64_t)h->isite.size();
   h->SB = round_up(std::max<int64_t>(h->NB, 1), 64);

@@ -147,9 +147,9 @@ int build_lattice(const hlb_geometry& g, HostLattice& L) {
     std::fill(cellInput.begin() + lo * spb, cellInput.begin() + hi * spb, -1);
   }, slotGrain);
   parallel_ranges(n, [&](int, int64_t lo, int64_t hi) {
-    const int32_t b = (int32_t)bs;
+    const uint32_t b = (uint32_t)bs;
     for (int64_t i = lo; i < hi; ++i) {
-      const int32_t x = g.coords[3 * i], y = g.coords[3 * i + 1], z = g.coords[3 * i + 2];
+      const uint32_t x = g.coords[3 * i], y = g.coords[3 * i + 1], z = g.coords[3 * i + 2];  // checked: not negative
       const int64_t slot = L.blockSlot[(size_t)(((x / b) * BY + (y / b)) * BZ + (z / b))];
       int32_t* cell = &cellInput[(size_t)(slot * spb + cell_in_block(x, y, z, b))];
       if (__atomic_exchange_n(cell, (int32_t)i, __ATOMIC_RELAXED) >= 0) {
@@ -169,7 +169,9 @@ int build_lattice(const hlb_geometry& g, HostLattice& L) {
   ioletId.resize((size_t)n);
   type.resize((size_t)n);
   cls.resize((size_t)n);
+  std::atomic<int64_t> links{0};
   parallel_ranges(n, [&](int, int64_t lo, int64_t hi) {
+    int64_t count = 0;
     for (int64_t i = lo; i < hi; ++i) {
       bool hadInlet = false, hadOutlet = false;
       uint32_t w = 0, io = 0;
@@ -177,6 +179,7 @@ int build_lattice(const hlb_geometry& g, HostLattice& L) {
       for (int d = 1; d < Q; ++d) {
         const uint8_t t = g.link_type[i * 18 + d - 1];
         if (t == HLB_LINK_NONE) continue;
+        ++count;
         if (t > HLB_LINK_OUTLET) {
           bad.store(true, std::memory_order_relaxed);
           return;
@@ -196,8 +199,10 @@ int build_lattice(const hlb_geometry& g, HostLattice& L) {
       const bool wl = w != 0;
       cls[i] = type[i] == kFluidType ? (wl ? 1 : 0) : type[i] == kInletType ? (wl ? 4 : 2) : (wl ? 5 : 3);
     }
+    links.fetch_add(count, std::memory_order_relaxed);
   });
   if (bad.load()) return fail(HLB_EGEOMETRY, "hlb_create: unknown link type");
+  L.links = links.load();
 
   // Class-major contiguous order: per block and class the first index, then
   // every cell's.  cellLinks: a cell's wall and iolet links, bit 31 where it is
@@ -261,9 +266,7 @@ int build_lattice(const hlb_geometry& g, HostLattice& L) {
 
   // The one-writer check, cell by cell: a plain link's neighbour must be
   // fluid with a plain link back, any other link's must not push here.
-  std::atomic<bool> inner{false};
   parallel_ranges(nslot, [&](int, int64_t lo, int64_t hi) {
-    uint32_t found = 0;  // what lies beyond wall and iolet links
     for (int64_t s = lo; s < hi; ++s) {
       const int64_t b = slotBlock[(size_t)s], bx = b / (BY * BZ), by = (b / BZ) % BY, bz = b % BZ;
       const uint32_t* around[27];  // the 3 x 3 x 3 blocks' cells
@@ -304,26 +307,24 @@ int build_lattice(const hlb_geometry& g, HostLattice& L) {
             bad.store(true, std::memory_order_relaxed);
             return;
           }
-          found |= plain ? 0 : src;
         }
       }
     }
-    if (found & kFluid) inner.store(true, std::memory_order_relaxed);
   }, slotGrain);
-  if (bad.load()) return one_writer_error(L);
-  if (inner.load()) {
-    L.inner.resize((size_t)n);
-    parallel_ranges(n, [&](int, int64_t lo, int64_t hi) {
-      for (int64_t k = lo; k < hi; ++k) {
-        L.inner[(size_t)k] = 0;
-        for (int d = 1; d < Q; ++d)
-          if (link_of(L, k, d) != HLB_LINK_NONE &&
-              L.site_at(L.coords[3 * k] + CX[d], L.coords[3 * k + 1] + CY[d], L.coords[3 * k + 2] + CZ[d]) >= 0)
-            L.inner[(size_t)k] |= 1u << (d - 1);
-      }
-    });
-  }
-  return HLB_OK;
+  return bad.load() ? one_writer_error(L) : HLB_OK;
+}
+
+void mark_inner_links(HostLattice& L) {
+  L.inner.resize((size_t)L.N);
+  parallel_ranges(L.N, [&](int, int64_t lo, int64_t hi) {
+    for (int64_t k = lo; k < hi; ++k) {
+      L.inner[(size_t)k] = 0;
+      for (int d = 1; d < Q; ++d)
+        if (link_of(L, k, d) != HLB_LINK_NONE &&
+            L.site_at(L.coords[3 * k] + CX[d], L.coords[3 * k + 1] + CY[d], L.coords[3 * k + 2] + CZ[d]) >= 0)
+          L.inner[(size_t)k] |= 1u << (d - 1);
+    }
+  });
 }
 
 void pull_table(const HostLattice& L, uint32_t* out) {

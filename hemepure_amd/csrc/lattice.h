@@ -30,8 +30,9 @@ struct HostLattice {
   RawVector<uint32_t> iolet;   // N, bit d-1 set for an inlet/outlet link d
   RawVector<int32_t> ioletId;  // N
   RawVector<int32_t> siteType; // N
+  int64_t links = 0;           // wall and iolet links, all sites
   // N, bit d-1 set for a wall or iolet link d that leads to a fluid site; empty
-  // when no link does.
+  // when no link does (mark_inner_links).
   RawVector<uint32_t> inner;
   RawVector<float> q;          // N*18 link distances as read
   RawVector<float> nrm;        // N*3 wall normal normalised in float (+inf if none)
@@ -45,6 +46,9 @@ struct HostLattice {
 
 // Builds the lattice; returns HLB_OK or an HLB_E* code with hlb_last_error set.
 int build_lattice(const hlb_geometry& g, HostLattice& L);
+
+// Fills L.inner.
+void mark_inner_links(HostLattice& L);
 
 // The pull table, 18*N: source of direction j = 1..18, or the site itself.
 void pull_table(const HostLattice& L, uint32_t* out);
