@@ -139,19 +139,25 @@ int build_lattice(const hlb_geometry& g, HostLattice& L) {
       L.blockSlot[(size_t)b] = (int64_t)slotBlock.size();
       slotBlock.push_back(b);
     }
-  const int64_t nslot = (int64_t)slotBlock.size();
-  const int64_t slotGrain = std::max<int64_t>(1, kGrain / spb);
+  const int64_t nslot = (int64_t)slotBlock.size(), cells = nslot * spb;
+  // Cells are shared out in parts of `per`: whole blocks, or the x layers of large
+  // ones, of which there may be few.
+  const int64_t per = spb > 4096 ? bs * bs : spb, parts = cells / per;
+  const bool sparse = n * 32 < cells;  // the work is by sites, where cells need not be looked at
+  const int64_t partGrain = std::max<int64_t>(1, (sparse ? 16 * kGrain : kGrain) / per);
   RawVector<int32_t> cellInput;
-  cellInput.resize((size_t)(nslot * spb));
-  parallel_ranges(nslot, [&](int, int64_t lo, int64_t hi) {
-    std::fill(cellInput.begin() + lo * spb, cellInput.begin() + hi * spb, -1);
-  }, slotGrain);
-  parallel_ranges(n, [&](int, int64_t lo, int64_t hi) {
+  cellInput.resize((size_t)cells);
+  parallel_ranges(parts, [&](int, int64_t lo, int64_t hi) {
+    std::fill(cellInput.begin() + lo * per, cellInput.begin() + hi * per, -1);
+  }, partGrain);
+  auto cell_of = [&](int64_t i) {
     const uint32_t b = (uint32_t)bs;
+    const uint32_t x = g.coords[3 * i], y = g.coords[3 * i + 1], z = g.coords[3 * i + 2];  // checked: not negative
+    return L.blockSlot[(size_t)(((x / b) * BY + (y / b)) * BZ + (z / b))] * spb + cell_in_block(x, y, z, b);
+  };
+  parallel_ranges(n, [&](int, int64_t lo, int64_t hi) {
     for (int64_t i = lo; i < hi; ++i) {
-      const uint32_t x = g.coords[3 * i], y = g.coords[3 * i + 1], z = g.coords[3 * i + 2];  // checked: not negative
-      const int64_t slot = L.blockSlot[(size_t)(((x / b) * BY + (y / b)) * BZ + (z / b))];
-      int32_t* cell = &cellInput[(size_t)(slot * spb + cell_in_block(x, y, z, b))];
+      int32_t* cell = &cellInput[(size_t)cell_of(i)];
       if (__atomic_exchange_n(cell, (int32_t)i, __ATOMIC_RELAXED) >= 0) {
         bad.store(true, std::memory_order_relaxed);
         return;
@@ -204,21 +210,25 @@ int build_lattice(const hlb_geometry& g, HostLattice& L) {
   if (bad.load()) return fail(HLB_EGEOMETRY, "hlb_create: unknown link type");
   L.links = links.load();
 
-  // Class-major contiguous order: per block and class the first index, then
+  // Class-major contiguous order: per part and class the first index, then
   // every cell's.  cellLinks: a cell's wall and iolet links, bit 31 where it is
-  // fluid.
+  // fluid, for the check by blocks.
   constexpr uint32_t kFluid = 1u << 31;
-  std::vector<int64_t> next((size_t)nslot * 6, 0);
-  parallel_ranges(nslot, [&](int, int64_t lo, int64_t hi) {
-    for (int64_t s = lo; s < hi; ++s)
-      for (int64_t c = s * spb; c < (s + 1) * spb; ++c)
-        if (cellInput[(size_t)c] >= 0) next[(size_t)(s * 6 + cls[(size_t)cellInput[(size_t)c]])]++;
-  }, slotGrain);
+  const bool by_block = spb > 1 && !sparse;
+  std::vector<int64_t> next((size_t)parts * 6, 0);
+  if (sparse)
+    for (int64_t i = 0; i < n; ++i) next[(size_t)(cell_of(i) / per * 6 + cls[(size_t)i])]++;
+  else
+    parallel_ranges(parts, [&](int, int64_t lo, int64_t hi) {
+      for (int64_t s = lo; s < hi; ++s)
+        for (int64_t c = s * per; c < (s + 1) * per; ++c)
+          if (cellInput[(size_t)c] >= 0) next[(size_t)(s * 6 + cls[(size_t)cellInput[(size_t)c]])]++;
+    }, partGrain);
   L.N = n;
   int64_t k = 0;
   for (int c = 0; c < 6; ++c) {
     L.off[c] = k;
-    for (int64_t s = 0; s < nslot; ++s) {
+    for (int64_t s = 0; s < parts; ++s) {
       const int64_t count = next[(size_t)(s * 6 + c)];
       next[(size_t)(s * 6 + c)] = k;
       k += count;
@@ -226,8 +236,8 @@ int build_lattice(const hlb_geometry& g, HostLattice& L) {
   }
   L.off[6] = k;
   RawVector<uint32_t> cellLinks;
-  cellLinks.resize((size_t)(nslot * spb));
-  L.slotSites.resize((size_t)(nslot * spb));
+  if (by_block) cellLinks.resize((size_t)cells);
+  L.slotSites.resize((size_t)cells);
   L.coords.resize((size_t)n * 3);
   L.wall.resize((size_t)n);
   L.iolet.resize((size_t)n);
@@ -235,18 +245,18 @@ int build_lattice(const hlb_geometry& g, HostLattice& L) {
   L.siteType.resize((size_t)n);
   L.q.resize((size_t)n * 18);
   L.nrm.resize((size_t)n * 3);
-  parallel_ranges(nslot, [&](int, int64_t lo, int64_t hi) {
+  parallel_ranges(parts, [&](int, int64_t lo, int64_t hi) {
     for (int64_t s = lo; s < hi; ++s)
-      for (int64_t c = s * spb; c < (s + 1) * spb; ++c) {
+      for (int64_t c = s * per; c < (s + 1) * per; ++c) {
         const int64_t i = cellInput[(size_t)c];
         if (i < 0) {
           L.slotSites[(size_t)c] = -1;
-          cellLinks[(size_t)c] = 0;
+          if (by_block) cellLinks[(size_t)c] = 0;
           continue;
         }
         const int64_t to = next[(size_t)(s * 6 + cls[(size_t)i])]++;
         L.slotSites[(size_t)c] = (int32_t)to;
-        cellLinks[(size_t)c] = wall[(size_t)i] | iol[(size_t)i] | kFluid;
+        if (by_block) cellLinks[(size_t)c] = wall[(size_t)i] | iol[(size_t)i] | kFluid;
         for (int a = 0; a < 3; ++a) L.coords[(size_t)(3 * to + a)] = g.coords[3 * i + a];
         L.wall[(size_t)to] = wall[(size_t)i];
         L.iolet[(size_t)to] = iol[(size_t)i];
@@ -262,13 +272,36 @@ int build_lattice(const hlb_geometry& g, HostLattice& L) {
         }
         for (int a = 0; a < 3; ++a) L.nrm[(size_t)(3 * to + a)] = v[a];
       }
-  }, slotGrain);
+  }, partGrain);
 
-  // The one-writer check, cell by cell: a plain link's neighbour must be
-  // fluid with a plain link back, any other link's must not push here.
-  parallel_ranges(nslot, [&](int, int64_t lo, int64_t hi) {
+  // The one-writer check: a plain link's neighbour must be fluid with a plain
+  // link back, any other link's must not push here.  Cell by cell with the blocks
+  // around found once, unless a block is one cell or blocks are mostly empty.
+  auto mismatch = [](uint32_t here, uint32_t src, int j) {
+    const bool plain = !((here >> (INV[j] - 1)) & 1u);
+    const bool srcPushes = (src & kFluid) && !((src >> (j - 1)) & 1u);
+    return plain != srcPushes;
+  };
+  if (!by_block) {
+    parallel_ranges(n, [&](int, int64_t lo, int64_t hi) {
+      for (int64_t k = lo; k < hi; ++k) {
+        const int64_t x = L.coords[3 * k], y = L.coords[3 * k + 1], z = L.coords[3 * k + 2];
+        const uint32_t here = L.wall[(size_t)k] | L.iolet[(size_t)k];
+        for (int j = 1; j < Q; ++j) {
+          const int64_t s = L.site_at(x - CX[j], y - CY[j], z - CZ[j]);
+          if (mismatch(here, s < 0 ? 0 : L.wall[(size_t)s] | L.iolet[(size_t)s] | kFluid, j)) {
+            bad.store(true, std::memory_order_relaxed);
+            return;
+          }
+        }
+      }
+    });
+    return bad.load() ? one_writer_error(L) : HLB_OK;
+  }
+  parallel_ranges(parts, [&](int, int64_t lo, int64_t hi) {
     for (int64_t s = lo; s < hi; ++s) {
-      const int64_t b = slotBlock[(size_t)s], bx = b / (BY * BZ), by = (b / BZ) % BY, bz = b % BZ;
+      const int64_t first = s * per % spb;  // of the block's cells
+      const int64_t b = slotBlock[(size_t)(s * per / spb)], bx = b / (BY * BZ), by = (b / BZ) % BY, bz = b % BZ;
       const uint32_t* around[27];  // the 3 x 3 x 3 blocks' cells
       for (int e = 0; e < 27; ++e) {
         const int64_t x = bx + e / 9 - 1, y = by + (e / 3) % 3 - 1, z = bz + e % 3 - 1;
@@ -277,40 +310,40 @@ int build_lattice(const hlb_geometry& g, HostLattice& L) {
         around[e] = t < 0 ? nullptr : &cellLinks[(size_t)(t * spb)];
       }
       const uint32_t* own = around[13];
-      for (int64_t c = 0; c < spb; ++c) {
-        const uint32_t here = own[c];
-        if (!(here & kFluid)) continue;
-        const int64_t x = c / (bs * bs), y = (c / bs) % bs, z = c % bs;
-        const bool inner = x > 0 && y > 0 && z > 0 && x < bs - 1 && y < bs - 1 && z < bs - 1;
-        for (int j = 1; j < Q; ++j) {
-          uint32_t src = 0;
-          if (inner) {
-            src = own[c - ((CX[j] * bs + CY[j]) * bs + CZ[j])];
-          } else {
-            int64_t p[3] = {x - CX[j], y - CY[j], z - CZ[j]};
-            int e = 13;
-            const int step[3] = {9, 3, 1};
-            for (int a = 0; a < 3; ++a) {
-              if (p[a] < 0) {
-                p[a] += bs;
-                e -= step[a];
-              } else if (p[a] >= bs) {
-                p[a] -= bs;
-                e += step[a];
+      for (int64_t x = first / (bs * bs); x < (first + per) / (bs * bs); ++x)
+        for (int64_t y = 0; y < bs; ++y)
+          for (int64_t z = 0; z < bs; ++z) {
+            const int64_t c = (x * bs + y) * bs + z;
+            const uint32_t here = own[c];
+            if (!(here & kFluid)) continue;
+            const bool inner = x > 0 && y > 0 && z > 0 && x < bs - 1 && y < bs - 1 && z < bs - 1;
+            for (int j = 1; j < Q; ++j) {
+              uint32_t src = 0;
+              if (inner) {
+                src = own[c - ((CX[j] * bs + CY[j]) * bs + CZ[j])];
+              } else {
+                int64_t p[3] = {x - CX[j], y - CY[j], z - CZ[j]};
+                int e = 13;
+                const int step[3] = {9, 3, 1};
+                for (int a = 0; a < 3; ++a) {
+                  if (p[a] < 0) {
+                    p[a] += bs;
+                    e -= step[a];
+                  } else if (p[a] >= bs) {
+                    p[a] -= bs;
+                    e += step[a];
+                  }
+                }
+                if (around[e]) src = around[e][(p[0] * bs + p[1]) * bs + p[2]];
+              }
+              if (mismatch(here, src, j)) {
+                bad.store(true, std::memory_order_relaxed);
+                return;
               }
             }
-            if (around[e]) src = around[e][(p[0] * bs + p[1]) * bs + p[2]];
           }
-          const bool plain = !((here >> (INV[j] - 1)) & 1u);
-          const bool srcPushes = (src & kFluid) && !((src >> (j - 1)) & 1u);
-          if (plain != srcPushes) {
-            bad.store(true, std::memory_order_relaxed);
-            return;
-          }
-        }
-      }
     }
-  }, slotGrain);
+  }, partGrain);
   return bad.load() ? one_writer_error(L) : HLB_OK;
 }
 
