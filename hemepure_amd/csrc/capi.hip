@@ -1627,7 +1627,7 @@ extern "C" int hlb_monitor(hlb_handle h, double out[4]) {
   // into pinned host memory
   volatile double* arrived = h->result() + 4;
   *arrived = h->nslab > 0 ? 0.0 : 1.0;
-  HLB_CHECK(launch_monitor(h->tables(), h->rho.p, h->u.p, h->S, h->mon_scratch.p, h->result(), h->stream));
+  HLB_CHECK(launch_monitor(h->tables(), h->rho.p, h->u.p, h->S, h->mon_scratch.p, h->result(), true, h->stream));
   const auto start = std::chrono::steady_clock::now();
   while (*arrived == 0.0 && std::chrono::steady_clock::now() - start < kMonitorPoll) {
   }
@@ -1801,7 +1801,7 @@ extern "C" int hlb_monitor_noalloc(hlb_handle h, double out[4]) {
   int rc = scratch_ptr(h->device, &base);
   if (rc == HLB_OK) {
     double* dout = reinterpret_cast<double*>(base + kScratchOut);
-    hipError_t e = launch_monitor(h->tables(), h->rho.p, h->u.p, h->S, base, dout, h->stream);
+    hipError_t e = launch_monitor(h->tables(), h->rho.p, h->u.p, h->S, base, dout, false, h->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(out, dout, 4 * sizeof(double), hipMemcpyDeviceToHost, h->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
     if (e != hipSuccess) rc = dev_fail(e, "hlb_monitor_noalloc");

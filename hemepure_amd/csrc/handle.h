@@ -23,7 +23,7 @@ hipError_t launch_gzs_fp32(const Member32* members, const GzsLink* links, int n,
 hipError_t launch_upstream_table(const BrickTables& bt, uint32_t* out, int64_t S, hipStream_t s);
 size_t monitor_scratch(int64_t nslab);
 hipError_t launch_monitor(const BrickTables& bt, const double* rho, const double* u, int64_t S, void* scratch,
-                          double* out, hipStream_t s);
+                          double* out, bool signal, hipStream_t s);
 hipError_t launch_gather_fp64(const StepArgs& a, double* F, int64_t S, hipStream_t s);
 hipError_t launch_stress_fp64(const StepArgs& a, int kernel, const void* F, bool fp32, double* out, hipStream_t s);
 hipError_t launch_fill_fp64(double* F, int64_t N, int64_t S, const double* vals, hipStream_t s);

@@ -569,7 +569,8 @@ __global__ __launch_bounds__(kBlock) void monitor_pass1(BrickTables bt, const do
   }
 }
 
-__global__ __launch_bounds__(kBlock) void monitor_pass2(const Mon* __restrict__ partial, int n, double* __restrict__ out) {
+__global__ __launch_bounds__(kBlock) void monitor_pass2(const Mon* __restrict__ partial, int n, double* __restrict__ out,
+                                                        bool signal) {
   __shared__ Mon w[kBlock / 64];
   Mon m{DBL_MAX, -DBL_MAX, 0.0, 0.0};
   // each lane folds a contiguous run, in order
@@ -585,8 +586,9 @@ __global__ __launch_bounds__(kBlock) void monitor_pass2(const Mon* __restrict__ 
     out[1] = t.hi;
     out[2] = t.umax;
     out[3] = t.mass;
-    // a host that sees out[4] set has the four before it
-    __hip_atomic_store(out + 4, 1.0, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    // a host that sees out[4] set has the four before it (0.5 us, which a caller
+    // that waits for the stream need not spend)
+    if (signal) __hip_atomic_store(out + 4, 1.0, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
 
@@ -753,12 +755,12 @@ hipError_t launch_upstream_table(const BrickTables& bt, uint32_t* out, int64_t S
 size_t monitor_scratch(int64_t nslab) { return sizeof(Mon) * std::max<size_t>(1, slab_grid(nslab)); }
 
 hipError_t launch_monitor(const BrickTables& bt, const double* rho, const double* u, int64_t S, void* scratch,
-                          double* out, hipStream_t s) {
+                          double* out, bool signal, hipStream_t s) {
   if (bt.nslab <= 0) return hipSuccess;
   const unsigned grid = slab_grid(bt.nslab);
   Mon* part = static_cast<Mon*>(scratch);
   hipLaunchKernelGGL(monitor_pass1, dim3(grid), dim3(kBlock), 0, s, bt, rho, u, S, part);
-  hipLaunchKernelGGL(monitor_pass2, dim3(1), dim3(kBlock), 0, s, part, (int)grid, out);
+  hipLaunchKernelGGL(monitor_pass2, dim3(1), dim3(kBlock), 0, s, part, (int)grid, out, signal);
   return hipGetLastError();
 }
 
