@@ -6,9 +6,10 @@
 // launch per time step: the launch walks a member table (Member32, one record
 // per member with its plane pointers, tau and boundary selection) and a
 // tile -> member map, so members can join and leave between calls without
-// copying any lattice.  Windkessel iolets of all members are served by one
-// pair of per-step launches.  Sequences of steps are captured once into a
-// hipGraph per (member set, length, property flag) and replayed.
+// copying any lattice.  The Windkessel iolets of all members ride in the step
+// launch (windkessel.h).  Sequences of 16 steps and more over at most 2048 slabs
+// (replay_pays) are captured once into a hipGraph per (member set, length,
+// property flag) and replayed; others are launched step by step.
 //
 // Every member computes exactly what it computes alone: the per-site
 // arithmetic does not depend on the table, the tile size or the order.

@@ -210,7 +210,11 @@ int hlb_step(hlb_handle h, int64_t nsteps, uint32_t flags);
  * a batch) reports variant 1, or its non-temporal-store twin (FP64 55, FP32
  * 109) while its distributions exceed the 256 MB Infinity Cache, and is
  * launched in the shape that fits their size: variant 5 while they fit the
- * cache, 55 / 109 up to 2.5 times its size (a batch 182), 92 / 182 beyond.  FP64 36..53 = block + 3 * level with
+ * cache, 55 / 109 up to 2.5 times its size (a batch 182), 92 / 182 beyond.
+ * Setting the reported variant launches that variant itself.  FP32 lattices with
+ * wall or iolet links between two fluid sites, and batches that hold one, are
+ * launched in variant 5's shape with the set or default one's store policy.
+ * FP64 36..53 = block + 3 * level with
  * block 0..2 = 128/256/64 slots in the XCD-chunk order (chunks of 32
  * workgroup tiles dealt to the XCDs in turn).  The FP32-shifted form takes
  * 0..35, 36..71 = 0..35 with two consecutive slabs per wavefront (both
@@ -236,8 +240,9 @@ int hlb_step_timed(hlb_handle h, int64_t nsteps, uint32_t flags, double* ms);
  * ranges).  Step sequences (16 to 1024 steps) of small lattices are captured
  * into HIP graphs on first use and replayed (the default, enable = 1), so they
  * are not bound by per-launch cost; short sequences and lattices whose steps
- * hide it, and with enable = 0 every sequence, are launched step by step.  Results are bit-identical either way.  Changing it, or tau via
- * hlb_set_params, drops the captured graphs. */
+ * hide it, and with enable = 0 every sequence, are launched step by step.
+ * Results are bit-identical either way.  Changing it, or tau via hlb_set_params,
+ * drops the captured graphs. */
 int hlb_set_graphs(hlb_handle h, int enable);
 /* Captured sequences the handle holds (at most 8), -1 for a null handle. */
 int hlb_captured_graphs(hlb_handle h);
