@@ -347,7 +347,10 @@ int export_sites(hlb_lattice* h, const TransferPart* parts, int count, bool shif
       row += parts[i].planes;
       widest = std::max<int64_t>(widest, parts[i].planes);
     }
-  if (N == 0 || np == 0) return HLB_OK;
+  if (N == 0 || np == 0) {
+    HLB_CHECK(hipStreamSynchronize(h->stream));
+    return HLB_OK;
+  }
   const int64_t per = (int64_t)(kSlotBytes / sizeof(double)) / row / 64 * 64;
   const int64_t chunks = (N + per - 1) / per;
   auto start = [&](char* slot, int64_t c) -> int {
