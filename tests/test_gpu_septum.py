@@ -107,6 +107,17 @@ def test_fp64_bitwise(name, wall_bc, general, monkeypatch):
             assert np.array_equal(got, want, equal_nan=True)
 
 
+@pytest.mark.parametrize("name", ["face", "mixed"])
+def test_neighbour_tables(name):
+    """The table from the device names the site itself for such links, as the host's does."""
+    case = _case(name, H.WALL_BFL)
+    lat = case.product()
+    push, pull = lat.neighbour_tables()
+    lat.init_equilibrium(1.0)
+    dpush, dpull = lat.neighbour_tables()
+    assert np.array_equal(push, dpush) and np.array_equal(pull, dpull)
+
+
 @pytest.mark.parametrize("wall_bc", [H.WALL_SBB, H.WALL_BFL])
 @pytest.mark.parametrize("name", NAMES)
 def test_fp32(name, wall_bc):
