@@ -118,10 +118,11 @@ int rebuild(hlb_batch* b) {
   b->grid = (uint32_t)map.size();
   HLB_CHECK(b->wg_member.alloc(std::max<size_t>(1, map.size())));
   if (!map.empty())
-    HLB_CHECK(hipMemcpy(b->wg_member.p, map.data(), sizeof(int32_t) * map.size(), hipMemcpyHostToDevice));
+    HLB_CHECK(copy_now(b->wg_member.p, map.data(), sizeof(int32_t) * map.size(), hipMemcpyHostToDevice, b->stream));
   b->nwk = (int)refs.size();
   HLB_CHECK(b->refs.alloc(std::max<size_t>(1, refs.size())));
-  if (!refs.empty()) HLB_CHECK(hipMemcpy(b->refs.p, refs.data(), sizeof(WkRef) * refs.size(), hipMemcpyHostToDevice));
+  if (!refs.empty())
+    HLB_CHECK(copy_now(b->refs.p, refs.data(), sizeof(WkRef) * refs.size(), hipMemcpyHostToDevice, b->stream));
   const size_t need = std::max<size_t>(1, b->members.size());
   if (b->h_mem_cap < need) {
     if (b->h_mem) HLB_CHECK(hipHostFree(b->h_mem));

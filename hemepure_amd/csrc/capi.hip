@@ -622,12 +622,12 @@ int upload_sponge(hlb_lattice* h) {
   if (h->sponge_life <= 0 || h->h_vtau.empty()) return HLB_OK;
   const size_t S = (size_t)h->S;
   HLB_CHECK(h->vtau64.alloc(S));
-  HLB_CHECK(hipMemcpy(h->vtau64.p, h->h_vtau.data(), sizeof(double) * S, hipMemcpyHostToDevice));
+  HLB_CHECK(copy_now(h->vtau64.p, h->h_vtau.data(), sizeof(double) * S, hipMemcpyHostToDevice, h->stream));
   if (h->fp32()) {
     std::vector<float> v(S);
     for (size_t i = 0; i < S; ++i) v[i] = (float)h->h_vtau[i];
     HLB_CHECK(h->vtau32.alloc(S));
-    HLB_CHECK(hipMemcpy(h->vtau32.p, v.data(), sizeof(float) * S, hipMemcpyHostToDevice));
+    HLB_CHECK(copy_now(h->vtau32.p, v.data(), sizeof(float) * S, hipMemcpyHostToDevice, h->stream));
   }
   return HLB_OK;
 }
@@ -746,8 +746,8 @@ int upload_lattice(hlb_lattice* h) {
                                         (int32_t)h->row(), h->fp32() ? 0 : 1, 0});
     if (!h->wk_refs_host.empty()) {
       HLB_CHECK(h->wk_refs.alloc(h->wk_refs_host.size()));
-      HLB_CHECK(hipMemcpy(h->wk_refs.p, h->wk_refs_host.data(), sizeof(WkRef) * h->wk_refs_host.size(),
-                          hipMemcpyHostToDevice));
+      HLB_CHECK(copy_now(h->wk_refs.p, h->wk_refs_host.data(), sizeof(WkRef) * h->wk_refs_host.size(),
+                         hipMemcpyHostToDevice, h->stream));
     }
   }
   {
@@ -1729,8 +1729,7 @@ extern "C" int hlb_iolet_state(hlb_handle h, int outlet, int index, double out[4
   const HostIolet& io = h->iolets[g];
   if (io.IsWK() && h->device_ready) {
     WkIolet w;
-    HLB_CHECK(hipStreamSynchronize(h->stream));
-    HLB_CHECK(hipMemcpy(&w, h->wk.p + g, sizeof(WkIolet), hipMemcpyDeviceToHost));
+    HLB_CHECK(copy_now(&w, h->wk.p + g, sizeof(WkIolet), hipMemcpyDeviceToHost, h->stream));
     out[0] = w.density;
     out[1] = w.densityNew;
     out[2] = w.flowRate;

@@ -141,6 +141,13 @@ class DevPack {
   std::vector<Item> items_;
 };
 
+// Blocking copy in s's order.  Not hipMemcpy: that runs on the legacy stream, which
+// fails, and breaks the capture, while any other thread captures a graph.
+inline hipError_t copy_now(void* dst, const void* src, size_t bytes, hipMemcpyKind kind, hipStream_t s) {
+  const hipError_t e = hipMemcpyAsync(dst, src, bytes, kind, s);
+  return e == hipSuccess ? hipStreamSynchronize(s) : e;
+}
+
 inline int dev_fail(hipError_t e, const char* what) {
   return fail(HLB_EDEVICE, std::string(what) + ": " + hipGetErrorString(e));
 }

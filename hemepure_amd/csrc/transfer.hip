@@ -277,9 +277,13 @@ int take_lane(int device, size_t doubles, HostLane& out) {
 
 void give_lane(HostLane& lane) {
   if (!lane.stream) return;
+  // a stream whose capture went wrong would fail in the lattice that gets it next
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  const bool usable = hipStreamIsCapturing(lane.stream, &status) == hipSuccess && status == hipStreamCaptureStatusNone &&
+                      hipStreamQuery(lane.stream) == hipSuccess;
   Pool& P = pool();
   std::unique_lock<std::mutex> lk(P.mu);
-  if (P.users > 0 && P.lanes.size() < kIdleLanes && lane.doubles <= kIdleLaneDoubles) {
+  if (usable && P.users > 0 && P.lanes.size() < kIdleLanes && lane.doubles <= kIdleLaneDoubles) {
     P.lanes.push_back(lane);
     lane = HostLane{};
     return;
@@ -307,12 +311,12 @@ hipError_t DevPack::commit(DevBuf<char>& arena, hipStream_t s) {
     }
     e = i.place(i.buf, nullptr, i.count);
     if (e != hipSuccess) return e;
-    e = i.data ? hipMemcpy(i.where(i.buf), i.data, bytes, hipMemcpyHostToDevice)
+    e = i.data ? copy_now(i.where(i.buf), i.data, bytes, hipMemcpyHostToDevice, s)
                : hipMemsetAsync(i.where(i.buf), 0, bytes, s);
   }
   items_.clear();
   if (e != hipSuccess || total == 0) return e;
-  return hipMemcpy(arena.p, host.data(), total, hipMemcpyHostToDevice);
+  return copy_now(arena.p, host.data(), total, hipMemcpyHostToDevice, s);
 }
 
 void transfer_open() {
